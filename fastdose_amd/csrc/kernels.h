@@ -118,6 +118,20 @@ hipError_t launch_global_rows(int n_mat, const uint64_t* row_first, const uint64
 // scale[r] = row maximum; q (nullable) = value / scale in BF16 or FP16
 hipError_t launch_pack_rows(uint64_t R, const uint64_t* rowptr, const float* values, int vtype, float* scale,
                             uint16_t* q, hipStream_t stream);
+// Voxel-major copy of rows whose columns ascend: tiles of consecutive columns (csc_tiles(C) of them).
+// launch_row_tiles: tiles[r (csc_tiles(C) + 1) + t] = row r's entries before tile t; scale (nullable)
+// = row maxima; *unsorted (zeroed by the caller) = 1 when a row's columns do not ascend below C (the
+// table then must not be used).  launch_tile_totals: total[t] (zeroed by the caller) = entries of tile
+// t.  launch_place_tiles: colptr (C + 1), crow and cval from the table and tile_base, the exclusive
+// scan of total.  C > 0, R x 2048 and every row's length below 2^32.
+uint64_t csc_tiles(uint64_t C);
+hipError_t launch_row_tiles(uint64_t R, const uint64_t* rowptr, const uint64_t* columns, const float* values,
+                            uint64_t C, uint32_t* tiles, float* scale, uint32_t* unsorted, hipStream_t stream);
+hipError_t launch_tile_totals(uint64_t R, uint64_t C, const uint32_t* tiles, uint32_t* total, hipStream_t stream);
+hipError_t launch_place_tiles(int vtype, uint64_t R, uint64_t C, const uint32_t* tiles, const uint64_t* rowptr,
+                              const uint64_t* columns, const float* values, const float* scale,
+                              const uint64_t* tile_base, uint64_t* colptr, uint32_t* crow, void* cval,
+                              hipStream_t stream);
 hipError_t launch_col_count(uint64_t nnz, const uint64_t* columns, uint32_t* count, hipStream_t stream);
 hipError_t launch_col_scatter(uint64_t R, const uint64_t* rowptr, const uint64_t* columns, const void* vals,
                               int vbytes, const uint64_t* colptr, uint32_t* cursor, uint32_t* crow, void* cval,

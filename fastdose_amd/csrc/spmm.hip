@@ -18,7 +18,7 @@ struct fd_spmm {
     DevBuf<uint64_t> colptr;  // cols + 1
     DevBuf<uint32_t> crow;    // nnz, row of each entry, ascending within a column
     DevBuf<uint8_t> cval;     // nnz values (4 or 2 bytes each)
-    DevBuf<float> scale;      // rows (16-bit types)
+    DevBuf<float> scale;      // rows (16-bit types only)
 };
 
 namespace {
@@ -51,6 +51,78 @@ int build_rowptr(const fd_dosemat* m, DevBuf<uint64_t>& rowptr, uint64_t* R_out,
         return FD_ERR_HIP;
     }
     return FD_OK;
+}
+
+int hip_result(hipError_t e) {
+    if (e == hipSuccess) return FD_OK;
+    set_error(std::string("spmm build: ") + hipGetErrorString(e));
+    return FD_ERR_HIP;
+}
+
+// The voxel-major copy tile by tile (launch_place_tiles); *built is false when a row's columns do
+// not ascend, and nothing of the copy is written then.
+int build_by_tiles(const fd_dosemat* m, fd_spmm& p, const uint64_t* rowptr, hipStream_t s, bool* built) {
+    const uint64_t nt = csc_tiles(p.cols), R = p.rows;
+    DevBuf<uint64_t> base;    // exclusive scan of the tiles' totals (nt + 1), then the scan's scratch
+    DevBuf<uint32_t> total;   // entries of each tile (nt), unsorted flag, the tile table
+    int r = base.reserve(nt + 1 + scan_scratch_size(nt));
+    if (r == FD_OK) r = total.reserve(nt + 1 + R * (nt + 1));
+    auto enqueue = [&]() -> hipError_t {
+        uint32_t unsorted = 0;
+        uint32_t* tiles = total.ptr + nt + 1;
+        hipError_t e = launch_fill_u32(total.ptr, nt + 1, 0u, s);
+        if (e == hipSuccess)
+            e = launch_row_tiles(R, rowptr, m->columns.ptr, m->values.ptr, p.cols, tiles,
+                                 p.vtype == FD_VAL_F32 ? nullptr : p.scale.ptr, total.ptr + nt, s);
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(&unsorted, total.ptr + nt, sizeof(unsorted), hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        if (e != hipSuccess || unsorted) return e;
+        e = launch_tile_totals(R, p.cols, tiles, total.ptr, s);
+        if (e == hipSuccess) e = launch_scan_u32(total.ptr, nt, base.ptr, base.ptr + nt, base.ptr + nt + 1, s);
+        if (e == hipSuccess)
+            e = launch_place_tiles(p.vtype, R, p.cols, tiles, rowptr, m->columns.ptr, m->values.ptr, p.scale.ptr,
+                                   base.ptr, p.colptr.ptr, p.crow.ptr, p.cval.ptr, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        *built = e == hipSuccess;
+        return e;
+    };
+    if (r == FD_OK) r = hip_result(enqueue());
+    base.release();
+    total.release();
+    return r;
+}
+
+// The same for any rows: counts and scatter with atomics, then a sort of every column by row.
+int build_by_sorting(const fd_dosemat* m, fd_spmm& p, const uint64_t* rowptr, hipStream_t s) {
+    const int vbytes = p.vtype == FD_VAL_F32 ? 4 : 2;
+    DevBuf<uint32_t> count;
+    DevBuf<uint16_t> q;
+    DevBuf<uint64_t> scan_tmp;
+    int r = count.reserve(p.cols);
+    if (r == FD_OK) r = scan_tmp.reserve(scan_scratch_size(p.cols));
+    if (r == FD_OK && vbytes == 2) r = q.reserve(std::max<uint64_t>(p.nnz, 1));
+    auto enqueue = [&]() -> hipError_t {
+        hipError_t e = hipSuccess;
+        if (vbytes == 2) e = launch_pack_rows(p.rows, rowptr, m->values.ptr, p.vtype, p.scale.ptr, q.ptr, s);
+        if (e == hipSuccess) e = launch_fill_u32(count.ptr, p.cols, 0u, s);
+        if (e == hipSuccess) e = launch_col_count(p.nnz, m->columns.ptr, count.ptr, s);
+        if (e == hipSuccess)
+            e = launch_scan_u32(count.ptr, p.cols, p.colptr.ptr, p.colptr.ptr + p.cols, scan_tmp.ptr, s);
+        if (e == hipSuccess) e = launch_fill_u32(count.ptr, p.cols, 0u, s);
+        if (e == hipSuccess)
+            e = launch_col_scatter(p.rows, rowptr, m->columns.ptr,
+                                   vbytes == 2 ? (const void*)q.ptr : (const void*)m->values.ptr, vbytes,
+                                   p.colptr.ptr, count.ptr, p.crow.ptr, p.cval.ptr, s);
+        if (e == hipSuccess) e = launch_col_sort(p.cols, p.colptr.ptr, p.crow.ptr, p.cval.ptr, vbytes, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        return e;
+    };
+    if (r == FD_OK) r = hip_result(enqueue());
+    count.release();
+    q.release();
+    scan_tmp.release();
+    return r;
 }
 
 bool valid_type(int t) { return t == FD_VAL_F32 || t == FD_VAL_BF16 || t == FD_VAL_FP16; }
@@ -114,53 +186,27 @@ int fd_spmm_create(const fd_dosemat* m, int value_type, fd_spmm** out, void* str
     p->nnz = m->used_nnz;
     const int vbytes = value_type == FD_VAL_F32 ? 4 : 2;
     DevBuf<uint64_t> rowptr;
-    DevBuf<uint32_t> count;
-    DevBuf<uint16_t> q;
-    auto fail = [&](int r) {
-        rowptr.release();
-        count.release();
-        q.release();
+    int r = build_rowptr(m, rowptr, &p->rows, s);
+    if (r == FD_OK && p->rows >= (1ull << 32)) {
+        set_error("more than 2^32 rows");
+        r = FD_ERR_ARG;
+    }
+    if (r == FD_OK) r = p->colptr.reserve(p->cols + 1);
+    if (r == FD_OK) r = p->crow.reserve(std::max<uint64_t>(p->nnz, 1));
+    if (r == FD_OK) r = p->cval.reserve(std::max<uint64_t>(p->nnz, 1) * vbytes);
+    if (r == FD_OK && vbytes == 2) r = p->scale.reserve(std::max<uint64_t>(p->rows, 1));
+    bool built = false;
+    // The tile table holds a u32 per (row, tile): rows of a few entries in a large volume, whose table
+    // would outgrow the entries themselves, take the general path, as do rows with unsorted columns.
+    if (r == FD_OK && p->cols < (1ull << 32) && p->rows <= (1ull << 20) &&
+        p->rows * (csc_tiles(p->cols) + 1) * sizeof(uint32_t) <= 8 * p->nnz + (1ull << 20))
+        r = build_by_tiles(m, *p, rowptr.ptr, s, &built);
+    if (r == FD_OK && !built) r = build_by_sorting(m, *p, rowptr.ptr, s);
+    rowptr.release();
+    if (r != FD_OK) {
         fd_spmm_destroy(p);
         return r;
-    };
-    int r = build_rowptr(m, rowptr, &p->rows, s);
-    if (r != FD_OK) return fail(r);
-    if (p->rows >= (1ull << 32)) {
-        set_error("more than 2^32 rows");
-        return fail(FD_ERR_ARG);
     }
-    if ((r = p->colptr.reserve(p->cols + 1)) != FD_OK || (r = p->crow.reserve(std::max<uint64_t>(p->nnz, 1))) != FD_OK ||
-        (r = p->cval.reserve(std::max<uint64_t>(p->nnz, 1) * vbytes)) != FD_OK ||
-        (r = p->scale.reserve(std::max<uint64_t>(p->rows, 1))) != FD_OK ||
-        (r = count.reserve(p->cols)) != FD_OK)
-        return fail(r);
-    const void* src = m->values.ptr;
-    if (vbytes == 2) {
-        if ((r = q.reserve(std::max<uint64_t>(p->nnz, 1))) != FD_OK) return fail(r);
-        src = q.ptr;
-    }
-    hipError_t e = launch_pack_rows(p->rows, rowptr.ptr, m->values.ptr, value_type, p->scale.ptr,
-                                    vbytes == 2 ? q.ptr : nullptr, s);
-    if (e == hipSuccess) e = launch_fill_u32(count.ptr, p->cols, 0u, s);
-    if (e == hipSuccess) e = launch_col_count(p->nnz, m->columns.ptr, count.ptr, s);
-    DevBuf<uint64_t> scan_tmp;
-    if (e == hipSuccess && scan_tmp.reserve(scan_scratch_size(p->cols)) != FD_OK) e = hipErrorOutOfMemory;
-    if (e == hipSuccess)
-        e = launch_scan_u32(count.ptr, p->cols, p->colptr.ptr, p->colptr.ptr + p->cols, scan_tmp.ptr, s);
-    if (e == hipSuccess) e = launch_fill_u32(count.ptr, p->cols, 0u, s);
-    if (e == hipSuccess)
-        e = launch_col_scatter(p->rows, rowptr.ptr, m->columns.ptr, src, vbytes, p->colptr.ptr, count.ptr,
-                               p->crow.ptr, p->cval.ptr, s);
-    if (e == hipSuccess) e = launch_col_sort(p->cols, p->colptr.ptr, p->crow.ptr, p->cval.ptr, vbytes, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    scan_tmp.release();
-    if (e != hipSuccess) {
-        set_error(std::string("spmm build: ") + hipGetErrorString(e));
-        return fail(FD_ERR_HIP);
-    }
-    rowptr.release();
-    count.release();
-    q.release();
     *out = p;
     return FD_OK;
 }

@@ -1,0 +1,116 @@
+"""The voxel-major operator (fd_spmm_create) over the shapes at which its kernels
+branch (needs an MI355X): column tiles of 2048, row blocks of 64, rows with more than 64 entries in a
+tile, rows in unsorted order and rows too short for the tile table (the general path)."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import fastdose_amd as fd
+from fastdose_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+U = 2.0 ** -24  # unit roundoff of FP32
+
+
+@pytest.fixture(scope="module")
+def torch_cuda():
+    import torch
+
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    return torch
+
+
+def random_rows(rng, R, cols, fill, long_row=False):
+    """(offsets, columns, values) of R rows with ascending columns: a run per row, a scatter of others,
+    empty rows among them; long_row: row R // 2 holds every column."""
+    offs, cs, vs = [0], [], []
+    for r in range(R):
+        n = int(rng.integers(0, max(2, int(2 * fill * cols))))
+        start = int(rng.integers(0, cols))
+        c = np.unique(np.concatenate([rng.integers(0, cols, n), np.arange(start, min(cols, start + n))]))
+        if r % 7 == 3:
+            c = c[:0]
+        if long_row and r == R // 2:
+            c = np.arange(cols)
+        cs.append(c)
+        vs.append(rng.uniform(0.01, 1.0, len(c)).astype(np.float32))
+        offs.append(offs[-1] + len(c))
+    return np.array(offs), np.concatenate(cs).astype(np.int64), np.concatenate(vs)
+
+
+def dose_mat(torch, cols, mats):
+    dm = fd.DoseMat(cols)
+    for off, c, v in mats:
+        d = [torch.as_tensor(np.ascontiguousarray(a)).cuda() for a in (off.astype(np.int64), c, v)]
+        csr = fd.CSR(len(off) - 1, len(c), len(c), *(t.data_ptr() for t in d))
+        torch.cuda.synchronize()
+        _lib.call("fd_dosemat_add_csr", dm._h, C.byref(csr), None)
+    return dm
+
+
+def dense(mats, cols):
+    out = []
+    for off, c, v in mats:
+        m = np.zeros((len(off) - 1, cols), np.float64)
+        for r in range(len(off) - 1):
+            m[r, c[off[r]:off[r + 1]]] = v[off[r]:off[r + 1]]
+        out.append(m)
+    return np.concatenate(out, 0)
+
+
+def rounded(D, vtype):
+    """The values the operator stores: FP32, or 16 bits of value / row maximum times the FP32 maximum."""
+    if vtype == fd.FD_VAL_F32:
+        return D
+    s = D.max(1, keepdims=True).astype(np.float32)
+    t = np.divide(D.astype(np.float32), s, out=np.zeros(D.shape, np.float32), where=s > 0)
+    if vtype == fd.FD_VAL_FP16:
+        q = t.astype(np.float16).astype(np.float32)
+    else:
+        u = t.view(np.uint32).astype(np.uint64)
+        q = (((u + 0x7FFF + ((u >> 16) & 1)) >> 16) << 16).astype(np.uint32).view(np.float32)
+    return (q * s).astype(np.float64)
+
+
+@pytest.mark.parametrize("vtype", [fd.FD_VAL_F32, fd.FD_VAL_BF16, fd.FD_VAL_FP16])
+@pytest.mark.parametrize("R,cols,fill", [(1, 1, 1.0), (1, 2047, 0.3), (63, 2048, 0.02), (64, 2049, 0.1),
+                                         (65, 4097, 0.05), (130, 6145, 0.02), (200, 40000, 0.004)])
+def test_operator_holds_every_entry_in_row_order(torch_cuda, vtype, R, cols, fill):
+    """D^T times the identity is D^T itself, each entry exactly (one term per sum)."""
+    torch = torch_cuda
+    rng = np.random.default_rng([R, cols, vtype])
+    mats = [random_rows(rng, R, cols, fill, long_row=True), random_rows(rng, 3, cols, fill)]
+    D = rounded(dense(mats, cols), vtype)
+    dm = dose_mat(torch, cols, mats)
+    with fd.Spmm(dm, vtype) as op:
+        y = op.run(torch.eye(R + 3, device="cuda")).cpu().numpy()
+    assert np.array_equal(y.T.astype(np.float64), D)
+
+
+def test_general_path_gives_the_same_operator(torch_cuda):
+    """Rows with their entries in another order, and rows of two entries in a wide volume, take the
+    general path; its product equals the tiles' bit for bit where both can be built."""
+    torch = torch_cuda
+    rng = np.random.default_rng(5)
+    off, c, v = random_rows(rng, 70, 5000, 0.03)
+    order = np.concatenate([off[r] + rng.permutation(off[r + 1] - off[r]) for r in range(70)])
+    x = torch.rand((70, 9), device="cuda")
+    y = []
+    for m in ((off, c, v), (off, c[order], v[order])):
+        with fd.Spmm(dose_mat(torch, 5000, [m])) as op:
+            y.append(op.run(x).cpu().numpy())
+    assert np.array_equal(*y)
+    cols, R = 3_000_000, 400
+    c = np.sort(rng.choice(cols, (R, 2)), 1).astype(np.int64)
+    c[:, 1] += c[:, 1] == c[:, 0]
+    c = np.minimum(c, cols - 1)
+    v = rng.uniform(0.01, 1.0, 2 * R).astype(np.float32)
+    with fd.Spmm(dose_mat(torch, cols, [(np.arange(0, 2 * R + 1, 2), c.reshape(-1), v)])) as op:
+        x = torch.rand((R, 1), device="cuda")
+        got = op.run(x).cpu().numpy()[:, 0].astype(np.float64)
+    want = np.zeros(cols)
+    np.add.at(want, c.reshape(-1), v.astype(np.float64) * np.repeat(x.cpu().numpy()[:, 0].astype(np.float64), 2))
+    assert np.all(np.abs(got - want) <= 4 * U * want)
