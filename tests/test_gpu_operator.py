@@ -1,6 +1,7 @@
-"""The voxel-major operator (fd_spmm_create) over the shapes at which its kernels
+"""The voxel-major operator (fd_spmm_create) and its product over the shapes at which its kernels
 branch (needs an MI355X): column tiles of 2048, row blocks of 64, rows with more than 64 entries in a
-tile, rows in unsorted order and rows too short for the tile table (the general path)."""
+tile, rows in unsorted order and rows too short for the tile table (the general path), and every
+arrangement of the product's lanes, against numpy in FP64."""
 import ctypes as C
 
 import numpy as np
@@ -114,3 +115,28 @@ def test_general_path_gives_the_same_operator(torch_cuda):
     want = np.zeros(cols)
     np.add.at(want, c.reshape(-1), v.astype(np.float64) * np.repeat(x.cpu().numpy()[:, 0].astype(np.float64), 2))
     assert np.all(np.abs(got - want) <= 4 * U * want)
+
+
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 7, 8, 12, 16, 20, 31, 33, 64, 65, 100, 128, 130, 132, 256, 260])
+def test_product_over_lane_arrangements(torch_cuda, k):
+    """Sparse, medium and crowded stretches of columns (each picks its own lanes per column, the crowded
+    one is split over the workgroup), a last partial tile, all value types."""
+    torch = torch_cuda
+    rng = np.random.default_rng(k)
+    R, cols = 300, 1000
+    p = np.concatenate([np.full(256, 0.003), np.full(300, 0.03), np.full(200, 0.12), np.full(244, 0.7)])
+    M = np.where(rng.random((R, cols)) < p, rng.uniform(0.01, 1.0, (R, cols)), 0.0).astype(np.float32)
+    M[:, 64:128] = 0.0
+    r, c = np.nonzero(M)
+    off = np.concatenate([[0], np.cumsum((M != 0).sum(1))])
+    dm = dose_mat(torch, cols, [(off, c.astype(np.int64), M[r, c])])
+    x = rng.uniform(-1.0, 1.0, (R, k)).astype(np.float32)
+    for vtype in (fd.FD_VAL_F32, fd.FD_VAL_BF16, fd.FD_VAL_FP16):
+        D = rounded(M.astype(np.float64), vtype)
+        with fd.Spmm(dm, vtype) as op:
+            y = op.run(torch.as_tensor(x).cuda())
+            again = op.run(torch.as_tensor(x).cuda())
+        assert torch.equal(y, again)
+        want, mag = D.T @ x.astype(np.float64), np.abs(D).T @ np.abs(x.astype(np.float64))
+        n = (D != 0).sum(0)[:, None]
+        assert np.all(np.abs(y.cpu().numpy() - want) <= (n + 2) * U * mag), (k, vtype)
