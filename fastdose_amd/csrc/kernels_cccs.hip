@@ -723,34 +723,44 @@ __device__ __forceinline__ bool march_chunk(MarchLane& M, const MarchConst& C, i
         M.act = lane < n_phi;
         M.nsteps = 0;
     }
-    // phase 1: lattice points; pos[f][0] is where the chunk starts
-    float4* mypos = S.pos + (lane < n_phi ? lane : 0) * (kRecCap + 1);
-    if (lane < n_phi) mypos[0] = make_float4(M.bxp, M.byp, M.bzp, 0.0f);
+    // phase 1: lattice points; pos[f][0] is where the chunk starts.  A serial chain of FP32 steps per
+    // lane, and the other wavefronts wait for it when the GPU is not full, so it is kept short: no
+    // branch on the slice end (both candidates are computed, lanes that have reached theirs keep
+    // their position and write past their last point, which nothing reads), two steps per test.
     int cnt = 0, k = 0;
-    for (; k < kRecCap; k++) {
-        if (__ballot(M.act) == 0) break;
-        if (M.act) {
+    if (lane < n_phi) {
+        float4* mypos = S.pos + lane * (kRecCap + 1);
+        mypos[0] = make_float4(M.bxp, M.byp, M.bzp, 0.0f);
+        auto step = [&](int at) {
             const float sx = axis_step(M.bxp, M.sgx, M.ix_);
             const float sy = axis_step(M.byp, M.sgy, M.iy_);
             const float sz = axis_step(M.bzp, M.sgz, M.iz_);
             const float st = fminf(fminf(sx, sy), sz);
-            float nx = fmaf(st, M.dx, M.bxp), ny = fmaf(st, M.dy, M.byp), nz = fmaf(st, M.dz, M.bzp);
+            const float nz = fmaf(st, M.dz, M.bzp);
             // rint == round here: a tie (.5) is never within 1e-4 of an integer
             const bool flag = fabsf(nz - rintf(nz)) < kEps;
-            if (flag) {
-                nx = fmaf(sz, M.dx, M.bxp);
-                ny = fmaf(sz, M.dy, M.byp);
-                nz = rintf(fmaf(sz, M.dz, M.bzp));
-            }
-            mypos[k + 1] = make_float4(nx, ny, nz, 0.0f);
-            M.bxp = nx;
-            M.byp = ny;
-            M.bzp = nz;
-            cnt = k + 1;
-            M.nsteps++;
-            if (flag || M.nsteps >= kMaxStepsPerSlice) M.act = false;
+            const float to = flag ? sz : st;
+            const float x = fmaf(to, M.dx, M.bxp), y = fmaf(to, M.dy, M.byp);
+            const float z = flag ? rintf(fmaf(sz, M.dz, M.bzp)) : nz;
+            mypos[at] = make_float4(x, y, z, 0.0f);
+            M.bxp = M.act ? x : M.bxp;
+            M.byp = M.act ? y : M.byp;
+            M.bzp = M.act ? z : M.bzp;
+            cnt += M.act ? 1 : 0;
+            M.act = M.act && !flag;
+        };
+        static_assert(kRecCap % 2 == 0, "two steps per test");
+        for (; k < kRecCap; k += 2) {
+            if (__ballot(M.act) == 0) break;
+            step(k + 1);
+            step(k + 2);
         }
+        M.nsteps += cnt;
+        // a lane still under way has taken whole chunks of kRecCap steps in this slice
+        static_assert(kMaxStepsPerSlice % kRecCap == 0, "the step limit falls on a chunk's end");
+        if (M.nsteps >= kMaxStepsPerSlice) M.act = false;
     }
+    k = __builtin_amdgcn_readfirstlane(k);
     const bool done = __ballot(M.act) == 0;
     if (lane < n_phi) hdr[lane] = cnt;
     if (lane == 0) {
