@@ -587,46 +587,51 @@ int fd_dense_to_csr(const float* dense_dev, uint64_t rows, uint64_t cols, fd_csr
     }
     hipStream_t s = (hipStream_t)stream;
     out->rows = rows;
-    uint32_t* cnt = nullptr;
+    const DenseSplit split = dense_split(rows, cols, 1ull << 25);
+    const uint64_t n = rows * split.per_row;  // segments
+    // one block, ordered on the stream: segment offsets and their total, scan scratch, segment counts
+    const uint64_t n_off = n + 1 + scan_scratch_size(n);
     uint64_t* off = nullptr;
-    uint64_t* host = nullptr;
-    auto cleanup = [&]() {
-        if (cnt) (void)hipFree(cnt);
-        if (off) (void)hipFree(off);
-        if (host) (void)hipHostFree(host);
-    };
-    auto hip_fail = [&](hipError_t e, const char* what) {
+    auto fail = [&](hipError_t e, const char* what) {
         set_error(std::string(what) + ": " + hipGetErrorString(e));
-        cleanup();
+        if (off) (void)hipFreeAsync(off, s);
         return FD_ERR_HIP;
     };
-    hipError_t e;
-    if ((e = hipMalloc((void**)&cnt, std::max<uint64_t>(rows, 1) * sizeof(uint32_t))) != hipSuccess)
-        return hip_fail(e, "hipMalloc");
-    if ((e = hipMalloc((void**)&off, (rows + 1) * sizeof(uint64_t))) != hipSuccess) return hip_fail(e, "hipMalloc");
-    if ((e = hipHostMalloc((void**)&host, sizeof(uint64_t), hipHostMallocDefault)) != hipSuccess)
-        return hip_fail(e, "hipHostMalloc");
-    if (rows > 0 && cols > 0) {
-        if ((e = launch_dense_count(dense_dev, rows, cols, cnt, s)) != hipSuccess) return hip_fail(e, "count");
-    } else if (rows > 0) {
-        if ((e = launch_fill_u32(cnt, rows, 0, s)) != hipSuccess) return hip_fail(e, "fill");
+    hipError_t e = hipMallocAsync((void**)&off, n_off * sizeof(uint64_t) + std::max<uint64_t>(n, 1) * sizeof(uint32_t), s);
+    if (e != hipSuccess) {
+        off = nullptr;
+        return fail(e, "hipMallocAsync");
     }
-    if ((e = launch_scan_u32(cnt, rows, off, off + rows, nullptr, s)) != hipSuccess) return hip_fail(e, "scan");
-    if ((e = hipMemcpyAsync(host, off + rows, sizeof(uint64_t), hipMemcpyDeviceToHost, s)) != hipSuccess)
-        return hip_fail(e, "copy");
-    if ((e = hipStreamSynchronize(s)) != hipSuccess) return hip_fail(e, "sync");
-    out->nnz = host[0];
+    uint32_t* cnt = (uint32_t*)(off + n_off);
+    if (rows > 0 && cols > 0) {
+        if ((e = launch_dense_count(dense_dev, rows, cols, split, cnt, s)) != hipSuccess) return fail(e, "count");
+    } else if (rows > 0) {
+        if ((e = launch_fill_u32(cnt, n, 0, s)) != hipSuccess) return fail(e, "fill");
+    }
+    if ((e = launch_scan_u32(cnt, n, off, off + n, off + n + 1, s)) != hipSuccess) return fail(e, "scan");
+    uint64_t total = 0;
+    if ((e = hipMemcpyAsync(&total, off + n, sizeof(uint64_t), hipMemcpyDeviceToHost, s)) != hipSuccess)
+        return fail(e, "copy");
+    if ((e = hipStreamSynchronize(s)) != hipSuccess) return fail(e, "sync");
+    out->nnz = total;
     if (out->nnz > out->capacity || (out->nnz > 0 && (!out->columns || !out->values))) {
-        cleanup();
+        (void)hipFreeAsync(off, s);
         set_error("CSR capacity too small; nnz reported in out->nnz");
         return FD_ERR_CAPACITY;
     }
     if (rows > 0 && cols > 0 && out->nnz > 0)
-        if ((e = launch_dense_fill(dense_dev, rows, cols, off, out->columns, out->values, s)) != hipSuccess)
-            return hip_fail(e, "fill");
-    if ((e = launch_write_offsets(off, off + rows, rows, out->offsets, s)) != hipSuccess) return hip_fail(e, "offsets");
-    if ((e = hipStreamSynchronize(s)) != hipSuccess) return hip_fail(e, "sync");
-    cleanup();
+        if ((e = launch_dense_fill(dense_dev, rows, cols, split, off, out->columns, out->values, s)) != hipSuccess)
+            return fail(e, "fill");
+    if ((e = launch_write_offsets(off, off + n, rows, split.per_row, out->offsets, s)) != hipSuccess)
+        return fail(e, "offsets");
+    if ((e = hipFreeAsync(off, s)) != hipSuccess) {
+        off = nullptr;
+        return fail(e, "hipFreeAsync");
+    }
+    if ((e = hipStreamSynchronize(s)) != hipSuccess) {
+        off = nullptr;
+        return fail(e, "sync");
+    }
     return FD_OK;
 }
 

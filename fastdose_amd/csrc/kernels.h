@@ -100,16 +100,23 @@ hipError_t launch_scan_u32(const uint32_t* count, uint64_t N, uint64_t* off, uin
                            hipStream_t stream);
 uint64_t scan_scratch_size(uint64_t N);
 
-// Dense (rows x cols, row-major) -> CSR: per-row nonzero counts, then fill.
-hipError_t launch_dense_count(const float* dense, uint64_t rows, uint64_t cols, uint32_t* row_count,
+// Dense (rows x cols, row-major) -> CSR, by segments of rows: nonzero counts per segment, then (after
+// an exclusive scan of them) the fill.
+struct DenseSplit {
+    uint32_t per_row;  // segments per row
+    uint32_t length;   // elements per segment (the row's last one may hold fewer)
+};
+// Segments for rows x cols with at most max(max_segments, rows) of them (cols < 2^32).
+DenseSplit dense_split(uint64_t rows, uint64_t cols, uint64_t max_segments);
+hipError_t launch_dense_count(const float* dense, uint64_t rows, uint64_t cols, const DenseSplit& s, uint32_t* count,
                               hipStream_t stream);
-hipError_t launch_dense_fill(const float* dense, uint64_t rows, uint64_t cols, const uint64_t* row_off,
-                             uint64_t* columns, float* values, hipStream_t stream);
-// offsets[r] = row_off[r] (r < rows), offsets[rows] = total[0].
+hipError_t launch_dense_fill(const float* dense, uint64_t rows, uint64_t cols, const DenseSplit& s,
+                             const uint64_t* seg_off, uint64_t* columns, float* values, hipStream_t stream);
 hipError_t launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t stream);
 hipError_t launch_fill_u64(uint64_t* p, uint64_t n, uint64_t v, hipStream_t stream);
-hipError_t launch_write_offsets(const uint64_t* row_off, const uint64_t* total, uint64_t rows, uint64_t* offsets,
-                                hipStream_t stream);
+// offsets[r] = seg_off[r n_seg] (r < rows), offsets[rows] = total[0].
+hipError_t launch_write_offsets(const uint64_t* seg_off, const uint64_t* total, uint64_t rows, uint32_t n_seg,
+                                uint64_t* offsets, hipStream_t stream);
 
 // Packing and D^T X products (kernels_spmm.hip).
 hipError_t launch_global_rows(int n_mat, const uint64_t* row_first, const uint64_t* off_off, const uint64_t* nnz_off,

@@ -1,7 +1,7 @@
 // noalloc.hip -- fd_dense_to_csr_noalloc: dense -> CSR with no allocation by the library.
 //
-// The same kernels as fd_dense_to_csr (count -> scan -> ordered fill -> offsets), but the per-row
-// counts and row offsets live in one file-scope device array instead of hipMalloc'd buffers, and the
+// The same kernels as fd_dense_to_csr (count -> scan -> ordered fill -> offsets), but the counts and
+// offsets live in one file-scope device array instead of hipMalloc'd buffers, and the
 // nonzero total comes back through a plain (pageable) host variable instead of pinned memory.
 // Each device that runs the library holds its own copy of the array until the process ends; its
 // device address is looked up once per device (hipGetSymbolAddress) and only that address is ever
@@ -20,8 +20,11 @@ namespace fdi {
 namespace {
 
 constexpr uint64_t kNoAllocMaxRows = FD_NOALLOC_MAX_ROWS;
-// row offsets: u64 [kNoAllocMaxRows + 1]; then per-row counts: u32 [kNoAllocMaxRows], 256-aligned
-constexpr size_t kOffBytes = (kNoAllocMaxRows + 1) * sizeof(uint64_t);
+// segment offsets and their total: u64 [kNoAllocMaxRows + 1], scan scratch: u64 [kScanScratch]; then
+// counts per segment: u32 [kNoAllocMaxRows], 256-aligned.  Rows are cut into fewer segments than
+// fd_dense_to_csr would take when there would be more of them than that.
+constexpr uint64_t kScanScratch = kNoAllocMaxRows / 4096 + 2;
+constexpr size_t kOffBytes = (kNoAllocMaxRows + 1 + kScanScratch) * sizeof(uint64_t);
 constexpr size_t kCntStart = (kOffBytes + 255) / 256 * 256;
 constexpr size_t kScratchBytes = kCntStart + kNoAllocMaxRows * sizeof(uint32_t);
 
@@ -80,22 +83,28 @@ extern "C" int fd_dense_to_csr_noalloc(const float* dense_dev, uint64_t rows, ui
     out->rows = rows;
     // every count is written by the count kernel (or the fill), the scan overwrites every offset
     // and the total: nothing left by an earlier call is read
+    const DenseSplit split = dense_split(rows, cols, kNoAllocMaxRows);
+    const uint64_t n = rows * split.per_row;
     if (rows > 0 && cols > 0) {
-        FD_HIP(launch_dense_count(dense_dev, rows, cols, cnt, s));
+        FD_HIP(launch_dense_count(dense_dev, rows, cols, split, cnt, s));
     } else if (rows > 0) {
-        FD_HIP(launch_fill_u32(cnt, rows, 0, s));
+        FD_HIP(launch_fill_u32(cnt, n, 0, s));
     }
-    FD_HIP(launch_scan_u32(cnt, rows, off, off + rows, nullptr, s));
+    if (scan_scratch_size(n) > kScanScratch) {  // the scan's own tile size decides
+        set_error("scan scratch of the allocation-free entry point too small");
+        return FD_ERR_UNSUPPORTED;
+    }
+    FD_HIP(launch_scan_u32(cnt, n, off, off + n, off + kNoAllocMaxRows + 1, s));
     uint64_t total = 0;
-    FD_HIP(hipMemcpyAsync(&total, off + rows, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
+    FD_HIP(hipMemcpyAsync(&total, off + n, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
     FD_HIP(hipStreamSynchronize(s));
     out->nnz = total;
     if (total > out->capacity || (total > 0 && (!out->columns || !out->values))) {
         set_error("CSR capacity too small; nnz reported in out->nnz");
         return FD_ERR_CAPACITY;
     }
-    if (rows > 0 && cols > 0 && total > 0) FD_HIP(launch_dense_fill(dense_dev, rows, cols, off, out->columns, out->values, s));
-    FD_HIP(launch_write_offsets(off, off + rows, rows, out->offsets, s));
+    if (rows > 0 && cols > 0 && total > 0) FD_HIP(launch_dense_fill(dense_dev, rows, cols, split, off, out->columns, out->values, s));
+    FD_HIP(launch_write_offsets(off, off + n, rows, split.per_row, out->offsets, s));
     FD_HIP(hipStreamSynchronize(s));
     return FD_OK;
 }

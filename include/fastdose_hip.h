@@ -242,8 +242,8 @@ int fd_dense_to_csr(const float* dense_dev, uint64_t rows, uint64_t cols, fd_csr
 
 /* fd_dense_to_csr without any allocation: no counterpart in the reference.  For callers that
  * cannot allocate device or pinned memory (tight serving loops, harnesses that forbid hipMalloc).
- * Same arguments, results and two-phase capacity rule as fd_dense_to_csr; its per-row counts and
- * row offsets live in a library-held device array of about 12 MiB per device (held until the
+ * Same arguments, results and two-phase capacity rule as fd_dense_to_csr; its counts and
+ * offsets live in a library-held device array of about 12 MiB per device (held until the
  * process ends), so rows is limited to FD_NOALLOC_MAX_ROWS (FD_ERR_ARG beyond).  Every call on
  * one device shares that array: calls that overlap in time on one device race.  The call
  * synchronises `stream` before it returns. */
