@@ -191,9 +191,10 @@ int fd_beamlet_flags(fd_ctx* ctx, const uint8_t* mask_dev, const fd_bundle* bund
     hipStream_t s = (hipStream_t)stream;
     FD_TRY(ctx->flag_desc.reserve(d.size()));
     FD_TRY(ctx->flag_out.reserve(total));
+    FD_TRY(ctx->flag_box.reserve(6));
     FD_HIP(hipMemcpyAsync(ctx->flag_desc.ptr, d.data(), d.size() * sizeof(FlagBeamDev), hipMemcpyHostToDevice, s));
     hipError_t e = launch_beamlet_flags(ctx->flag_desc.ptr, n_bundles, max_pixels, mask_dev, ctx->vol,
-                                        ctx->flag_out.ptr, s);
+                                        ctx->flag_box.ptr, ctx->flag_out.ptr, s);
     if (e != hipSuccess) {
         set_error(std::string("beamlet flags launch: ") + hipGetErrorString(e));
         return FD_ERR_HIP;
@@ -435,6 +436,7 @@ int fd_ctx_destroy(fd_ctx* ctx) {
     ctx->ws.release();
     ctx->flag_desc.release();
     ctx->flag_out.release();
+    ctx->flag_box.release();
     for (auto& w : ctx->parked_ws) w.release();  // frees ordered on park_stream
     for (auto& c : ctx->parked_csr) {
         c.cols.release();

@@ -1,0 +1,74 @@
+"""Device beamlet flags against the host's, bit for bit, where the mask's bounding box and the depth
+range cut from it can go wrong: single texels at corners and edges, one-texel-thick planes, an empty and a
+full mask, masks at every byte alignment, odd dimensions, beams along the axes (needs an MI355X)."""
+import numpy as np
+import pytest
+
+import fastdose_amd as fd
+from fastdose_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+DIM = (37, 29, 23)
+
+
+@pytest.fixture(scope="module")
+def torch_cuda():
+    import torch
+
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    return torch
+
+
+def masks():
+    X, Y, Z = DIM
+    out = {}
+    for name, at in {"corner": (0, 0, 0), "far corner": (Z - 1, Y - 1, X - 1), "edge": (Z // 2, 0, X - 1),
+                     "middle": (Z // 2, Y // 2, X // 2)}.items():
+        m = np.zeros((Z, Y, X), np.uint8)
+        m[at] = 1
+        out[name] = m
+    plane = np.zeros((Z, Y, X), np.uint8)
+    plane[:, Y // 3, :] = 255
+    out["plane"] = plane
+    two = np.zeros((Z, Y, X), np.uint8)
+    two[1, 2, 3] = two[Z - 2, Y - 3, X - 4] = 7
+    out["two texels"] = two
+    out["empty"] = np.zeros((Z, Y, X), np.uint8)
+    out["full"] = np.ones((Z, Y, X), np.uint8)
+    out["speckle"] = (np.random.default_rng(1).random((Z, Y, X)) < 0.002).astype(np.uint8)
+    return out
+
+
+@pytest.mark.parametrize("name", list(masks()))
+def test_flags_equal_the_host(torch_cuda, name):
+    torch = torch_cuda
+    m = masks()[name]
+    vol = synth.make_volume(DIM, 0.25)
+    rng = np.random.default_rng(sum(map(ord, name)))
+    iso = [0.25 * d / 2 for d in DIM]
+    angles = [(0, 0, 0), (90, 0, 0), (180, 0, 0), (270, 90, 0), (90, 90, 0)] + \
+        [tuple(rng.uniform(0, 360, 3)) for _ in range(12)]
+    bundles = []
+    for a in angles:
+        at = [c + float(rng.uniform(-2, 2)) for c in iso]
+        bundles.append(synth.make_bundle(at, a, fluence_dim=int(rng.integers(1, 24)), beamlet_size=0.4,
+                                         long_spacing=float(rng.choice([0.25, 0.1, 0.7]))))
+    want = []
+    for b in bundles:
+        try:
+            want.append(fd.beamlet_flag_init(b, m, vol))
+        except fd.FastDoseError:
+            want.append(np.zeros(b.fluence_dim[0] ** 2, np.uint8))
+    with fd.Context(vol, np.ones(DIM[::-1], np.float32), synth.synthetic_spectrum(1), synth.synthetic_kernel(1)) as ctx:
+        for shift in (0, 1, 7, 15):
+            buf = torch.zeros(m.size + 16, dtype=torch.uint8, device="cuda")
+            buf[:shift] = 1            # texels beside the mask are not part of it
+            buf[shift + m.size:] = 1
+            buf[shift:shift + m.size] = torch.from_numpy(m.reshape(-1)).cuda()
+            got = ctx.beamlet_flags(buf[shift:], bundles)
+            for w, g in zip(want, got):
+                assert np.array_equal(w, g)
+    if name in ("full", "plane"):
+        assert any(w.any() for w in want)
