@@ -126,8 +126,9 @@ struct Workspace {
     size_t tab_stage_cap = 0;
     std::vector<int32_t> tab_geom;
     int tab_n_gt = 0;
-    uint64_t* host_totals = nullptr;  // pinned: candidates, nonzeros, overflow flags (resampler, tables)
-    uint64_t* host_rowoff = nullptr;  // pinned copy of rowoff
+    // pinned, written by the batch's last kernel: candidates, nonzeros, overflow flags (resampler, tables)
+    uint64_t* host_totals = nullptr;
+    uint64_t* host_rowoff = nullptr;  // pinned copy of rowoff, likewise
     size_t host_rowoff_cap = 0;
     double cand_per_beamlet = 0.0;    // running estimate that sizes the staging up front
     // kernel timers: slot k uses ev[2k] / ev[2k+1] (the cone sum starts at the CCCS end event);
@@ -279,8 +280,12 @@ int run_cccs(const fd_ctx* ctx, Workspace& w, int options, int n, int max_L, con
 // staging overflows).  thr > 0 keeps only entries >= thr * (the beamlet's maximum value).
 int run_resample_csr(const fd_ctx* ctx, Workspace& w, const fd_beam* beams, int n, const float* dose, float extent,
                      float thr, const fd_csr& out, uint64_t* nnz_total, hipStream_t stream);
+// Also leaves the totals in w.host_totals (and the row offsets in w.host_rowoff: rows) for the host to
+// read after the stream's next synchronisation.
 int run_resample_compact(const fd_ctx* ctx, Workspace& w, int n, float thr, uint64_t* offsets, const CsrDst& dst0,
-                         const CsrDst& dst1, hipStream_t stream);
+                         const CsrDst& dst1, bool rows, hipStream_t stream);
+// Entries the resampler's staging is sized for on these beamlets (candidates, with headroom).
+uint64_t candidate_estimate(const fd_ctx* ctx, Workspace& w, const fd_beam* beams, int n, double* frustum);
 
 // The whole path for a batch of beamlets (host descriptors and host fluence, 256 floats each):
 // Terma -> CCCS -> resampling, one host synchronisation (two when the resampler staging estimate

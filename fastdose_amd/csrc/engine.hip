@@ -226,6 +226,13 @@ void update_candidate_estimate(Workspace& w, double ratio) {
 
 }  // namespace
 
+uint64_t candidate_estimate(const fd_ctx* ctx, Workspace& w, const fd_beam* beams, int n, double* frustum) {
+    *frustum = 0;
+    for (int i = 0; i < n; i++) *frustum += frustum_voxels(beams[i], ctx->vol);
+    if (w.cand_per_beamlet <= 0) w.cand_per_beamlet = 2.0;  // candidates per frustum voxel, first guess
+    return std::max<uint64_t>((uint64_t)std::ceil(w.cand_per_beamlet * *frustum), 1024);
+}
+
 size_t batch_footprint(const fd_ctx* ctx, const fd_beam* beams, int n) {
     if (n <= 0) return 0;
     uint64_t bev = 0;  // BEV floats of the batch (packed volumes)
@@ -341,7 +348,7 @@ int reserve_segments(const fd_ctx* ctx, Workspace& w, int n) {
     FD_TRY(w.nnz_count.reserve(segs));
     FD_TRY(w.cand_off.reserve(segs + 1));
     FD_TRY(w.nnz_off.reserve(segs + 1));
-    FD_TRY(w.flags.reserve(4));  // [0] overflow, [1] zero (read as one u64 with [0]), [2] table overflow
+    FD_TRY(w.flags.reserve(4));  // [0] overflow, [2] table overflow
     FD_TRY(w.rowmax.reserve(n));
     FD_TRY(w.scan_tmp.reserve(scan_scratch_size(segs)));
     return FD_OK;
@@ -350,7 +357,8 @@ int reserve_segments(const fd_ctx* ctx, Workspace& w, int n) {
 int launch_count(const fd_ctx* ctx, Workspace& w, int n, hipStream_t stream) {
     const size_t segs = (size_t)n * ctx->vol.dim[2];
     w.mark(FD_T_RESAMPLE_COUNT, 0, stream);
-    hipError_t e = launch_resample_count(w.desc.ptr, n, ctx->vol, w.cand_count.ptr, w.cand_rows.ptr, stream);
+    hipError_t e =
+        launch_resample_count(w.desc.ptr, n, ctx->vol, w.cand_count.ptr, w.cand_rows.ptr, w.flags.ptr, stream);
     if (e == hipSuccess) e = launch_scan_u32(w.cand_count.ptr, segs, w.cand_off.ptr, w.cand_off.ptr + segs, w.scan_tmp.ptr, stream);
     w.mark(FD_T_RESAMPLE_COUNT, 1, stream);
     if (e != hipSuccess) {
@@ -360,12 +368,13 @@ int launch_count(const fd_ctx* ctx, Workspace& w, int n, hipStream_t stream) {
     return FD_OK;
 }
 
+// again: a second pass over the same count (which cleared the overflow flag for the first)
 int launch_values(const fd_ctx* ctx, Workspace& w, int n, const float* dose, float extent, float thr, uint64_t cap,
-                  hipStream_t stream) {
+                  hipStream_t stream, bool again = false) {
     const size_t segs = (size_t)n * ctx->vol.dim[2];
     const int Z = (int)ctx->vol.dim[2];
     w.mark(FD_T_RESAMPLE_VALUES, 0, stream);
-    hipError_t e = launch_fill_u32(w.flags.ptr, 2, 0u, stream);
+    hipError_t e = again ? launch_fill_u32(w.flags.ptr, 1, 0u, stream) : hipSuccess;
     if (e == hipSuccess && thr > 0.0f) e = launch_fill_u32(w.rowmax.ptr, (uint64_t)n, 0u, stream);
     if (e == hipSuccess)
         e = launch_resample_values(w.desc.ptr, n, ctx->vol, extent, dose, w.cand_off.ptr, w.cand_rows.ptr, cap, w.flags.ptr,
@@ -392,19 +401,6 @@ int launch_values(const fd_ctx* ctx, Workspace& w, int n, const float* dose, flo
 
 int reserve_host_rowoff(Workspace& w, int n) { return grow_pinned(w.host_rowoff, w.host_rowoff_cap, (size_t)n + 1); }
 
-// totals of the last resampler pass -> pinned host: [0] candidates, [1] nonzeros, [2] overflow;
-// with rows, also the batch's row offsets -> w.host_rowoff (reserved by the caller)
-int fetch_totals(const fd_ctx* ctx, Workspace& w, int n, hipStream_t stream, bool rows) {
-    const size_t segs = (size_t)n * ctx->vol.dim[2];
-    if (rows)
-        FD_HIP(hipMemcpyAsync(w.host_rowoff, w.rowoff.ptr, ((size_t)n + 1) * sizeof(uint64_t),
-                              hipMemcpyDeviceToHost, stream));
-    FD_HIP(hipMemcpyAsync(w.host_totals, w.cand_off.ptr + segs, sizeof(uint64_t), hipMemcpyDeviceToHost, stream));
-    FD_HIP(hipMemcpyAsync(w.host_totals + 1, w.nnz_off.ptr + segs, sizeof(uint64_t), hipMemcpyDeviceToHost, stream));
-    FD_HIP(hipMemcpyAsync(w.host_totals + 2, w.flags.ptr, sizeof(uint64_t), hipMemcpyDeviceToHost, stream));
-    return FD_OK;
-}
-
 }  // namespace
 
 int run_resample_csr(const fd_ctx* ctx, Workspace& w, const fd_beam* beams, int n, const float* dose, float extent,
@@ -414,26 +410,23 @@ int run_resample_csr(const fd_ctx* ctx, Workspace& w, const fd_beam* beams, int 
     // (skipped on the device when they are too small) issued before the host learns the totals:
     // one synchronisation, a second pass only when the estimated staging overflows.
     double est = 0;
-    for (int i = 0; i < n; i++) est += frustum_voxels(beams[i], ctx->vol);
-    if (w.cand_per_beamlet <= 0) w.cand_per_beamlet = 2.0;
-    uint64_t cap = std::max<uint64_t>((uint64_t)std::ceil(w.cand_per_beamlet * est), 1024);
+    uint64_t cap = candidate_estimate(ctx, w, beams, n, &est);
     const uint64_t capacity = (out.columns && out.values) ? out.capacity : 0;
-    auto pass = [&]() -> int {
+    auto pass = [&](bool again) -> int {
         FD_TRY(w.tmp_cols.reserve(cap));
         FD_TRY(w.tmp_vals.reserve(cap));
-        FD_TRY(launch_values(ctx, w, n, dose, extent, thr, cap, stream));
+        FD_TRY(launch_values(ctx, w, n, dose, extent, thr, cap, stream, again));
         FD_TRY(run_resample_compact(ctx, w, n, thr, out.offsets, CsrDst{out.columns, out.values, capacity}, CsrDst{},
-                                    stream));
-        FD_TRY(fetch_totals(ctx, w, n, stream, false));
+                                    false, stream));
         FD_HIP(hipStreamSynchronize(stream));
         return FD_OK;
     };
     FD_TRY(launch_count(ctx, w, n, stream));
-    FD_TRY(pass());
+    FD_TRY(pass(false));
     const uint64_t ncand = w.host_totals[0];
     if (w.host_totals[2]) {
         cap = ncand;
-        FD_TRY(pass());
+        FD_TRY(pass(true));
         if (w.host_totals[2]) {
             set_error("resampler staging overflow with exact sizing");
             return FD_ERR_HIP;
@@ -445,11 +438,12 @@ int run_resample_csr(const fd_ctx* ctx, Workspace& w, const fd_beam* beams, int 
 }
 
 int run_resample_compact(const fd_ctx* ctx, Workspace& w, int n, float thr, uint64_t* offsets, const CsrDst& dst0,
-                         const CsrDst& dst1, hipStream_t stream) {
+                         const CsrDst& dst1, bool rows, hipStream_t stream) {
     w.mark(FD_T_RESAMPLE_COMPACT, 0, stream);
     hipError_t e = launch_resample_compact(n, (int)ctx->vol.dim[2], w.cand_off.ptr, w.nnz_off.ptr, w.nnz_count.ptr,
                                            w.tmp_cols.ptr, w.tmp_vals.ptr, thr > 0.0f ? w.rowmax.ptr : nullptr, thr,
-                                           offsets, dst0, dst1, stream);
+                                           w.flags.ptr, offsets, rows ? w.host_rowoff : nullptr, w.host_totals, dst0,
+                                           dst1, stream);
     w.mark(FD_T_RESAMPLE_COMPACT, 1, stream);
     if (e != hipSuccess) {
         set_error(std::string("resample compact: ") + hipGetErrorString(e));
@@ -571,14 +565,10 @@ int run_batch(const fd_ctx* ctx, Workspace& w, int options, const fd_beam* beams
     // packed BEV volumes: beamlet i at bev_offs[i], the sum of L_j * 256 over j < i
     w.bev_offs.resize((size_t)n + 1);
     w.bev_offs[0] = 0;
-    double est = 0;
-    for (int i = 0; i < n; i++) {
-        w.bev_offs[i + 1] = w.bev_offs[i] + (uint64_t)beams[i].long_dim * kNpix;
-        est += frustum_voxels(beams[i], ctx->vol);
-    }
+    for (int i = 0; i < n; i++) w.bev_offs[i + 1] = w.bev_offs[i] + (uint64_t)beams[i].long_dim * kNpix;
     const uint64_t bev = w.bev_offs[n];
-    if (w.cand_per_beamlet <= 0) w.cand_per_beamlet = 2.0;  // candidates per frustum voxel, first guess
-    uint64_t cap = std::max<uint64_t>((uint64_t)std::ceil(w.cand_per_beamlet * est), 1024);
+    double est = 0;
+    uint64_t cap = candidate_estimate(ctx, w, beams, n, &est);
 
     w.desc_valid = false;  // the batch's descriptors replace the single-stage ones
     FD_TRY(w.desc.reserve(n));
@@ -609,7 +599,6 @@ int run_batch(const fd_ctx* ctx, Workspace& w, int options, const fd_beam* beams
     CsrDst dst0 = sink ? *sink : dst1;
     if (w.tab_n_gt)
         for (int i = 0; i < n; i++) w.stage[i].geom = w.tab_geom[i];
-    w.host_totals[3] = 0;
 
     // Everything from the uploads to the host copies of the totals is one stream-ordered sequence
     // with no host synchronisation, so it can run as a captured HIP graph (FD_OPT_GRAPH).
@@ -643,11 +632,7 @@ int run_batch(const fd_ctx* ctx, Workspace& w, int options, const fd_beam* beams
         else
             FD_TRY(launch_count(ctx, w, n, st));
         FD_TRY(launch_values(ctx, w, n, w.dose_bev.ptr, extent, thr, cap, st));
-        FD_TRY(run_resample_compact(ctx, w, n, thr, w.rowoff.ptr, dst0, dst1, st));
-        FD_TRY(fetch_totals(ctx, w, n, st, true));
-        if (w.tab_n_gt)  // the table overflow flag into the low half of host_totals[3]
-            FD_HIP(hipMemcpyAsync(w.host_totals + 3, w.flags.ptr + 2, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-        return FD_OK;
+        return run_resample_compact(ctx, w, n, thr, w.rowoff.ptr, dst0, dst1, true, st);
     };
     if (options & FD_OPT_GRAPH) {
         if (!stream) {
@@ -699,11 +684,10 @@ int run_batch(const fd_ctx* ctx, Workspace& w, int options, const fd_beam* beams
         FD_TRY(w.tmp_vals.reserve(cap));
         FD_TRY(w.out_cols.reserve(cap));
         FD_TRY(w.out_vals.reserve(cap));
-        FD_TRY(launch_values(ctx, w, n, w.dose_bev.ptr, extent, thr, cap, stream));
+        FD_TRY(launch_values(ctx, w, n, w.dose_bev.ptr, extent, thr, cap, stream, true));
         dst1 = CsrDst{w.out_cols.ptr, w.out_vals.ptr, cap};
         if (!sink) dst0 = dst1;
-        FD_TRY(run_resample_compact(ctx, w, n, thr, w.rowoff.ptr, dst0, dst1, stream));
-        FD_TRY(fetch_totals(ctx, w, n, stream, true));
+        FD_TRY(run_resample_compact(ctx, w, n, thr, w.rowoff.ptr, dst0, dst1, true, stream));
         FD_HIP(hipStreamSynchronize(stream));
         if (w.host_totals[2]) {
             set_error("resampler staging overflow with exact sizing");

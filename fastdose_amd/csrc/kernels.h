@@ -64,9 +64,10 @@ hipError_t launch_cccs(const BeamletDev* beams, int n, int max_L, const ConeTabl
                        const CccsTables* tab = nullptr);
 
 // Resampling into CSR rows.  Stage 1 counts candidate voxels per (beamlet, z-plane) segment and
-// records the rows [y_lo, y_hi) of the segment that hold them in cand_rows ((0, 0) when none).
+// records the rows [y_lo, y_hi) of the segment that hold them in cand_rows ((0, 0) when none).  Clears
+// overflow[0] for stage 2.
 hipError_t launch_resample_count(const BeamletDev* beams, int n, const fd_volume& vol, uint32_t* cand_count,
-                                 uint2* cand_rows, hipStream_t stream);
+                                 uint2* cand_rows, uint32_t* overflow, hipStream_t stream);
 // Stage 2: values of every candidate, nonzeros compacted in voxel order into tmp_cols/tmp_vals
 // at cand_off[b * Z + z]; nonzero counts into nnz_count.  A segment whose candidates would end
 // beyond `cap` entries writes nothing, gets a zero count and sets overflow[0] = 1.
@@ -88,11 +89,13 @@ hipError_t launch_resample_threshold_count(int n, int Z, const uint64_t* cand_of
 // those >= thr * rowmax); row offsets from nnz_off.  The entries go to dst0 when its capacity
 // holds the total (nnz_off[n Z]), else to dst1 when that one does, else nowhere (the columns and
 // values are left untouched; the offsets are still written).  A destination with a null array
-// counts as capacity 0.
+// counts as capacity 0.  host_offsets (nullable) and host_totals: pinned host memory that receives the row
+// offsets again, and the candidates (cand_off[n Z]), nonzeros, flags[0] and flags[2].
 hipError_t launch_resample_compact(int n, int Z, const uint64_t* cand_off, const uint64_t* nnz_off,
                                    const uint32_t* nnz_count, const uint64_t* tmp_cols, const float* tmp_vals,
-                                   const uint32_t* rowmax_bits, float thr, uint64_t* offsets, CsrDst dst0,
-                                   CsrDst dst1, hipStream_t stream);
+                                   const uint32_t* rowmax_bits, float thr, const uint32_t* flags, uint64_t* offsets,
+                                   uint64_t* host_offsets, uint64_t* host_totals, CsrDst dst0, CsrDst dst1,
+                                   hipStream_t stream);
 
 // Exclusive scan of count[0..N) (u32) into off[0..N) (u64) plus total[0] = sum.  With scratch
 // (scan_scratch_size(N) u64, nullable) large inputs take a three-pass multi-workgroup scan.

@@ -128,9 +128,11 @@ constexpr int kCountPlanes = 8;
 __global__ __launch_bounds__(kRowThreads) void resample_count_kernel(const BeamletDev* __restrict__ beams, int X,
                                                                      int Y, int Z, float vsx, float vsy, float vsz,
                                                                      uint32_t* __restrict__ cand_count,
-                                                                     uint2* __restrict__ cand_rows) {
+                                                                     uint2* __restrict__ cand_rows,
+                                                                     uint32_t* __restrict__ overflow) {
     __shared__ uint32_t s_cnt[kCountPlanes], s_ylo[kCountPlanes], s_yhi[kCountPlanes];
     const int z0 = blockIdx.x * kCountPlanes, b = blockIdx.y;
+    if (blockIdx.x == 0 && b == 0 && threadIdx.x == 0) overflow[0] = 0u;  // for the values pass
     const BeamletDev& B = beams[b];
     const double rho = rho_of(vsx, vsy, vsz);
     // Planes (rows) whose voxel centres lie outside the z-range (y-range) of the widened frustum
@@ -518,22 +520,35 @@ __global__ __launch_bounds__(256) void rcp_check_kernel(int exp0, uint32_t* __re
     if (r != 1.0f / b) atomicAdd(mismatches, 1u);
 }
 
-__global__ void row_offsets_kernel(int n, int Z, const uint64_t* __restrict__ nnz_off,
-                                   const uint64_t* __restrict__ total, uint64_t* __restrict__ offsets) {
+// Row offsets, and what the host waits for, written straight into its pinned memory: three or four
+// small copies after the last kernel took about as long as the kernel itself each.
+__global__ void row_offsets_kernel(int n, int Z, const uint64_t* __restrict__ cand_off,
+                                   const uint64_t* __restrict__ nnz_off, const uint32_t* __restrict__ flags,
+                                   uint64_t* __restrict__ offsets, uint64_t* __restrict__ host_offsets,
+                                   uint64_t* __restrict__ host_totals) {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b < n) offsets[b] = nnz_off[(size_t)b * Z];
-    if (b == n) offsets[n] = total[0];
+    if (b <= n) {
+        const uint64_t o = nnz_off[(size_t)b * Z];  // b = n: the total
+        offsets[b] = o;
+        if (host_offsets) host_offsets[b] = o;
+    }
+    if (b == 0) {
+        host_totals[0] = cand_off[(size_t)n * Z];
+        host_totals[1] = nnz_off[(size_t)n * Z];
+        host_totals[2] = flags[0];
+        host_totals[3] = flags[2];
+    }
 }
 
 }  // namespace
 
 hipError_t launch_resample_count(const BeamletDev* beams, int n, const fd_volume& vol, uint32_t* cand_count,
-                                 uint2* cand_rows, hipStream_t stream) {
+                                 uint2* cand_rows, uint32_t* overflow, hipStream_t stream) {
     if (n <= 0) return hipSuccess;
     dim3 grid((vol.dim[2] + kCountPlanes - 1) / kCountPlanes, n), block(kRowThreads);
     hipLaunchKernelGGL(resample_count_kernel, grid, block, 0, stream, beams, (int)vol.dim[0], (int)vol.dim[1],
                        (int)vol.dim[2], vol.voxel_size[0], vol.voxel_size[1], vol.voxel_size[2], cand_count,
-                       cand_rows);
+                       cand_rows, overflow);
     return hipGetLastError();
 }
 
@@ -571,8 +586,9 @@ hipError_t launch_resample_threshold_count(int n, int Z, const uint64_t* cand_of
 
 hipError_t launch_resample_compact(int n, int Z, const uint64_t* cand_off, const uint64_t* nnz_off,
                                    const uint32_t* nnz_count, const uint64_t* tmp_cols, const float* tmp_vals,
-                                   const uint32_t* rowmax_bits, float thr, uint64_t* offsets, CsrDst dst0,
-                                   CsrDst dst1, hipStream_t stream) {
+                                   const uint32_t* rowmax_bits, float thr, const uint32_t* flags, uint64_t* offsets,
+                                   uint64_t* host_offsets, uint64_t* host_totals, CsrDst dst0, CsrDst dst1,
+                                   hipStream_t stream) {
     if (n <= 0) return hipSuccess;
     dim3 grid(Z, n), block(256);
     const uint64_t* total = nnz_off + (size_t)n * Z;
@@ -591,8 +607,8 @@ hipError_t launch_resample_compact(int n, int Z, const uint64_t* cand_off, const
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     // nnz_off has n*Z entries followed by the total at index n*Z
-    hipLaunchKernelGGL(row_offsets_kernel, dim3((n + 1 + 255) / 256), dim3(256), 0, stream, n, Z, nnz_off,
-                       nnz_off + (size_t)n * Z, offsets);
+    hipLaunchKernelGGL(row_offsets_kernel, dim3((n + 1 + 255) / 256), dim3(256), 0, stream, n, Z, cand_off, nnz_off,
+                       flags, offsets, host_offsets, host_totals);
     return hipGetLastError();
 }
 
