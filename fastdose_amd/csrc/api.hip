@@ -578,6 +578,17 @@ int fd_resample_csr(fd_ctx* ctx, const fd_beam* beams, int n, const float* dose_
     return FD_OK;
 }
 
+int fd_resample_capacity(fd_ctx* ctx, const fd_beam* beams, int n, uint64_t* capacity) {
+    if (!ctx || !capacity) {
+        set_error("null argument");
+        return FD_ERR_ARG;
+    }
+    FD_TRY(check_beams(beams, n));
+    double frustum;
+    *capacity = n > 0 ? candidate_estimate(ctx, ctx->ws, beams, n, &frustum) : 0;
+    return FD_OK;
+}
+
 int fd_dense_to_csr(const float* dense_dev, uint64_t rows, uint64_t cols, fd_csr* out, void* stream) {
     if (!out || !out->offsets || (rows > 0 && cols > 0 && !dense_dev)) {
         set_error("null argument");

@@ -216,19 +216,24 @@ class Context:
         arr = beam_array(beams)
         n = len(arr)
         dev = dose_dev.device
-        offsets = torch.zeros(n + 1, dtype=torch.int64, device=dev)
-        csr = CSR(0, 0, 0, offsets.data_ptr(), None, None)
-        rc = load().fd_resample_csr(self._h, arr, n, C.c_void_p(dose_dev.data_ptr()), stride, extent,
-                                    C.byref(csr), _stream_arg(stream))
-        if rc not in (_lib.FD_OK, _lib.FD_ERR_CAPACITY):
-            _lib.check(rc, "fd_resample_csr")
-        nnz = int(csr.nnz)
-        cols = torch.empty(max(nnz, 1), dtype=torch.int64, device=dev)
-        vals = torch.empty(max(nnz, 1), dtype=torch.float32, device=dev)
-        if rc == _lib.FD_ERR_CAPACITY:
-            csr = CSR(0, 0, nnz, offsets.data_ptr(), cols.data_ptr(), vals.data_ptr())
-            call("fd_resample_csr", self._h, arr, n, C.c_void_p(dose_dev.data_ptr()), stride, extent, C.byref(csr),
-                 _stream_arg(stream))
+        offsets = torch.empty(n + 1, dtype=torch.int64, device=dev)
+        cap = C.c_uint64()
+        call("fd_resample_capacity", self._h, arr, n, C.byref(cap))
+        # room for the estimate, so that one call does; twice only when it was too small
+        while True:
+            room = max(cap.value, 1)
+            cols = torch.empty(room, dtype=torch.int64, device=dev)
+            vals = torch.empty(room, dtype=torch.float32, device=dev)
+            csr = CSR(0, 0, room, offsets.data_ptr(), cols.data_ptr(), vals.data_ptr())
+            rc = load().fd_resample_csr(self._h, arr, n, C.c_void_p(dose_dev.data_ptr()), stride, extent,
+                                        C.byref(csr), _stream_arg(stream))
+            nnz = int(csr.nnz)
+            if rc != _lib.FD_ERR_CAPACITY:
+                break
+            cap.value = nnz
+        _lib.check(rc, "fd_resample_csr")
+        if room > 2 * nnz + 1024:  # the result should not hold on to much more memory than it needs
+            return offsets, cols[:nnz].clone(), vals[:nnz].clone()
         return offsets, cols[:nnz], vals[:nnz]
 
     def cccs_segments(self, beams) -> np.ndarray:

@@ -236,6 +236,12 @@ int fd_cccs(fd_ctx* ctx, const fd_beam* beams, int n, const float* terma_dev, co
 int fd_resample_csr(fd_ctx* ctx, const fd_beam* beams, int n, const float* dose_bev_dev, uint64_t stride,
                     float extent, fd_csr* out, void* stream);
 
+/* The capacity that fd_resample_csr is likely to need for these beamlets (host only; from their
+ * frustums' volume and what earlier calls on this context found).  A caller that allocates so many
+ * entries up front needs one call; no counterpart in the reference, whose dense intermediate has a
+ * fixed size. */
+int fd_resample_capacity(fd_ctx* ctx, const fd_beam* beams, int n, uint64_t* capacity);
+
 /* cusparseDenseToSparse as used by MatCSREnsemble::addMat (IMRTSparseMatEns.cu:78-161):
  * row-major dense (dev) -> CSR.  Same two-phase capacity rule as fd_resample_csr. */
 int fd_dense_to_csr(const float* dense_dev, uint64_t rows, uint64_t cols, fd_csr* out, void* stream);
