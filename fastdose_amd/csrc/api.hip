@@ -397,13 +397,13 @@ int fd_ctx_create(int device, const fd_volume* vol, const float* density_host, c
     if ((e = hipMemcpy(c->density, density_host, nvox * sizeof(float), hipMemcpyHostToDevice)) != hipSuccess)
         return fail(e, "density upload");
     {
-        // per-voxel trilinear cell records for the Terma ray trace (built on the device)
+        // per-voxel trilinear corner records for the Terma ray trace (built on the device)
         const size_t nrec = density_records_floats(*vol);
-        if ((e = hipMalloc((void**)&c->cells, nrec * sizeof(float))) != hipSuccess)
-            return fail(e, "hipMalloc density cell records");
-        if ((e = launch_expand_density(c->density, *vol, c->cells, nullptr)) != hipSuccess ||
+        if ((e = hipMalloc((void**)&c->density_pad, nrec * sizeof(float))) != hipSuccess)
+            return fail(e, "hipMalloc density corner records");
+        if ((e = launch_expand_density(c->density, *vol, c->density_pad, nullptr)) != hipSuccess ||
             (e = hipDeviceSynchronize()) != hipSuccess)
-            return fail(e, "density cell records");
+            return fail(e, "density corner records");
     }
     if ((e = rcp_exact_on_device(c->device, c->rcp_exact)) != hipSuccess) return fail(e, "reciprocal check");
     if ((e = hipMalloc((void**)&c->spec_tab, tab.size() * sizeof(float))) != hipSuccess)
@@ -430,7 +430,7 @@ int fd_ctx_destroy(fd_ctx* ctx) {
     (void)hipSetDevice(ctx->device);
     (void)hipDeviceSynchronize();
     if (ctx->density) (void)hipFree(ctx->density);
-    if (ctx->cells) (void)hipFree(ctx->cells);
+    if (ctx->density_pad) (void)hipFree(ctx->density_pad);
     if (ctx->cones_dev) (void)hipFree(ctx->cones_dev);
     if (ctx->spec_tab) (void)hipFree(ctx->spec_tab);
     ctx->ws.release();

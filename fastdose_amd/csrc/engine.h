@@ -211,7 +211,7 @@ struct fd_ctx {
     int device = 0;
     fd_volume vol{};
     float* density = nullptr;
-    float* cells = nullptr;  // per-voxel trilinear cell records of the density (Terma)
+    float* density_pad = nullptr;  // per-voxel trilinear corner records of the density (Terma)
     fd_spectrum spectrum{};
     fd_kernel kernel{};
     fdi::SpectrumDev spec_dev{};

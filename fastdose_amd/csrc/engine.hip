@@ -282,7 +282,7 @@ int run_terma(const fd_ctx* ctx, Workspace& w, int options, int n, const float* 
     // the per-cone partial buffer (4 floats per BEV value at least) is free until the CCCS stage
     FD_TRY(reserve_cccs(ctx, w, bev_floats));
     w.mark(FD_T_TERMA, 0, stream);
-    hipError_t e = launch_terma(w.desc.ptr, n, fluence, ctx->cells, ctx->vol, ctx->spec_dev, rpl64_len, terma,
+    hipError_t e = launch_terma(w.desc.ptr, n, fluence, ctx->density_pad, ctx->vol, ctx->spec_dev, rpl64_len, terma,
                                 dens, w.partial.ptr, ctx->tune.terma_segments, stream);
     w.mark(FD_T_TERMA, 1, stream);
     if (e != hipSuccess) {

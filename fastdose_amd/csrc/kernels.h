@@ -19,18 +19,18 @@ struct CsrDst {
 hipError_t launch_beamlet_flags(const FlagBeamDev* beams, int n, int max_pixels, const uint8_t* mask,
                                 const fd_volume& vol, uint32_t* box, uint8_t* flags, hipStream_t stream);
 
-// Per-voxel trilinear cell records of the density (8 floats per base voxel of the zero-bordered
+// Per-voxel trilinear corner records of the density (8 floats per base voxel of the zero-bordered
 // volume, 4 x 4 x 4 bricks) for the Terma kernel; density_records_floats(vol) floats.
 uint64_t density_records_floats(const fd_volume& vol);
 hipError_t launch_expand_density(const float* density, const fd_volume& vol, float* records, hipStream_t stream);
 
 // Terma + mean density along the 256 BEV rays of each beamlet (TermaComp.cu:179-253).
-// cells: the records of launch_expand_density.
+// density_pad: the corner records of launch_expand_density.
 // scratch: 4 floats per BEV value (the layout of terma, 16-byte aligned), overwritten.
 // segments: ray segments per ray (1, 2, 4, 8 or 16); a workgroup holds min(256, 1024 / segments)
 // rays times `segments` threads, so with 8 or 16 a beamlet takes two or four workgroups.
 // Beamlets with long_dim * long_spacing > rpl64_len [cm] accumulate the radiological path in FP64.
-hipError_t launch_terma(const BeamletDev* beams, int n, const float* fluence, const float* cells,
+hipError_t launch_terma(const BeamletDev* beams, int n, const float* fluence, const float* density_pad,
                         const fd_volume& vol, const SpectrumDev& spec, float rpl64_len, float* terma,
                         float* dens_bev, float* scratch, int segments, hipStream_t stream);
 

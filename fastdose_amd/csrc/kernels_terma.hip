@@ -8,16 +8,10 @@
 // and the density output is the substep mean of rho.  The spectrum sum is read from a table over
 // the radiological depth built with the context (linear interpolation, error below ~5e-6).  The
 // density is sampled with a hand-written trilinear filter (texel centres at i + 0.5, zero outside
-// the volume) instead of a texture unit.  It reads per-voxel cell records built once per context (the
-// trilinear polynomial of the voxel's cell with a zero border, in 4 x 4 x 4 bricks): one 32-byte
-// read per sample instead of eight gathers, no bounds tests per corner, and rays of any direction
+// the volume) instead of a texture unit.  It reads per-voxel corner records built once per context
+// (the eight corners of the voxel's trilinear cell with a zero border, in 4 x 4 x 4 bricks): one
+// 32-byte read per sample instead of eight gathers, no bounds tests, and rays of any direction
 // share cache lines.
-//
-// It was bound by vector instructions (0.92 issued per CU and cycle at 256 beamlets of 175 slices), so
-// they are what the sample is written for: positions advance by a per-ray step, floors and fractions
-// are one instruction each, record offsets fit 32 bits where the records do, and the polynomial takes
-// seven FMAs where the corners took ten operations.  45.4 -> 33.7 M wavefront instructions, 80 -> 68 us;
-// now 0.76 issued per cycle, the rest waits for records and stores.
 //
 // The radiological path is a prefix sum along each ray, which one lane per ray would walk alone
 // (256 rays per beamlet: one wavefront per SIMD on small batches).  Each ray is cut into 1, 2, 4,
@@ -41,23 +35,14 @@ namespace {
 constexpr int kTermaThreads = 1024;  // workgroup size limit: ray segments x rays per workgroup
 constexpr int kTermaMaxSeg = 16;    // most ray segments (16: four workgroups of 64 rays per beamlet)
 
-// Cell records: for every base voxel (x, y, z) in [0, X] x [0, Y] x [0, Z] of the density with a
-// one-voxel zero border, the trilinear polynomial of its cell (corners x..x+1, y..y+1, z..z+1) in the
-// offsets (ax, ay, az) from the base corner, rho = (a + b ax) + (c + d ax) ay + ((e + f ax) +
-// (g + h ax) ay) az, as two float4 (a, b, c, d), (e, f, g, h): seven FMAs a sample.  Coefficients in FP64
-// from the corners, rounded once.  Records in 4 x 4 x 4 bricks: record
+// Corner records: for every base voxel (x, y, z) in [0, X] x [0, Y] x [0, Z] of the density with a
+// one-voxel zero border, its eight trilinear corners c0..c7 (x..x+1, y..y+1, z..z+1; x fastest) as
+// two float4 (c0, c1 - c0, c2, c3 - c2), (c4, c5 - c4, c6, c7 - c6): the x differences the first
+// interpolation step needs, rounded as it would round them.  Records in 4 x 4 x 4 bricks: record
 // ((z/4 nby + y/4) nbx + x/4) 64 + 16 (z%4) + 4 (y%4) + x%4, nb* = ceil((dim + 1) / 4).  A sample
 // reads one 32-byte record.
-// Index: uint64_t, or uint32_t for records that span less than 4 GiB (then fewer than 2^21 bricks, and
-// 24-bit products do).
-template <typename Index>
-__device__ __forceinline__ Index cell_record(uint32_t x, uint32_t y, uint32_t z, uint32_t nbx, uint32_t nby) {
-    Index brick;
-    if constexpr (sizeof(Index) == 4)
-        brick = __umul24(__umul24(z >> 2, nby) + (y >> 2), nbx) + (x >> 2);
-    else
-        brick = ((Index)(z >> 2) * nby + (y >> 2)) * nbx + (x >> 2);
-    return (((((brick << 2) + (z & 3)) << 2) + (y & 3)) << 2) + (x & 3);
+__device__ __forceinline__ uint64_t corner_record(uint32_t x, uint32_t y, uint32_t z, uint32_t nbx, uint32_t nby) {
+    return ((((uint64_t)(z >> 2) * nby + (y >> 2)) * nbx + (x >> 2)) << 6) + ((z & 3) << 4) + ((y & 3) << 2) + (x & 3);
 }
 
 __global__ __launch_bounds__(256) void expand_density_kernel(const float* __restrict__ density, int X, int Y, int Z,
@@ -66,60 +51,54 @@ __global__ __launch_bounds__(256) void expand_density_kernel(const float* __rest
     const uint64_t nx = (uint64_t)X + 1, ny = (uint64_t)Y + 1, nz = (uint64_t)Z + 1;
     if (i >= nx * ny * nz) return;
     const uint32_t x = (uint32_t)(i % nx), y = (uint32_t)((i / nx) % ny), z = (uint32_t)(i / (nx * ny));
-    double v[8];
+    float v[8];
 #pragma unroll
     for (int c = 0; c < 8; c++) {
         // padded coordinate x + (c & 1) is original coordinate x + (c & 1) - 1
         const int ox = (int)x + (c & 1) - 1, oy = (int)y + ((c >> 1) & 1) - 1, oz = (int)z + (c >> 2) - 1;
         const bool in = ox >= 0 && ox < X && oy >= 0 && oy < Y && oz >= 0 && oz < Z;
-        v[c] = in ? (double)density[((size_t)oz * Y + oy) * X + ox] : 0.0;
+        v[c] = in ? density[((size_t)oz * Y + oy) * X + ox] : 0.0f;
     }
-    const double bx0 = v[1] - v[0], bx1 = v[3] - v[2], bx2 = v[5] - v[4], bx3 = v[7] - v[6];
-    const uint64_t r = cell_record<uint64_t>(x, y, z, nbx, nby);
-    out[2 * r] = make_float4((float)v[0], (float)bx0, (float)(v[2] - v[0]), (float)(bx1 - bx0));
-    out[2 * r + 1] = make_float4((float)(v[4] - v[0]), (float)(bx2 - bx0), (float)((v[6] - v[4]) - (v[2] - v[0])),
-                                 (float)((bx3 - bx2) - (bx1 - bx0)));
+    const uint64_t r = corner_record(x, y, z, nbx, nby);
+    out[2 * r] = make_float4(v[0], v[1] - v[0], v[2], v[3] - v[2]);
+    out[2 * r + 1] = make_float4(v[4], v[5] - v[4], v[6], v[7] - v[6]);
 }
 
-// floor(v) as an integer, and v - floor(v)
-__device__ __forceinline__ int floor_int(float v) {
-    int r;
-    asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(r) : "v"(v));
-    return r;
-}
-
-// Trilinear density at position g (voxel units plus one half: base voxel floor(g), texel centres at
-// i + 0.5 of the volume's own units, zero outside) from the cell records (nbx, nby: bricks along x and
-// y).  The last record read stays in registers: consecutive samples of a ray are a fraction of a voxel
-// apart (four per slice), so most fall in the base voxel of the one before and need no load; a lane
-// loads only when its base voxel changes.  (r, lo, hi): the record held, r = ~0 for none.
-template <typename Index>
-__device__ __forceinline__ float density_at(const float4* __restrict__ rec, uint32_t X, uint32_t Y, uint32_t Z,
-                                            uint32_t nbx, uint32_t nby, float gx, float gy, float gz, Index& r,
-                                            float4& lo, float4& hi) {
-    const uint32_t x = (uint32_t)floor_int(gx), y = (uint32_t)floor_int(gy), z = (uint32_t)floor_int(gz);
+// Trilinear density at voxel-unit position (cx, cy, cz) (texel centres at i + 0.5, zero outside
+// the volume) from the corner records (nbx, nby: bricks along x and y).  The last record read stays
+// in registers: consecutive samples of a ray are a fraction of a voxel apart (four per slice), so
+// most fall in the base voxel of the one before and need no load; a lane loads only when its base
+// voxel changes.  (r, lo, hi): the record held, r = ~0 for none.
+__device__ __forceinline__ float density_at(const float4* __restrict__ rec, int X, int Y, int Z, uint32_t nbx,
+                                            uint32_t nby, float cx, float cy, float cz, uint64_t& r, float4& lo,
+                                            float4& hi) {
+    const float xb = cx - 0.5f, yb = cy - 0.5f, zb = cz - 0.5f;
+    const float fx = floorf(xb), fy = floorf(yb), fz = floorf(zb);
     // outside: every corner is in the zero border or beyond (and the record index stays in range)
-    if (!(x <= X && y <= Y && z <= Z)) return 0.0f;
-    const Index rn = cell_record<Index>(x, y, z, nbx, nby);
+    if (!(fx > -2.0f && fx < (float)X && fy > -2.0f && fy < (float)Y && fz > -2.0f && fz < (float)Z)) return 0.0f;
+    const float ax = xb - fx, ay = yb - fy, az = zb - fz;
+    const uint64_t rn =
+        corner_record((uint32_t)((int)fx + 1), (uint32_t)((int)fy + 1), (uint32_t)((int)fz + 1), nbx, nby);
     if (rn != r) {
-        const char* at = reinterpret_cast<const char*>(rec) + (Index)(rn * 32);
-        lo = reinterpret_cast<const float4*>(at)[0];
-        hi = reinterpret_cast<const float4*>(at)[1];
+        lo = rec[2 * rn];
+        hi = rec[2 * rn + 1];
         r = rn;
     }
-    const float ax = __builtin_amdgcn_fractf(gx), ay = __builtin_amdgcn_fractf(gy), az = __builtin_amdgcn_fractf(gz);
-    const float c0 = fmaf(fmaf(ax, lo.w, lo.z), ay, fmaf(ax, lo.y, lo.x));
-    const float c1 = fmaf(fmaf(ax, hi.w, hi.z), ay, fmaf(ax, hi.y, hi.x));
-    return fmaf(az, c1, c0);
+    const float c00 = fmaf(ax, lo.y, lo.x);
+    const float c10 = fmaf(ax, lo.w, lo.z);
+    const float c01 = fmaf(ax, hi.y, hi.x);
+    const float c11 = fmaf(ax, hi.w, hi.z);
+    const float c0 = fmaf(ay, c10 - c00, c00);
+    const float c1 = fmaf(ay, c11 - c01, c01);
+    return fmaf(az, c1 - c0, c0);
 }
 
 // rpl64_len: beamlets whose central-axis path (long_dim * long_spacing) exceeds this many cm
 // accumulate the radiological path in FP64 (0: every beamlet; infinity: none).
 // Workgroup (beamlet blockIdx.x, ray block blockIdx.y): `rays` consecutive BEV pixels (a multiple
 // of 64) times blockDim.x / rays segments.
-template <typename Index>
 __global__ __launch_bounds__(kTermaThreads) __attribute__((amdgpu_waves_per_eu(8, 8))) void terma_kernel(
-    const BeamletDev* __restrict__ beams, const float* __restrict__ fluence, const float* __restrict__ cells,
+    const BeamletDev* __restrict__ beams, const float* __restrict__ fluence, const float* __restrict__ density_pad,
     int X, int Y, int Z, float vsx, float vsy, float vsz, SpectrumDev spec, float rpl64_len,
     float* __restrict__ terma, float* __restrict__ dens_bev, float4* __restrict__ scratch, int rays) {
     __shared__ float s_seg[kTermaThreads];
@@ -143,31 +122,26 @@ __global__ __launch_bounds__(kTermaThreads) __attribute__((amdgpu_waves_per_eu(8
     const float dt = B.ls / (B.sad * kSuperSampling);
     const float step_len = sqrtf(px * px + py * py + pz * pz) * dt;
     const float t0 = B.lim_min / B.sad;
-    // sample k at g(k) = g0 + k dg: position (src + p (t0 + k dt)) / vs in voxel units, plus one half
-    // (density_at); origin and step in FP64, rounded once
-    const double dtd = (double)B.ls / ((double)B.sad * kSuperSampling), t0d = (double)B.lim_min / (double)B.sad;
-    const float dgx = (float)((double)px * dtd / vsx), dgy = (float)((double)py * dtd / vsy),
-                dgz = (float)((double)pz * dtd / vsz);
-    const float g0x = (float)(((double)B.src[0] + (double)px * t0d) / vsx + 0.5),
-                g0y = (float)(((double)B.src[1] + (double)py * t0d) / vsy + 0.5),
-                g0z = (float)(((double)B.src[2] + (double)pz * t0d) / vsz + 0.5);
+    // positions in voxel units: c(t) = (src + p t) / vs
+    const float ax = px / vsx, ay = py / vsy, az = pz / vsz;
+    const float sx = B.src[0] / vsx, sy = B.src[1] / vsy, sz = B.src[2] / vsz;
     const float fl = fluence[(size_t)b * kNpix + p];
     const bool lit = fl != 0.0f;
 
     const uint32_t nbx = ((uint32_t)X + 4) / 4, nby = ((uint32_t)Y + 4) / 4;
-    const float4* __restrict__ rec = reinterpret_cast<const float4*>(cells);
-    Index rc = ~(Index)0;
+    const float4* __restrict__ rec = reinterpret_cast<const float4*>(density_pad);
+    uint64_t rc = ~uint64_t(0);
     float4 rlo = make_float4(0.0f, 0.0f, 0.0f, 0.0f), rhi = rlo;
-    auto rho_at = [&](float k) {
-        return density_at<Index>(rec, X, Y, Z, nbx, nby, fmaf(k, dgx, g0x), fmaf(k, dgy, g0y), fmaf(k, dgz, g0z), rc,
-                                rlo, rhi);
+    auto rho_at = [&](int k) {
+        const float t = fmaf((float)k, dt, t0);
+        return density_at(rec, X, Y, Z, nbx, nby, fmaf(ax, t, sx), fmaf(ay, t, sy), fmaf(az, t, sz), rc, rlo, rhi);
     };
     // the FP64 path's second walk keeps no record in registers (fewer live registers there)
-    auto rho_fresh = [&](float k) {
-        Index r = ~(Index)0;
+    auto rho_fresh = [&](int k) {
+        const float t = fmaf((float)k, dt, t0);
+        uint64_t r = ~uint64_t(0);
         float4 lo, hi;
-        return density_at<Index>(rec, X, Y, Z, nbx, nby, fmaf(k, dgx, g0x), fmaf(k, dgy, g0y), fmaf(k, dgz, g0z), r,
-                                lo, hi);
+        return density_at(rec, X, Y, Z, nbx, nby, fmaf(ax, t, sx), fmaf(ay, t, sy), fmaf(az, t, sz), r, lo, hi);
     };
 
     float* __restrict__ T = terma + B.bev_off + p;
@@ -184,7 +158,7 @@ __global__ __launch_bounds__(kTermaThreads) __attribute__((amdgpu_waves_per_eu(8
         float q[kSuperSampling];
 #pragma unroll
         for (int j = 0; j < kSuperSampling; j++) {
-            const float rho = rho_at((float)(kSuperSampling * i + j + 1));
+            const float rho = rho_at(kSuperSampling * i + j + 1);
             if (RPL64)
                 lpath64 += (double)rho * (double)step_len;
             else
@@ -226,7 +200,7 @@ __global__ __launch_bounds__(kTermaThreads) __attribute__((amdgpu_waves_per_eu(8
             const float t = fmaf((float)k, dt, t0);
             float path;
             if (RPL64) {
-                rpl64 += (double)rho_fresh((float)k) * (double)step_len;
+                rpl64 += (double)rho_fresh(k) * (double)step_len;
                 path = (float)rpl64;
             } else {
                 path = seg == 0 ? q[j] : rpl + q[j];
@@ -259,7 +233,7 @@ hipError_t launch_expand_density(const float* density, const fd_volume& vol, flo
     return hipGetLastError();
 }
 
-hipError_t launch_terma(const BeamletDev* beams, int n, const float* fluence, const float* cells,
+hipError_t launch_terma(const BeamletDev* beams, int n, const float* fluence, const float* density_pad,
                         const fd_volume& vol, const SpectrumDev& spec, float rpl64_len, float* terma,
                         float* dens_bev, float* scratch, int segments, hipStream_t stream) {
     if (n <= 0) return hipSuccess;
@@ -268,9 +242,7 @@ hipError_t launch_terma(const BeamletDev* beams, int n, const float* fluence, co
     const int rays = std::min(kNpix, kTermaThreads / segments);
     dim3 grid(n, kNpix / rays), block(segments * rays);
     const int X = vol.dim[0], Y = vol.dim[1], Z = vol.dim[2];
-    const auto kernel = density_records_floats(vol) * sizeof(float) < (1ull << 32) ? terma_kernel<uint32_t>
-                                                                                   : terma_kernel<uint64_t>;
-    hipLaunchKernelGGL(kernel, grid, block, 0, stream, beams, fluence, cells, X, Y, Z, vol.voxel_size[0],
+    hipLaunchKernelGGL(terma_kernel, grid, block, 0, stream, beams, fluence, density_pad, X, Y, Z, vol.voxel_size[0],
                        vol.voxel_size[1], vol.voxel_size[2], spec, rpl64_len, terma, dens_bev,
                        reinterpret_cast<float4*>(scratch), rays);
     return hipGetLastError();
