@@ -29,7 +29,6 @@
 // cones in a fixed order so results are bitwise reproducible.
 #include <hip/hip_runtime.h>
 
-
 #include "kernels.h"
 
 namespace fdi {
@@ -58,6 +57,13 @@ __device__ __forceinline__ float axis_step(float c, float sgn, float inv) {
 // A wave-uniform float kept in a scalar register.
 __device__ __forceinline__ float uniform(float v) {
     return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+}
+
+// The same wave-uniform value, of which the compiler does not know it: keeps a test of one of its bits
+// in the branch that needs it (hoisted and merged, such tests cost more scalar instructions).
+__device__ __forceinline__ uint32_t apart(uint32_t w) {
+    asm volatile("" : "+s"(w));
+    return w;
 }
 
 // value of the neighbouring lane in the same 16-lane row (DPP row rotation)
@@ -541,8 +547,9 @@ constexpr uint32_t kUnitX = 1u << 30, kUnitY = 1u << 31;
 constexpr uint32_t kShiftBits = 0x3FFu, kResetBits = kColReset | kRowReset | kGeneralReset;
 constexpr int kMaxMarchPhi = 10;  // azimuths of the march kernel (64 KiB of LDS); more: inline kernel
 constexpr int kMaxPhiPerWave1 = 16;  // self-marching kernel: one azimuth per wavefront up to 16, then two
-// A slab in LDS: A/a T, B/b T, -a log2(e) rho and -b log2(e) rho of the slice, 256 each (read by
-// the compute wavefronts when the slice starts), and rho itself (read by the slice's combine).
+// A slab in LDS: A/a T, B/b T, -a log2(e) rho and -b log2(e) rho of the slice, 256 each, read by the
+// compute wavefronts when the slice starts.  Its arrays and the doses are stored in the order in
+// which a lane holds its voxels (lds_place): one 16-byte access per array and lane.
 constexpr int kSlab = 4 * kNpix;
 constexpr float kLn2 = 0.6931471805599453f;
 
@@ -551,8 +558,6 @@ struct CcLds {
     float4* pos;   // [n_phi][kRecCap + 1] lattice points of the chunk being marched
     int2* carry;   // [n_phi] (padded to 2 n_phi) midpoint voxel of the last step marched
     float* slab;   // [2][kSlab], slice i in buffer i & 1
-    float* rho;    // [3][256], slice i in buffer i % 3 (the combine of slice i - 1 still reads its rho
-                   // while slice i + 1 is being prefetched)
     float* sC;     // [2][256], slice i in buffer i & 1
     float* sD;     // [2][n_phi][256], slice i in buffer i & 1
     int* hdr;      // [2][kHdr]
@@ -564,7 +569,7 @@ constexpr int kRecStride = 2 * kRecCap + 1;
 
 __host__ __device__ constexpr size_t march_lds_bytes(int n_phi) {
     return (size_t)2 * n_phi * kRecStride * sizeof(float4) + (size_t)n_phi * (kRecCap + 1) * sizeof(float4) +
-           (size_t)2 * n_phi * sizeof(int2) + (size_t)(2 * kSlab + (3 + 2 + 2 * n_phi) * kNpix) * sizeof(float) +
+           (size_t)2 * n_phi * sizeof(int2) + (size_t)(2 * kSlab + (2 + 2 * n_phi) * kNpix) * sizeof(float) +
            (size_t)2 * kHdr * sizeof(int);
 }
 
@@ -578,8 +583,7 @@ __device__ __forceinline__ CcLds carve_lds(float4* base, int n_phi) {
     S.carry = reinterpret_cast<int2*>(S.pos + n_phi * (kRecCap + 1));
     float* f = reinterpret_cast<float*>(S.carry + 2 * n_phi);
     S.slab = f;
-    S.rho = f + 2 * kSlab;
-    S.sC = S.rho + 3 * kNpix;
+    S.sC = f + 2 * kSlab;
     S.sD = S.sC + 2 * kNpix;
     S.hdr = reinterpret_cast<int*>(S.sD + 2 * n_phi * kNpix);
     return S;
@@ -587,12 +591,12 @@ __device__ __forceinline__ CcLds carve_lds(float4* base, int n_phi) {
 
 // LDS of cccs_tab_kernel: two block buffers per compute wavefront (kTabRec float4: a block of
 // kRecCap records of its azimuth's stream and one more, the read past a chunk's last), two chunk
-// headers, then the slabs, rho, cumulative length and per-azimuth doses as in carve_lds.  Block
+// headers, then the slabs, cumulative length and per-azimuth doses as in carve_lds.  Block
 // b + 1 is loaded into LDS while the chunks of block b run; chunk c's header during chunk c - 1.
 constexpr int kTabRec = 2 * (kRecCap + 1);
 __host__ __device__ constexpr size_t tab_lds_bytes(int n_phi) {
     return (size_t)2 * n_phi * kTabRec * sizeof(float4) + (size_t)2 * kTabHdr * sizeof(int) +
-           (size_t)(2 * kSlab + (3 + 2 + 2 * n_phi) * kNpix) * sizeof(float);
+           (size_t)(2 * kSlab + (2 + 2 * n_phi) * kNpix) * sizeof(float);
 }
 
 __device__ __forceinline__ CcLds carve_lds_tab(float4* base, int n_phi) {
@@ -601,63 +605,106 @@ __device__ __forceinline__ CcLds carve_lds_tab(float4* base, int n_phi) {
     S.hdr = reinterpret_cast<int*>(base + 2 * n_phi * kTabRec);
     float* f = reinterpret_cast<float*>(S.hdr + 2 * kTabHdr);
     S.slab = f;
-    S.rho = f + 2 * kSlab;
-    S.sC = S.rho + 3 * kNpix;
+    S.sC = f + 2 * kSlab;
     S.sD = S.sC + 2 * kNpix;
     return S;
 }
 
-// What every wavefront of the workgroup shares: the beamlet's slabs and output, thread layout.
+// What every wavefront of the workgroup shares: the beamlet's slabs and output, wavefront layout.
 struct CcBlock {
     const float* Tg;
     const float* Rg;
     float* P;
-    int L, tid, nthreads, n_phi;
-    bool two, prefetch;
+    int L, wave, n_waves, n_phi;
     float A_a, B_b, na, nb;  // cone constants the slab is scaled with
 };
 
-// Slab element e = 64 q + lane (q wave-uniform) of slice z: Terma for q < 4, density above, so
-// the source pointer is a scalar and only the lane offset is a vector register.
+// A slice's 256 voxels are four groups of 64 (16 x by 4 y); lane l loads, and combines, voxel 64 q + l
+// of group q, but a compute wavefront's lane holds the four voxels of a column (x, 4 g .. 4 g + 3).
+// Arrays in LDS that compute wavefronts access are in the latter order.
+__device__ __forceinline__ int lds_place(int lane) { return ((lane & 15) << 2) | (lane >> 4); }
+
+// The slab's eight groups are numbered density 0-3, Terma 4-7; wavefront w loads group w and, when
+// there are fewer than eight wavefronts, group w + n_waves.  So wavefront w < 4, which also combines
+// group w, holds that group's density in a register.  Workgroups with less than four wavefronts load
+// each slab when its slice starts, with all wavefronts.  WIDE: at least eight wavefronts.
+template <bool WIDE>
+__device__ __forceinline__ bool loads_ahead(const CcBlock& K) { return WIDE || K.n_waves >= 4; }
+
+// Element lane of a wavefront-uniform address (kept in scalars).
+using GlobalF = __attribute__((address_space(1))) float;
+__device__ __forceinline__ GlobalF* uniform_base(const float* p, uint32_t at) {
+    GlobalF* b = (GlobalF*)(p + at);
+    asm("" : "+s"(b));
+    return b;
+}
 __device__ __forceinline__ float slab_value(const CcBlock& K, int z, int q) {
-    const float* src = (q < 4 ? K.Tg : K.Rg) + (uint32_t)z * kNpix + (q & 3) * kWave;
-    return src[threadIdx.x & 63];
+    return uniform_base(q < 4 ? K.Rg : K.Tg, (uint32_t)z * kNpix + (uint32_t)((q & 3) * kWave))[threadIdx.x & 63];
 }
-// Slab element e (e < 256: Terma, else density; wave-uniform) of slice ordinal si into LDS.
-__device__ __forceinline__ void store_slab(const CcBlock& K, const CcLds& S, int si, int e, float v) {
-    float* slab = S.slab + (si & 1) * kSlab;
-    if (e < kNpix) {
-        slab[e] = K.A_a * v;
-        slab[kNpix + e] = K.B_b * v;
-    } else {
-        slab[kNpix + e] = K.na * v;  // 2 kNpix + (e - kNpix)
-        slab[2 * kNpix + e] = K.nb * v;
-        S.rho[(si % 3) * kNpix + e - kNpix] = v;
-    }
+__device__ __forceinline__ void store_slab(const CcBlock& K, const CcLds& S, int si, int q, float v) {
+    float* slab = S.slab + ((si & 1) * kSlab + (q & 3) * kWave + (q < 4 ? 2 * kNpix : 0)) + lds_place(threadIdx.x & 63);
+    slab[0] = (q < 4 ? K.na : K.A_a) * v;
+    slab[kNpix] = (q < 4 ? K.nb : K.B_b) * v;
 }
-__device__ __forceinline__ void slab_regs(const CcBlock& K, int z, float& pf0, float& pf1) {
-    const int q0 = K.tid >> 6, q1 = (K.tid + K.nthreads) >> 6;  // wave-uniform
-    if (q0 < 8) pf0 = slab_value(K, z, __builtin_amdgcn_readfirstlane(q0));
-    if (K.two && q1 < 8) pf1 = slab_value(K, z, __builtin_amdgcn_readfirstlane(q1));
+// The groups this wavefront loads ahead.
+struct CcAhead {
+    float v0 = 0.0f, v1 = 0.0f;
+};
+template <bool WIDE>
+__device__ __forceinline__ void slab_regs(const CcBlock& K, int z, CcAhead& A) {
+    if (K.wave < 8) A.v0 = slab_value(K, z, K.wave);
+    if (!WIDE && K.wave + K.n_waves < 8) A.v1 = slab_value(K, z, K.wave + K.n_waves);
 }
+template <bool WIDE>
+__device__ __forceinline__ void store_ahead(const CcBlock& K, const CcLds& S, int si, const CcAhead& A) {
+    if (K.wave < 8) store_slab(K, S, si, K.wave, A.v0);
+    if (!WIDE && K.wave + K.n_waves < 8) store_slab(K, S, si, K.wave + K.n_waves, A.v1);
+}
+// The whole slab of slice z, ordinal si, by all wavefronts.
+__device__ __forceinline__ void load_slab(const CcBlock& K, const CcLds& S, int z, int si) {
+    for (int q = K.wave; q < 8; q += K.n_waves) store_slab(K, S, si, q, slab_value(K, z, q));
+}
+__device__ __forceinline__ void zero_slice(const CcBlock& K, int z) {
+    for (int q = K.wave; q < 4; q += K.n_waves)
+        uniform_base(K.P, (uint32_t)z * kNpix + (uint32_t)(q * kWave))[threadIdx.x & 63] = 0.0f;
+}
+
+// Where the march stands, in every wavefront alike.
+struct CcSlice {
+    int s = 0, si = 0, written = 0;  // slice being processed, its ordinal, slices written so far
+    float rho = 0.0f;                // density of this wavefront's group of the slice (loads_ahead, wave < 4)
+};
+template <bool WIDE>
+__device__ __forceinline__ CcSlice first_slice(const CcBlock& K) {
+    CcSlice Z;
+    if (loads_ahead<WIDE>(K) && K.wave < 4) Z.rho = slab_value(K, 0, K.wave);
+    return Z;
+}
+
 // End of a chunk, executed by every wavefront: store the prefetched slab, barrier, and after a
 // slice end the combine of the slice into P.  Returns false once the beamlet is finished.
 // DMA: this wavefront may have loads into LDS in flight (cccs_tab_kernel's next chunk header or
 // record block), complete before the barrier (vector memory operations complete in issue order).
-__device__ __forceinline__ bool chunk_end(const CcBlock& K, const CcLds& S, int done, int sn, float pf0,
-                                          float pf1, int& s, int& si, int& written, bool dma = false) {
-    if (done && sn < K.L && K.prefetch) {
-        const int i0 = K.tid, i1 = K.tid + K.nthreads;
-        if (i0 < 2 * kNpix) store_slab(K, S, si + 1, i0, pf0);
-        if (K.two && i1 < 2 * kNpix) store_slab(K, S, si + 1, i1, pf1);
-    }
+// Runs once per slice and wavefront, against 1.5 to 12 lattice steps of about 60 vector instructions,
+// and a full GPU is bound by instructions issued and fetched (vector units over 95 % busy, 0.77
+// instruction cache fetches per cycle and CU pair): wavefront-uniform conditions and addresses are
+// kept in scalars, the common workgroup (WIDE) has no loops over groups, a lane's four voxels are one
+// LDS access and the combine's density is a register.  Together with the step's X kept in place:
+// cccs_tab_kernel in a 20-beam plan 14.2 -> 13.6 ms, 400 beamlets of cccs_kernel 3.91 -> 3.60 ms,
+// 121 beamlets (one workgroup per CU and a half, latency) 1.20 -> 1.16 ms.
+template <bool WIDE>
+__device__ __forceinline__ bool chunk_end(const CcBlock& K, const CcLds& S, int done, int sn, const CcAhead& A,
+                                          CcSlice& Z, bool dma = false) {
+    if (done && sn < K.L && loads_ahead<WIDE>(K)) store_ahead<WIDE>(K, S, Z.si + 1, A);
     if (dma) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (!done) return true;
     // slice s: rho sum over azimuths (in azimuth order) of the dose in units of geometric length /
     // (rho cumulative length of the last azimuth + 1e-4); the quotient from the hardware reciprocal
-    for (int i = K.tid; i < kNpix; i += K.nthreads) {
-        const float* d = S.sD + (si & 1) * K.n_phi * kNpix + i;
+    const int lane = threadIdx.x & 63;
+    for (int q = K.wave; q < 4; q += K.n_waves) {
+        const int i = q * kWave + lds_place(lane);
+        const float* d = S.sD + (Z.si & 1) * K.n_phi * kNpix + i;
         float sum = 0.0f;
         int f = 0;
         for (; f + 4 <= K.n_phi; f += 4) {  // four reads in flight, summed in azimuth order
@@ -665,27 +712,27 @@ __device__ __forceinline__ bool chunk_end(const CcBlock& K, const CcLds& S, int 
             sum = (((sum + v0) + v1) + v2) + v3;
         }
         for (; f < K.n_phi; f++) sum += d[f * kNpix];
-        const float rho = S.rho[(si % 3) * kNpix + i];
-        K.P[(uint32_t)s * kNpix + i] = sum * rho * __builtin_amdgcn_rcpf(fmaf(S.sC[(si & 1) * kNpix + i], rho, kEps));
+        const float rho = loads_ahead<WIDE>(K) ? Z.rho : slab_value(K, Z.s, q);
+        uniform_base(K.P, (uint32_t)Z.s * kNpix + (uint32_t)(q * kWave))[lane] =
+            sum * rho * __builtin_amdgcn_rcpf(fmaf(S.sC[(Z.si & 1) * kNpix + i], rho, kEps));
+        if (WIDE) break;
     }
-    for (int z = s + 1; z < sn && z < K.L; z++)  // slices the phi-0 march stepped over
-        for (int i = K.tid; i < kNpix; i += K.nthreads) K.P[(uint32_t)z * kNpix + i] = 0.0f;
-    written = sn < K.L ? sn : K.L;
+    for (int z = Z.s + 1; z < sn && z < K.L; z++) zero_slice(K, z);  // slices the phi-0 march stepped over
+    Z.written = sn < K.L ? sn : K.L;
     if (sn >= K.L) return false;
-    if (!K.prefetch) {  // small workgroups load the next slab here
+    if (!loads_ahead<WIDE>(K)) {  // small workgroups load the next slab here
         __syncthreads();
-        for (int i = K.tid; i < 2 * kNpix; i += K.nthreads)
-            store_slab(K, S, si + 1, i, i < kNpix ? K.Tg[(uint32_t)sn * kNpix + i] : K.Rg[(uint32_t)sn * kNpix + i - kNpix]);
+        load_slab(K, S, sn, Z.si + 1);
         __syncthreads();
     }
-    s = sn;
-    si++;
+    Z.rho = A.v0;
+    Z.s = sn;
+    Z.si++;
     return true;
 }
 
 __device__ __forceinline__ void zero_tail(const CcBlock& K, int written) {
-    for (int z = written; z < K.L; z++)
-        for (int i = K.tid; i < kNpix; i += K.nthreads) K.P[(uint32_t)z * kNpix + i] = 0.0f;
+    for (int z = written; z < K.L; z++) zero_slice(K, z);
 }
 
 // March wavefront, in two phases per chunk.  Phase 1: lane f < n_phi marches azimuth f with the
@@ -906,6 +953,7 @@ __device__ __forceinline__ void march_init(MarchLane& M, MarchConst& C, const Co
     C.lf = C.lk < C.kper ? lane - C.lk * n_phi : n_phi;  // n_phi: idle in phase 2
 }
 
+template <bool WIDE>
 __device__ __forceinline__ void cccs_march(const BeamletDev& B, const ConeTable* __restrict__ cones, int t,
                                            const CcBlock& K, const CcLds& S) {
     const int lane = threadIdx.x & 63;
@@ -919,18 +967,19 @@ __device__ __forceinline__ void cccs_march(const BeamletDev& B, const ConeTable*
 
     march_chunk<false>(M, C, K.n_phi, S, S.rec, S.hdr, 0, true);
     __syncthreads();
-    int s = 0, buf = 0, si = 0, written = 0;  // si: ordinal of the slice being processed
+    CcSlice Z = first_slice<WIDE>(K);
+    int buf = 0;
     for (;;) {
         const int done = S.hdr[buf * kHdr + kMaxPhi], sn = S.hdr[buf * kHdr + kMaxPhi + 1];
-        float pf0 = 0.0f, pf1 = 0.0f;
-        if (done && sn < K.L && K.prefetch) slab_regs(K, sn, pf0, pf1);
+        CcAhead ahead;
+        if (done && sn < K.L && loads_ahead<WIDE>(K)) slab_regs<WIDE>(K, sn, ahead);
         if (!(done && sn >= K.L))
             march_chunk<false>(M, C, n_phi, S, S.rec + (buf ^ 1) * n_phi * kRecStride, S.hdr + (buf ^ 1) * kHdr,
-                               done ? sn : s, done != 0);
-        if (!chunk_end(K, S, done, sn, pf0, pf1, s, si, written)) break;
+                               done ? sn : Z.s, done != 0);
+        if (!chunk_end<WIDE>(K, S, done, sn, ahead, Z)) break;
         buf ^= 1;
     }
-    zero_tail(K, written);
+    zero_tail(K, Z.written);
 }
 
 // March tables: one wavefront per (march geometry, forward cone) walks the lattice of every azimuth
@@ -1042,7 +1091,7 @@ static_assert(2 * kRecCap == kWave, "a table block is one 16-byte load per lane"
 // X states are kept pre-scaled by A/a and B/b, and the dose and cumulative length are summed in
 // units of the geometric length s (p = s rho), multiplied by rho in the combine.  TAB: the chunks
 // come from a march table (cccs_tab_kernel), else from the march wavefront's LDS records.
-template <bool EXACT_G, bool CUMU, bool TAB = false>
+template <bool EXACT_G, bool WIDE, bool CUMU, bool TAB = false>
 __device__ __forceinline__ void cccs_compute(const CcBlock& K, const CcLds& S, int wave,
                                              const TabRead& TR = TabRead{}) {
     const int lane = threadIdx.x & 63;
@@ -1050,7 +1099,6 @@ __device__ __forceinline__ void cccs_compute(const CcBlock& K, const CcLds& S, i
 
     const int vx = lane & 15;
     const int g = lane >> 4;
-    const int vbase = vx + 64 * g;
     const int up_lane = (lane + 48) & 63;    // lane (x, g - 1)
     const int down_lane = (lane + 16) & 63;  // lane (x, g + 1)
 
@@ -1074,7 +1122,8 @@ __device__ __forceinline__ void cccs_compute(const CcBlock& K, const CcLds& S, i
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
     __syncthreads();  // chunk 0's header, block 0 and slab 0 are in LDS
-    int s = 0, buf = 0, si = 0, written = 0;  // si: ordinal of the slice being processed
+    CcSlice Z = first_slice<WIDE>(K);
+    int buf = 0;
     // TAB: chunk, stream position after the previous chunk, block finished last (-1: none)
     uint32_t tc = 0, tofs = 0;
     int blk = -1;
@@ -1091,9 +1140,9 @@ __device__ __forceinline__ void cccs_compute(const CcBlock& K, const CcLds& S, i
             // the block arrived during an earlier chunk) and starts loading the next block into the
             // other buffer, which the previous block no longer needs.
             const int* h = S.hdr + (tc & 1) * kTabHdr;
-            done = h[kTabHdr - 2];
-            sn = h[kTabHdr - 1];
-            cnt = min(max(__builtin_amdgcn_readfirstlane(h[wave]), 0), kRecCap);
+            done = __builtin_amdgcn_readfirstlane(h[kTabHdr - 2]);
+            sn = __builtin_amdgcn_readfirstlane(h[kTabHdr - 1]);
+            cnt = (int)min((uint32_t)__builtin_amdgcn_readfirstlane(h[wave]), (uint32_t)kRecCap);
             uint32_t o = tofs;
             if ((o & (kRecCap - 1)) + (uint32_t)cnt > (uint32_t)kRecCap)
                 o = (o + kRecCap - 1) & ~(uint32_t)(kRecCap - 1);
@@ -1121,21 +1170,22 @@ __device__ __forceinline__ void cccs_compute(const CcBlock& K, const CcLds& S, i
             tc++;
             tab_load_header(TR, tc, S.hdr + (tc & 1) * kTabHdr, wave);
         } else {
-            done = S.hdr[buf * kHdr + kMaxPhi];
-            sn = S.hdr[buf * kHdr + kMaxPhi + 1];
+            done = __builtin_amdgcn_readfirstlane(S.hdr[buf * kHdr + kMaxPhi]);
+            sn = __builtin_amdgcn_readfirstlane(S.hdr[buf * kHdr + kMaxPhi + 1]);
             cnt = __builtin_amdgcn_readfirstlane(S.hdr[buf * kHdr + wave]);
             rp = S.rec + (buf * n_phi + wave) * kRecStride;
         }
-        float pf0 = 0.0f, pf1 = 0.0f;
-        if (done && sn < K.L && K.prefetch) slab_regs(K, sn, pf0, pf1);
+        CcAhead ahead;
+        if (done && sn < K.L && loads_ahead<WIDE>(K)) slab_regs<WIDE>(K, sn, ahead);
         if (fresh) {
-            const float* slab = S.slab + (si & 1) * kSlab + vbase;
+            const float4* slab = reinterpret_cast<const float4*>(S.slab + (Z.si & 1) * kSlab) + lane;
+            const float4 ta = slab[0], tb = slab[kWave], ra = slab[2 * kWave], rb = slab[3 * kWave];
+            TA[0] = ta.x, TA[1] = ta.y, TA[2] = ta.z, TA[3] = ta.w;
+            TB[0] = tb.x, TB[1] = tb.y, TB[2] = tb.z, TB[3] = tb.w;
+            nRa[0] = ra.x, nRa[1] = ra.y, nRa[2] = ra.z, nRa[3] = ra.w;
+            nRb[0] = rb.x, nRb[1] = rb.y, nRb[2] = rb.z, nRb[3] = rb.w;
 #pragma unroll
             for (int r = 0; r < kSlots; r++) {
-                TA[r] = slab[16 * r];
-                TB[r] = slab[kNpix + 16 * r];
-                nRa[r] = slab[2 * kNpix + 16 * r];
-                nRb[r] = slab[3 * kNpix + 16 * r];
                 D[r] = 0.0f;
                 Cs[r] = 0.0f;
             }
@@ -1152,7 +1202,7 @@ __device__ __forceinline__ void cccs_compute(const CcBlock& K, const CcLds& S, i
                 // rotate the X state (and my rays' x offsets) to follow the midpoint voxel
                 if (w & kUnitX) {
                     if (w & 0x10u) {  // ddx = -1
-                        if (w & kZeroFillX) {  // with the previous step's reset of column 0
+                        if (apart(w) & kZeroFillX) {  // with the previous step's reset of column 0
 #pragma unroll
                             for (int r = 0; r < kSlots; r++) {
                                 XA[r] = row_from_right_zero(XA[r]);
@@ -1167,7 +1217,7 @@ __device__ __forceinline__ void cccs_compute(const CcBlock& K, const CcLds& S, i
                         }
                         fix = row_from_right(fix);
                     } else {  // ddx = +1
-                        if (w & kZeroFillX) {  // with the previous step's reset of column 15
+                        if (apart(w) & kZeroFillX) {  // with the previous step's reset of column 15
 #pragma unroll
                             for (int r = 0; r < kSlots; r++) {
                                 XA[r] = row_from_left_zero(XA[r]);
@@ -1230,6 +1280,9 @@ __device__ __forceinline__ void cccs_compute(const CcBlock& K, const CcLds& S, i
                 // X <- T (1 - e) + e X = T - e (T - X)
                 XA[r] = fmaf(-ea, TA[r] - XA[r], TA[r]);
                 XB[r] = fmaf(-eb, TB[r] - XB[r], TB[r]);
+                // the dose is summed here: moved behind the resets, it would keep the old X alive and the
+                // state would go back and forth between two register sets
+                asm volatile("" : "+v"(D[r]));
             }
             // rays that crossed the lateral BEV edge restart with X = 0 (DoseComp.cu:372-377)
             if (w & kResetBits) {
@@ -1288,23 +1341,21 @@ __device__ __forceinline__ void cccs_compute(const CcBlock& K, const CcLds& S, i
             q += 4;
         }
         if (done) {  // publish this azimuth's slice dose (and the last azimuth's cumulative length)
-            float* myD = S.sD + ((si & 1) * n_phi + wave) * kNpix;
-#pragma unroll
-            for (int r = 0; r < kSlots; r++) {
-                myD[vbase + 16 * r] = D[r];
-                if (CUMU) S.sC[(si & 1) * kNpix + vbase + 16 * r] = Cs[r];
-            }
+            reinterpret_cast<float4*>(S.sD + ((Z.si & 1) * n_phi + wave) * kNpix)[lane] =
+                make_float4(D[0], D[1], D[2], D[3]);
+            if (CUMU)
+                reinterpret_cast<float4*>(S.sC + (Z.si & 1) * kNpix)[lane] = make_float4(Cs[0], Cs[1], Cs[2], Cs[3]);
         }
-        if (!chunk_end(K, S, done, sn, pf0, pf1, s, si, written, TAB)) break;
+        if (!chunk_end<WIDE>(K, S, done, sn, ahead, Z, TAB)) break;
         fresh = done != 0;
         buf ^= 1;
     }
-    zero_tail(K, written);
+    zero_tail(K, Z.written);
 }
 
-// 72 VGPRs (7 wavefronts per SIMD) and 49.6 KiB of LDS fit three workgroups of 9 wavefronts on a CU
+// 72 VGPRs (7 wavefronts per SIMD) and 47.0 KiB of LDS fit three workgroups of 9 wavefronts on a CU
 // (the few values the compiler then spills live outside the step loop); 80 VGPRs fit two.
-template <bool EXACT_G>
+template <bool EXACT_G, bool WIDE>
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(7, 8))) void cccs_kernel(
     const BeamletDev* __restrict__ beams, int n, const ConeTable* __restrict__ cones, int n_fwd,
     const float* __restrict__ terma, const float* __restrict__ dens_bev, float* __restrict__ partial) {
@@ -1315,35 +1366,32 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(7, 8))) vo
     CcBlock K;
     K.L = B.L;
     if (K.L <= 0) return;
-    K.tid = threadIdx.x;
-    K.nthreads = blockDim.x;
-    K.n_phi = (blockDim.x >> 6) - 1;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    K.wave = wave;
+    K.n_waves = blockDim.x >> 6;
+    K.n_phi = K.n_waves - 1;
     K.Tg = terma + B.bev_off;
     K.Rg = dens_bev + B.bev_off;
     K.P = cone_partial(partial, B, n_fwd, t);
-    K.two = K.nthreads < 2 * kNpix;  // each thread prefetches two slab values
-    K.prefetch = K.nthreads >= kNpix;  // smaller workgroups reload each slab
     const CcLds S = carve_lds(lds4, K.n_phi);
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
     K.A_a = cones->A_a[t];
     K.B_b = cones->B_b[t];
     K.na = cones->na[t];
     K.nb = cones->nb[t];
-    // slab of slice 0 into buffer 0
-    for (int i = K.tid; i < 2 * kNpix; i += K.nthreads) store_slab(K, S, 0, i, i < kNpix ? K.Tg[i] : K.Rg[i - kNpix]);
+    load_slab(K, S, 0, 0);
     if (wave == K.n_phi)
-        cccs_march(B, cones, t, K, S);
+        cccs_march<WIDE>(B, cones, t, K, S);
     else if (wave == K.n_phi - 1)
-        cccs_compute<EXACT_G, true>(K, S, wave);
+        cccs_compute<EXACT_G, WIDE, true>(K, S, wave);
     else
-        cccs_compute<EXACT_G, false>(K, S, wave);
+        cccs_compute<EXACT_G, WIDE, false>(K, S, wave);
 }
 
 // cccs_kernel without the march wavefront: the workgroup's n_phi compute wavefronts read their
 // chunks from the march table of the beamlet's geometry (cccs_table_kernel) and finish the
 // records with the beamlet's lim_min and sad themselves.  Same arithmetic, same results.
-template <bool EXACT_G>
+template <bool EXACT_G, bool WIDE>
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(6, 8))) void cccs_tab_kernel(
     const BeamletDev* __restrict__ beams, int n, const ConeTable* __restrict__ cones, int n_fwd,
     const float* __restrict__ terma, const float* __restrict__ dens_bev, float* __restrict__ partial,
@@ -1356,16 +1404,14 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(6, 8))) vo
     CcBlock K;
     K.L = B.L;
     if (K.L <= 0) return;
-    K.tid = threadIdx.x;
-    K.nthreads = blockDim.x;
-    K.n_phi = blockDim.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    K.wave = wave;
+    K.n_waves = blockDim.x >> 6;
+    K.n_phi = K.n_waves;
     K.Tg = terma + B.bev_off;
     K.Rg = dens_bev + B.bev_off;
     K.P = cone_partial(partial, B, n_fwd, t);
-    K.two = K.nthreads < 2 * kNpix;
-    K.prefetch = K.nthreads >= kNpix;
     const CcLds S = carve_lds_tab(lds4, K.n_phi);
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
     K.A_a = cones->A_a[t];
     K.B_b = cones->B_b[t];
@@ -1382,11 +1428,11 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(6, 8))) vo
     TR.bsx = B.bs[0];
     TR.bsy = B.bs[1];
     TR.ls = B.ls;
-    for (int i = K.tid; i < 2 * kNpix; i += K.nthreads) store_slab(K, S, 0, i, i < kNpix ? K.Tg[i] : K.Rg[i - kNpix]);
+    load_slab(K, S, 0, 0);
     if (wave == K.n_phi - 1)
-        cccs_compute<EXACT_G, true, true>(K, S, wave, TR);
+        cccs_compute<EXACT_G, WIDE, true, true>(K, S, wave, TR);
     else
-        cccs_compute<EXACT_G, false, true>(K, S, wave, TR);
+        cccs_compute<EXACT_G, WIDE, false, true>(K, S, wave, TR);
 }
 
 // dose[b][s][p] = sum over forward cones of partial[b][t][s][p], cone slots in order.
@@ -1450,12 +1496,10 @@ hipError_t launch_cccs(const BeamletDev* beams, int n, int max_L, const ConeTabl
         // compute wavefronts only, reading their chunks from the tables
         const dim3 grid((unsigned)(n * n_fwd)), block(n_phi * kWave);
         const size_t shm = tab_lds_bytes(n_phi);
-        if (exact_g)
-            hipLaunchKernelGGL(cccs_tab_kernel<true>, grid, block, shm, stream, beams, n, cones_dev, n_fwd, terma,
-                               dens_bev, partial, tab->ent, tab->rec, tab->hdr);
-        else
-            hipLaunchKernelGGL(cccs_tab_kernel<false>, grid, block, shm, stream, beams, n, cones_dev, n_fwd, terma,
-                               dens_bev, partial, tab->ent, tab->rec, tab->hdr);
+        const auto kernel = n_phi >= 8 ? (exact_g ? cccs_tab_kernel<true, true> : cccs_tab_kernel<false, true>)
+                                       : (exact_g ? cccs_tab_kernel<true, false> : cccs_tab_kernel<false, false>);
+        hipLaunchKernelGGL(kernel, grid, block, shm, stream, beams, n, cones_dev, n_fwd, terma, dens_bev, partial,
+                           tab->ent, tab->rec, tab->hdr);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     } else if (n_fwd > 0) {
@@ -1464,12 +1508,9 @@ hipError_t launch_cccs(const BeamletDev* beams, int n, int max_L, const ConeTabl
         if (n_phi <= kMaxMarchPhi) {
             const dim3 block((n_phi + 1) * kWave);
             const size_t shm = march_lds_bytes(n_phi);
-            if (exact_g)
-                hipLaunchKernelGGL(cccs_kernel<true>, grid, block, shm, stream, beams, n, cones_dev, n_fwd, terma,
-                                   dens_bev, partial);
-            else
-                hipLaunchKernelGGL(cccs_kernel<false>, grid, block, shm, stream, beams, n, cones_dev, n_fwd, terma,
-                                   dens_bev, partial);
+            const auto kernel = n_phi + 1 >= 8 ? (exact_g ? cccs_kernel<true, true> : cccs_kernel<false, true>)
+                                               : (exact_g ? cccs_kernel<true, false> : cccs_kernel<false, false>);
+            hipLaunchKernelGGL(kernel, grid, block, shm, stream, beams, n, cones_dev, n_fwd, terma, dens_bev, partial);
         } else {
             // one azimuth per wavefront up to 16 azimuths (1024 threads), two beyond
             const int apw = n_phi <= kMaxPhiPerWave1 ? 1 : 2;

@@ -1,0 +1,48 @@
+"""CCCS workgroups of every size of the march and table kernels (needs an MI355X).
+
+A workgroup has one wavefront per azimuth, and one more in the march kernel.  With less than four
+wavefronts each slab is loaded when its slice starts, with four to seven a wavefront loads two groups
+of the next slab ahead, from eight on one: the azimuth counts on both sides of these lines, against
+the oracle at the tolerances of the other kernel shapes, and the table kernel against the march
+kernel bit for bit.
+"""
+import numpy as np
+import pytest
+
+import fastdose_amd as fd
+import oracle as orc
+from fastdose_amd import synth
+
+from gpu_util import beamlets_of, gpu_stages, log, same_matrix
+from test_gpu_parity import check_against_oracle
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def torch_cuda():
+    import torch
+
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    return torch
+
+
+@pytest.mark.parametrize("n_phi", [1, 3, 4, 6, 7, 9])
+@pytest.mark.parametrize("exact_g", [False, True])
+def test_workgroup_sizes(torch_cuda, n_phi, exact_g):
+    cfg = synth.small_config(seed=70 + n_phi, dim=(22, 26, 23), fluence_dim=2, angles=(40.0, -30.0, 15.0))
+    cfg.kernel = synth.synthetic_kernel(1070 + n_phi, n_phi=n_phi)
+    flag = fd.FD_OPT_EXACT_G if exact_g else 0
+    beams, flu = beamlets_of(cfg)
+    log(f"azimuths {n_phi} exact_g={exact_g}")
+    with fd.Context(cfg.volume, cfg.density, cfg.spectrum, cfg.kernel, options=flag) as ctx:
+        g = gpu_stages(ctx, beams, flu, cfg.extent)
+    check_against_oracle(cfg, beams, flu, g, range(len(beams)), flags=orc.EXACT_G if exact_g else 0)
+    flags = [np.ones(4, dtype=np.uint8)]
+    mats = []
+    for how in (fd.FD_OPT_NO_TABLES, fd.FD_OPT_TABLES):
+        with fd.Context(cfg.volume, cfg.density, cfg.spectrum, cfg.kernel, options=flag | how) as ctx:
+            mats.append(fd.dose_mat_construction(ctx, cfg.bundles, flags, cfg.extent, batched=True))
+    assert mats[0].info() == mats[1].info() and mats[0].info()[2] > 0
+    assert same_matrix(mats[0].matrix(0), mats[1].matrix(0))
