@@ -546,6 +546,7 @@ constexpr uint32_t kColReset = 1u << 18, kRowReset = 1u << 23, kGeneralReset = 1
 constexpr uint32_t kUnitX = 1u << 30, kUnitY = 1u << 31;
 constexpr uint32_t kShiftBits = 0x3FFu, kResetBits = kColReset | kRowReset | kGeneralReset;
 constexpr int kMaxMarchPhi = 10;  // azimuths of the march kernel (64 KiB of LDS); more: inline kernel
+constexpr unsigned kFewGroups = 2 * 256;  // workgroups up to which cccs_kernel's FEW instance is used
 constexpr int kMaxPhiPerWave1 = 16;  // self-marching kernel: one azimuth per wavefront up to 16, then two
 // A slab in LDS: A/a T, B/b T, -a log2(e) rho and -b log2(e) rho of the slice, 256 each, read by the
 // compute wavefronts when the slice starts.  Its arrays and the doses are stored in the order in
@@ -1091,7 +1092,7 @@ static_assert(2 * kRecCap == kWave, "a table block is one 16-byte load per lane"
 // X states are kept pre-scaled by A/a and B/b, and the dose and cumulative length are summed in
 // units of the geometric length s (p = s rho), multiplied by rho in the combine.  TAB: the chunks
 // come from a march table (cccs_tab_kernel), else from the march wavefront's LDS records.
-template <bool EXACT_G, bool WIDE, bool CUMU, bool TAB = false>
+template <bool EXACT_G, bool WIDE, bool CUMU, bool TAB, bool FEW>
 __device__ __forceinline__ void cccs_compute(const CcBlock& K, const CcLds& S, int wave,
                                              const TabRead& TR = TabRead{}) {
     const int lane = threadIdx.x & 63;
@@ -1330,15 +1331,31 @@ __device__ __forceinline__ void cccs_compute(const CcBlock& K, const CcLds& S, i
         const float4* q = rp;
         float4 ra = q[0], qa;
         float2 rb = reinterpret_cast<const float2*>(q)[2], qb;
-        for (int k = 0; k < cnt; k += 2) {
-            qa = q[2];
-            qb = reinterpret_cast<const float2*>(q + 2)[2];
-            step(ra, rb, k);
-            if (k + 1 >= cnt) break;
-            ra = q[4];
-            rb = reinterpret_cast<const float2*>(q + 4)[2];
-            step(qa, qb, k + 1);
-            q += 4;
+        auto steps_until = [&](int& k, int stop) {
+            for (; k < stop; k += 2) {
+                qa = q[2];
+                qb = reinterpret_cast<const float2*>(q + 2)[2];
+                step(ra, rb, k);
+                if (k + 1 >= cnt) break;
+                ra = q[4];
+                rb = reinterpret_cast<const float2*>(q + 4)[2];
+                step(qa, qb, k + 1);
+                q += 4;
+            }
+        };
+        int k = 0;
+        if (FEW) {
+            // Wavefronts w and w + 4 share a SIMD, whose arbiter prefers the older one: 634 against 885
+            // cycles per step, and the slice waits for the younger.  With few wavefronts per SIMD the
+            // younger ones go first in the first half of their steps.
+            for (int stop = wave >= 4 ? (cnt >> 1) & ~1 : cnt;; stop = cnt) {
+                if (stop < cnt) __builtin_amdgcn_s_setprio(1);
+                steps_until(k, stop);
+                if (stop == cnt) break;
+                __builtin_amdgcn_s_setprio(0);
+            }
+        } else {
+            steps_until(k, cnt);
         }
         if (done) {  // publish this azimuth's slice dose (and the last azimuth's cumulative length)
             reinterpret_cast<float4*>(S.sD + ((Z.si & 1) * n_phi + wave) * kNpix)[lane] =
@@ -1355,8 +1372,11 @@ __device__ __forceinline__ void cccs_compute(const CcBlock& K, const CcLds& S, i
 
 // 72 VGPRs (7 wavefronts per SIMD) and 47.0 KiB of LDS fit three workgroups of 9 wavefronts on a CU
 // (the few values the compiler then spills live outside the step loop); 80 VGPRs fit two.
-template <bool EXACT_G, bool WIDE>
-__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(7, 8))) void cccs_kernel(
+// FEW: at most two workgroups per CU, where a slice takes as long as its slowest wavefront's serial
+// chain: up to 96 VGPRs, and the wavefronts of a SIMD take turns (cccs_compute).  16 beamlets of a slab
+// beam (64 workgroups) 476 -> 459 us, 121 (484) 1157 -> 1115; with 196 (784) the turns cost 2 %.
+template <bool EXACT_G, bool WIDE, bool FEW>
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(FEW ? 5 : 7, 8))) void cccs_kernel(
     const BeamletDev* __restrict__ beams, int n, const ConeTable* __restrict__ cones, int n_fwd,
     const float* __restrict__ terma, const float* __restrict__ dens_bev, float* __restrict__ partial) {
     extern __shared__ float4 lds4[];
@@ -1383,9 +1403,9 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(7, 8))) vo
     if (wave == K.n_phi)
         cccs_march<WIDE>(B, cones, t, K, S);
     else if (wave == K.n_phi - 1)
-        cccs_compute<EXACT_G, WIDE, true>(K, S, wave);
+        cccs_compute<EXACT_G, WIDE, true, false, FEW>(K, S, wave);
     else
-        cccs_compute<EXACT_G, WIDE, false>(K, S, wave);
+        cccs_compute<EXACT_G, WIDE, false, false, FEW>(K, S, wave);
 }
 
 // cccs_kernel without the march wavefront: the workgroup's n_phi compute wavefronts read their
@@ -1430,9 +1450,9 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(6, 8))) vo
     TR.ls = B.ls;
     load_slab(K, S, 0, 0);
     if (wave == K.n_phi - 1)
-        cccs_compute<EXACT_G, WIDE, true, true>(K, S, wave, TR);
+        cccs_compute<EXACT_G, WIDE, true, true, false>(K, S, wave, TR);
     else
-        cccs_compute<EXACT_G, WIDE, false, true>(K, S, wave, TR);
+        cccs_compute<EXACT_G, WIDE, false, true, false>(K, S, wave, TR);
 }
 
 // dose[b][s][p] = sum over forward cones of partial[b][t][s][p], cone slots in order.
@@ -1508,8 +1528,11 @@ hipError_t launch_cccs(const BeamletDev* beams, int n, int max_L, const ConeTabl
         if (n_phi <= kMaxMarchPhi) {
             const dim3 block((n_phi + 1) * kWave);
             const size_t shm = march_lds_bytes(n_phi);
-            const auto kernel = n_phi + 1 >= 8 ? (exact_g ? cccs_kernel<true, true> : cccs_kernel<false, true>)
-                                               : (exact_g ? cccs_kernel<true, false> : cccs_kernel<false, false>);
+            const bool few = grid.x <= kFewGroups;
+            const auto kernel =
+                n_phi + 1 < 8 ? (exact_g ? cccs_kernel<true, false, false> : cccs_kernel<false, false, false>)
+                : few         ? (exact_g ? cccs_kernel<true, true, true> : cccs_kernel<false, true, true>)
+                              : (exact_g ? cccs_kernel<true, true, false> : cccs_kernel<false, true, false>);
             hipLaunchKernelGGL(kernel, grid, block, shm, stream, beams, n, cones_dev, n_fwd, terma, dens_bev, partial);
         } else {
             // one azimuth per wavefront up to 16 azimuths (1024 threads), two beyond

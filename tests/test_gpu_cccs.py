@@ -46,3 +46,23 @@ def test_workgroup_sizes(torch_cuda, n_phi, exact_g):
             mats.append(fd.dose_mat_construction(ctx, cfg.bundles, flags, cfg.extent, batched=True))
     assert mats[0].info() == mats[1].info() and mats[0].info()[2] > 0
     assert same_matrix(mats[0].matrix(0), mats[1].matrix(0))
+
+
+def test_few_and_many_workgroups(torch_cuda):
+    """144 beamlets (four forward cones: 576 workgroups) in one call and in calls of 128 and 16: the
+    instances for few and for many workgroups, the first at its largest."""
+    cfg = synth.small_config(seed=91, dim=(30, 26, 28), fluence_dim=12, angles=(20.0, 15.0, 0.0))
+    beams, flu = beamlets_of(cfg)
+    assert len(beams) == 144
+    for options in (0, fd.FD_OPT_EXACT_G):
+        log(f"few and many workgroups, options {options}")
+        with fd.Context(cfg.volume, cfg.density, cfg.spectrum, cfg.kernel, options=options) as ctx:
+            dose = gpu_stages(ctx, beams, flu, cfg.extent)["dose"]
+            parts = [gpu_stages(ctx, fd.beam_array(beams[a:b]), flu[a:b], cfg.extent)["dose"]
+                     for a, b in ((0, 128), (128, 144))]
+        k = 0
+        for part in parts:
+            for d in part:
+                L = beams[k].long_dim
+                assert np.array_equal(d[:L], dose[k, :L]) and d[:L].max() > 0
+                k += 1
