@@ -13,6 +13,13 @@
 // 32-byte read per sample instead of eight gathers, no bounds tests, and rays of any direction
 // share cache lines.
 //
+// It is bound by vector instructions on small batches (1.0 issued per CU and cycle at 256 beamlets of
+// 175 slices) and by the record reads on large ones (the data path of vector memory 99 % busy in a
+// 20-beam plan: a read is issued for nearly every sample, since some lane of the wavefront changes its
+// base voxel).  So a sample has few instructions: base voxel and fraction are one conversion and one
+// v_fract per axis, the record offset is two 24-bit multiply-adds and three bit selects.  45.4 -> 37.2 M
+// wavefront instructions and 80 -> 69 us for 256 beamlets, 2.16 -> 2.05 ms in the plan.
+//
 // The radiological path is a prefix sum along each ray, which one lane per ray would walk alone
 // (256 rays per beamlet: one wavefront per SIMD on small batches).  Each ray is cut into 1, 2, 4,
 // 8 or 16 segments of slices (a launch parameter; with 8 or 16, a beamlet's rays take two
@@ -41,8 +48,27 @@ constexpr int kTermaMaxSeg = 16;    // most ray segments (16: four workgroups of
 // interpolation step needs, rounded as it would round them.  Records in 4 x 4 x 4 bricks: record
 // ((z/4 nby + y/4) nbx + x/4) 64 + 16 (z%4) + 4 (y%4) + x%4, nb* = ceil((dim + 1) / 4).  A sample
 // reads one 32-byte record.
-__device__ __forceinline__ uint64_t corner_record(uint32_t x, uint32_t y, uint32_t z, uint32_t nbx, uint32_t nby) {
-    return ((((uint64_t)(z >> 2) * nby + (y >> 2)) * nbx + (x >> 2)) << 6) + ((z & 3) << 4) + ((y & 3) << 2) + (x & 3);
+// Index: uint64_t, or uint32_t for records that span less than 4 GiB: then there are fewer than 2^21
+// bricks and 24-bit products do (the line is where the offset stops fitting; 80 us with 64-bit offsets
+// on all volumes, 71 with 32-bit ones).
+__device__ __forceinline__ uint32_t mad24(uint32_t a, uint32_t b, uint32_t c) {
+    uint32_t r;
+    asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(b), "v"(c));
+    return r;
+}
+// Bits of a where mask has a one, of b elsewhere.
+__device__ __forceinline__ uint32_t select_bits(uint32_t mask, uint32_t a, uint32_t b) {
+    return (mask & a) | (~mask & b);
+}
+template <typename Index>
+__device__ __forceinline__ Index corner_record(uint32_t x, uint32_t y, uint32_t z, uint32_t nbx, uint32_t nby) {
+    if constexpr (sizeof(Index) == 4) {
+        const uint32_t column = mad24(mad24(z >> 2, nby, y >> 2), 4 * nbx, x);  // brick 4 + x % 4
+        return select_bits(3, column, select_bits(12, y << 2, select_bits(48, z << 4, column << 4)));
+    } else {
+        const Index brick = ((Index)(z >> 2) * nby + (y >> 2)) * nbx + (x >> 2);
+        return (((((brick << 2) + (z & 3)) << 2) + (y & 3)) << 2) + (x & 3);
+    }
 }
 
 __global__ __launch_bounds__(256) void expand_density_kernel(const float* __restrict__ density, int X, int Y, int Z,
@@ -59,29 +85,40 @@ __global__ __launch_bounds__(256) void expand_density_kernel(const float* __rest
         const bool in = ox >= 0 && ox < X && oy >= 0 && oy < Y && oz >= 0 && oz < Z;
         v[c] = in ? density[((size_t)oz * Y + oy) * X + ox] : 0.0f;
     }
-    const uint64_t r = corner_record(x, y, z, nbx, nby);
+    const uint64_t r = corner_record<uint64_t>(x, y, z, nbx, nby);
     out[2 * r] = make_float4(v[0], v[1] - v[0], v[2], v[3] - v[2]);
     out[2 * r + 1] = make_float4(v[4], v[5] - v[4], v[6], v[7] - v[6]);
+}
+
+// floor(v + 1/2), exactly (checked for every float below 2^22), for a voxel-unit position v: the base
+// voxel's record coordinate floor(v - 1/2) + 1, as an integer that wraps to a large unsigned number
+// below zero.
+__device__ __forceinline__ uint32_t base_of(float v) {
+    uint32_t r;
+    asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(r) : "v"(v));
+    return r;
 }
 
 // Trilinear density at voxel-unit position (cx, cy, cz) (texel centres at i + 0.5, zero outside
 // the volume) from the corner records (nbx, nby: bricks along x and y).  The last record read stays
 // in registers: consecutive samples of a ray are a fraction of a voxel apart (four per slice), so
 // most fall in the base voxel of the one before and need no load; a lane loads only when its base
-// voxel changes.  (r, lo, hi): the record held, r = ~0 for none.
-__device__ __forceinline__ float density_at(const float4* __restrict__ rec, int X, int Y, int Z, uint32_t nbx,
-                                            uint32_t nby, float cx, float cy, float cz, uint64_t& r, float4& lo,
-                                            float4& hi) {
+// voxel changes.  (r, lo, hi): the record held, r = ~0 for none.  nx: X + 1, or 0 for a ray whose
+// positions are not numbers (it lies outside everywhere).
+template <typename Index>
+__device__ __forceinline__ float density_at(const float4* __restrict__ rec, uint32_t nx, uint32_t ny, uint32_t nz,
+                                            uint32_t nbx, uint32_t nby, float cx, float cy, float cz, Index& r,
+                                            float4& lo, float4& hi) {
     const float xb = cx - 0.5f, yb = cy - 0.5f, zb = cz - 0.5f;
-    const float fx = floorf(xb), fy = floorf(yb), fz = floorf(zb);
+    const uint32_t x = base_of(cx), y = base_of(cy), z = base_of(cz);
     // outside: every corner is in the zero border or beyond (and the record index stays in range)
-    if (!(fx > -2.0f && fx < (float)X && fy > -2.0f && fy < (float)Y && fz > -2.0f && fz < (float)Z)) return 0.0f;
-    const float ax = xb - fx, ay = yb - fy, az = zb - fz;
-    const uint64_t rn =
-        corner_record((uint32_t)((int)fx + 1), (uint32_t)((int)fy + 1), (uint32_t)((int)fz + 1), nbx, nby);
+    if (!(x < nx && y < ny && z < nz)) return 0.0f;
+    const float ax = __builtin_amdgcn_fractf(xb), ay = __builtin_amdgcn_fractf(yb), az = __builtin_amdgcn_fractf(zb);
+    const Index rn = corner_record<Index>(x, y, z, nbx, nby);
     if (rn != r) {
-        lo = rec[2 * rn];
-        hi = rec[2 * rn + 1];
+        const char* at = reinterpret_cast<const char*>(rec) + (Index)(rn * 32);
+        lo = reinterpret_cast<const float4*>(at)[0];
+        hi = reinterpret_cast<const float4*>(at)[1];
         r = rn;
     }
     const float c00 = fmaf(ax, lo.y, lo.x);
@@ -97,6 +134,7 @@ __device__ __forceinline__ float density_at(const float4* __restrict__ rec, int 
 // accumulate the radiological path in FP64 (0: every beamlet; infinity: none).
 // Workgroup (beamlet blockIdx.x, ray block blockIdx.y): `rays` consecutive BEV pixels (a multiple
 // of 64) times blockDim.x / rays segments.
+template <typename Index>
 __global__ __launch_bounds__(kTermaThreads) __attribute__((amdgpu_waves_per_eu(8, 8))) void terma_kernel(
     const BeamletDev* __restrict__ beams, const float* __restrict__ fluence, const float* __restrict__ density_pad,
     int X, int Y, int Z, float vsx, float vsy, float vsz, SpectrumDev spec, float rpl64_len,
@@ -130,18 +168,24 @@ __global__ __launch_bounds__(kTermaThreads) __attribute__((amdgpu_waves_per_eu(8
 
     const uint32_t nbx = ((uint32_t)X + 4) / 4, nby = ((uint32_t)Y + 4) / 4;
     const float4* __restrict__ rec = reinterpret_cast<const float4*>(density_pad);
-    uint64_t rc = ~uint64_t(0);
+    // (a conversion to an integer would make a voxel of a position that is not a number)
+    const bool numbers = 0.0f * ax + 0.0f * ay + 0.0f * az + 0.0f * sx + 0.0f * sy + 0.0f * sz + 0.0f * t0 +
+                             0.0f * dt == 0.0f;
+    const uint32_t nx = numbers ? (uint32_t)X + 1 : 0u, ny = (uint32_t)Y + 1, nz = (uint32_t)Z + 1;
+    Index rc = ~(Index)0;
     float4 rlo = make_float4(0.0f, 0.0f, 0.0f, 0.0f), rhi = rlo;
     auto rho_at = [&](int k) {
         const float t = fmaf((float)k, dt, t0);
-        return density_at(rec, X, Y, Z, nbx, nby, fmaf(ax, t, sx), fmaf(ay, t, sy), fmaf(az, t, sz), rc, rlo, rhi);
+        return density_at<Index>(rec, nx, ny, nz, nbx, nby, fmaf(ax, t, sx), fmaf(ay, t, sy), fmaf(az, t, sz), rc, rlo,
+                                 rhi);
     };
     // the FP64 path's second walk keeps no record in registers (fewer live registers there)
     auto rho_fresh = [&](int k) {
         const float t = fmaf((float)k, dt, t0);
-        uint64_t r = ~uint64_t(0);
+        Index r = ~(Index)0;
         float4 lo, hi;
-        return density_at(rec, X, Y, Z, nbx, nby, fmaf(ax, t, sx), fmaf(ay, t, sy), fmaf(az, t, sz), r, lo, hi);
+        return density_at<Index>(rec, nx, ny, nz, nbx, nby, fmaf(ax, t, sx), fmaf(ay, t, sy), fmaf(az, t, sz), r, lo,
+                                 hi);
     };
 
     float* __restrict__ T = terma + B.bev_off + p;
@@ -242,7 +286,9 @@ hipError_t launch_terma(const BeamletDev* beams, int n, const float* fluence, co
     const int rays = std::min(kNpix, kTermaThreads / segments);
     dim3 grid(n, kNpix / rays), block(segments * rays);
     const int X = vol.dim[0], Y = vol.dim[1], Z = vol.dim[2];
-    hipLaunchKernelGGL(terma_kernel, grid, block, 0, stream, beams, fluence, density_pad, X, Y, Z, vol.voxel_size[0],
+    const auto kernel = density_records_floats(vol) * sizeof(float) < (1ull << 32) ? terma_kernel<uint32_t>
+                                                                                   : terma_kernel<uint64_t>;
+    hipLaunchKernelGGL(kernel, grid, block, 0, stream, beams, fluence, density_pad, X, Y, Z, vol.voxel_size[0],
                        vol.voxel_size[1], vol.voxel_size[2], spec, rpl64_len, terma, dens_bev,
                        reinterpret_cast<float4*>(scratch), rays);
     return hipGetLastError();
