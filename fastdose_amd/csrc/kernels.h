@@ -133,15 +133,17 @@ hipError_t launch_pack_rows(uint64_t R, const uint64_t* rowptr, const float* val
 // = row maxima; *unsorted (zeroed by the caller) = 1 when a row's columns do not ascend below C (the
 // table then must not be used).  launch_tile_totals: total[t] (zeroed by the caller) = entries of tile
 // t.  launch_place_tiles: colptr (C + 1), crow and cval from the table and tile_base, the exclusive
-// scan of total.  C > 0, R x 2048 and every row's length below 2^32.
+// scan of total; order: csc_tile_groups(C) words of scratch.  C > 0, R <= 2^20 and every row's length
+// below 2^32.
 uint64_t csc_tiles(uint64_t C);
+uint64_t csc_tile_groups(uint64_t C);
 hipError_t launch_row_tiles(uint64_t R, const uint64_t* rowptr, const uint64_t* columns, const float* values,
                             uint64_t C, uint32_t* tiles, float* scale, uint32_t* unsorted, hipStream_t stream);
 hipError_t launch_tile_totals(uint64_t R, uint64_t C, const uint32_t* tiles, uint32_t* total, hipStream_t stream);
 hipError_t launch_place_tiles(int vtype, uint64_t R, uint64_t C, const uint32_t* tiles, const uint64_t* rowptr,
                               const uint64_t* columns, const float* values, const float* scale,
-                              const uint64_t* tile_base, uint64_t* colptr, uint32_t* crow, void* cval,
-                              hipStream_t stream);
+                              const uint64_t* tile_base, uint32_t* order, uint64_t* colptr, uint32_t* crow,
+                              void* cval, hipStream_t stream);
 hipError_t launch_col_count(uint64_t nnz, const uint64_t* columns, uint32_t* count, hipStream_t stream);
 hipError_t launch_col_scatter(uint64_t R, const uint64_t* rowptr, const uint64_t* columns, const void* vals,
                               int vbytes, const uint64_t* colptr, uint32_t* cursor, uint32_t* crow, void* cval,

@@ -52,20 +52,22 @@ __global__ void global_rows_kernel(int n_mat, const uint64_t* __restrict__ row_f
 //
 // The columns are cut into tiles of kTileCols.  A row's entries of one tile are contiguous, so one
 // pass over the rows (row_tiles_kernel, HBM-bound on the 8-byte columns) writes where every tile
-// starts in every row, and one workgroup per tile then places the tile's entries: it counts them per
-// column in LDS, scans the counts into the column pointers, and takes the rows 64 at a time in
-// order.  Within such a block each entry sets the bit of its row in its column's 64-bit LDS mask;
-// after a barrier the entry's place is its column's running offset plus the mask's bits below its
-// row.  Every column comes out sorted by row without a sort, and without global atomics.  Before, an
-// atomic scatter and one insertion sort per column took 16.9 ms for 52 M entries (20 beams, 2 726
+// starts in every row, and one workgroup per tile then places the tile's entries: it lists the rows
+// that reach the tile (list_rows), counts the entries per column in LDS, scans the counts into the
+// column pointers, and takes the listed rows in order, up to 64 rows and 64 units of 64 entries at a
+// time (row_group).  Within such a group each entry sets the bit of its row in its column's 64-bit LDS
+// mask; after a barrier the entry's place is its column's running offset plus the mask's bits below
+// its row.  Every column comes out sorted by row without a sort, and without global atomics.  Before,
+// an atomic scatter and one insertion sort per column took 16.9 ms for 52 M entries (20 beams, 2 726
 // rows, 200 x 200 x 160 voxels; 14.2 of them the sort: the voxels of the target hold hundreds of
-// entries each).
+// entries each).  Placing takes 1.06 ms of the 1.3 now; it took 1.55 with groups of 64 consecutive rows
+// of the matrix, of which about 15 reach a tile (few loads in flight per barrier), 1.22 with the tiles in
+// volume order.  What is left waits for scattered loads and stores (1.4 GB of HBM traffic, 1.3 TB/s).
 // kTileCols: a beamlet's footprint is about ten voxels wide, so 2048 columns (ten x-rows of a
-// 200-voxel plane) hold about one wavefront of a row's entries, and the tile's LDS (24 KiB) lets
+// 200-voxel plane) hold about one wavefront of a row's entries, and the tile's LDS (39.5 KiB) lets
 // four workgroups of eight wavefronts share a CU.
 constexpr int kTileCols = 2048;
 constexpr int kPlaceThreads = 512;
-constexpr int kBlockRows = 64;  // rows per block: one bit each in a column's mask
 
 // tiles[r * (n_tiles + 1) + t] = entries of row r before tile t (t = n_tiles: all of them), and for
 // 16-bit values scale[r] = the row maximum.  Sets *unsorted when a row's columns do not ascend
@@ -143,79 +145,184 @@ __device__ __forceinline__ uint64_t lane_u64(uint64_t v, int src) {
     return ((uint64_t)lane_u32((uint32_t)(v >> 32), src) << 32) | lane_u32((uint32_t)v, src);
 }
 
-// Lane l: start and length of row (r0 + l)'s entries of the tile
-__device__ __forceinline__ void block_segments(uint64_t r0, uint64_t R, uint32_t n_tiles, uint32_t tile,
-                                               const uint32_t* __restrict__ tiles, const uint64_t* __restrict__ rowptr,
-                                               uint64_t& start, uint32_t& len) {
-    const uint64_t r = r0 + (threadIdx.x & 63);
-    start = 0;
-    len = 0;
-    if (r < R) {
-        const uint32_t* row = tiles + r * (uint64_t)(n_tiles + 1) + tile;
-        const uint32_t lo = row[0];
-        len = row[1] - lo;
-        start = rowptr[r] + lo;
+// The rows that reach a tile, in order: appended to a list in LDS, kPlaceThreads rows of the matrix at
+// a time, until it could overflow or the rows end.  Called by the whole workgroup.
+constexpr int kListRows = 1984;  // four workgroups to a CU with the masks and offsets
+constexpr int kRowBits = 20;  // of a list word; the entries of a row in a tile (kTileCols at most) above
+static_assert(kTileCols < (1 << (32 - kRowBits)), "a list word holds a row's entry count");
+struct TileRows {
+    uint32_t* before;  // [kListRows] entries of the row before the tile
+    uint32_t* word;    // [kListRows] row | entries << kRowBits
+    uint32_t* wave;    // [kPlaceThreads / 64 + 1]
+};
+__device__ __forceinline__ uint32_t list_rows(const TileRows& T, uint64_t& r0, uint64_t R, uint32_t n_tiles,
+                                              uint32_t tile, const uint32_t* __restrict__ tiles) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint32_t n = 0;
+    while (r0 < R && n + kPlaceThreads <= kListRows) {
+        const uint64_t r = r0 + threadIdx.x;
+        uint32_t lo = 0, len = 0;
+        if (r < R) {
+            const uint32_t* row = tiles + r * (uint64_t)(n_tiles + 1) + tile;
+            lo = row[0];
+            len = row[1] - lo;
+        }
+        const uint64_t some = __ballot(len != 0);
+        if (lane == 0) T.wave[wave] = (uint32_t)__popcll(some);
+        __syncthreads();
+        uint32_t at = n + (uint32_t)__popcll(some & ((1ull << lane) - 1ull));
+        for (int w = 0; w < kPlaceThreads / 64; w++) {
+            const uint32_t c = T.wave[w];
+            at += w < wave ? c : 0u;
+            n += c;
+        }
+        if (len != 0) {
+            T.before[at] = lo;
+            T.word[at] = (uint32_t)r | (len << kRowBits);
+        }
+        r0 += kPlaceThreads;
+        __syncthreads();
     }
+    return n;
 }
 
-// Tile of workgroup id.  Neighbouring tiles share lines of the tile table, so groups of 16 of them go
-// to one XCD (the dispatcher deals workgroups to the 8 XCDs round-robin); the groups are dealt in
-// turn, because a whole contiguous range per XCD would give the full tiles, in the middle of the
-// volume, to two of the eight.
-__device__ __forceinline__ uint32_t tile_of_workgroup(uint32_t id, uint32_t n_tiles) {
-    constexpr uint32_t kXcd = 8, kGroup = 16;
-    if (id >= n_tiles / (kXcd * kGroup) * (kXcd * kGroup)) return id;
-    const uint32_t x = id % kXcd, k = id / kXcd;
-    return ((k / kGroup) * kXcd + x) * kGroup + k % kGroup;
+// Rows g .. g + taken - 1 of the list, cut into units of up to 64 entries: lane l holds row g + l's first
+// entry, list word and the number of units before it.
+struct RowGroup {
+    uint64_t start;
+    uint32_t word, first;
+    int taken;       // rows
+    uint32_t units;
+    // unit u's row (its place in the group), first entry and number of entries, all wavefront-uniform
+    __device__ __forceinline__ int unit(uint32_t u, uint64_t& e0, uint32_t& n) const {
+        const int l = __popcll(__ballot((int)(threadIdx.x & 63) < taken && first <= u)) - 1;
+        const uint32_t skip = 64u * (u - lane_u32(first, l));
+        e0 = lane_u64(start, l) + skip;
+        n = min((lane_u32(word, l) >> kRowBits) - skip, 64u);
+        return l;
+    }
+};
+// most: units the group may have (a single row has at most kTileCols / 64); at most 64 rows
+__device__ __forceinline__ RowGroup row_group(const TileRows& T, const uint64_t* __restrict__ rowptr, uint32_t g,
+                                              uint32_t n_list, uint32_t most) {
+    const int lane = threadIdx.x & 63;
+    const uint32_t i = g + lane;
+    RowGroup G;
+    G.word = i < n_list ? T.word[i] : 0u;
+    G.start = i < n_list ? rowptr[G.word & ((1u << kRowBits) - 1u)] + T.before[i] : 0u;
+    const uint32_t nu = ((G.word >> kRowBits) + 63) >> 6;
+    uint32_t x = nu;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = __shfl_up(x, o, 64);
+        if (lane >= o) x += y;
+    }
+    G.first = x - nu;
+    G.taken = __popcll(__ballot(nu != 0 && x <= most));
+    G.units = lane_u32(x, G.taken - 1);
+    return G;
+}
+
+// Order in which the tiles are placed.  Neighbouring tiles share lines of the tile table, so groups of
+// kTileGroup of them go to one XCD (the dispatcher deals workgroups to the 8 XCDs round-robin); the
+// fullest groups first, since the tiles of the target, in the middle of the volume, hold many times
+// the entries of the others and would finish last (CUs busy for 60 % of the kernel in volume order).
+// order[i] = the i-th group, by falling totals in classes of a quarter octave; one workgroup.
+constexpr uint32_t kXcd = 8, kTileGroup = 16;
+__device__ __forceinline__ uint32_t size_class(uint64_t n) {  // 0: fullest
+    if (n < 4) return 255u - (uint32_t)n;
+    const uint32_t e = 63u - (uint32_t)__builtin_clzll(n);
+    return 255u - (4u * (e - 1u) + (uint32_t)((n >> (e - 2)) & 3u));
+}
+__global__ __launch_bounds__(1024) void tile_order_kernel(uint32_t n_tiles, const uint64_t* __restrict__ tile_base,
+                                                          uint32_t* __restrict__ order) {
+    __shared__ uint32_t s_at[256];
+    const uint32_t n_groups = (n_tiles + kTileGroup - 1) / kTileGroup;
+    auto cls = [&](uint32_t g) {
+        return size_class(tile_base[min((g + 1) * kTileGroup, n_tiles)] - tile_base[g * kTileGroup]);
+    };
+    if (threadIdx.x < 256) s_at[threadIdx.x] = 0;
+    __syncthreads();
+    for (uint32_t g = threadIdx.x; g < n_groups; g += blockDim.x) atomicAdd(&s_at[cls(g)], 1u);
+    __syncthreads();
+    if (threadIdx.x < 64) {  // exclusive scan, four classes per lane
+        uint32_t c[4], sum = 0;
+        for (int i = 0; i < 4; i++) {
+            c[i] = s_at[4 * threadIdx.x + i];
+            sum += c[i];
+        }
+        uint32_t x = sum;
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = __shfl_up(x, o, 64);
+            if ((int)threadIdx.x >= o) x += y;
+        }
+        uint32_t run = x - sum;
+        for (int i = 0; i < 4; i++) {
+            s_at[4 * threadIdx.x + i] = run;
+            run += c[i];
+        }
+    }
+    __syncthreads();
+    for (uint32_t g = threadIdx.x; g < n_groups; g += blockDim.x) order[atomicAdd(&s_at[cls(g)], 1u)] = g;
 }
 
 template <int VT>
 __global__ __launch_bounds__(kPlaceThreads) void place_tile_kernel(
     uint64_t R, uint64_t C, uint32_t n_tiles, const uint32_t* __restrict__ tiles, const uint64_t* __restrict__ rowptr,
     const uint64_t* __restrict__ columns, const float* __restrict__ values, const float* __restrict__ scale,
-    const uint64_t* __restrict__ tile_base, uint64_t* __restrict__ colptr, uint32_t* __restrict__ crow,
-    void* __restrict__ cval_out) {
+    const uint64_t* __restrict__ tile_base, const uint32_t* __restrict__ order, uint64_t* __restrict__ colptr,
+    uint32_t* __restrict__ crow, void* __restrict__ cval_out) {
     typedef typename StoredValue<VT>::type V;
     __shared__ uint32_t s_next[kTileCols];     // counts, then where each column's next entry goes
     __shared__ uint32_t s_mask[2][kTileCols];  // rows of the block that hold the column (low, high half)
     __shared__ uint32_t s_wave[kPlaceThreads / 64 + 1];
-    constexpr int kWaves = kPlaceThreads / 64, kPerWave = kBlockRows / kWaves, kCols = kTileCols / kPlaceThreads;
-    const uint32_t tile = tile_of_workgroup(blockIdx.x, n_tiles);
+    __shared__ uint32_t s_before[kListRows];
+    __shared__ uint32_t s_word[kListRows];
+    constexpr int kWaves = kPlaceThreads / 64, kCols = kTileCols / kPlaceThreads;
+    constexpr uint32_t kUnits = 64;  // a group's units: eight to a wavefront, all in flight
+    static_assert(kUnits >= kTileCols / 64 && kUnits == 8 * kWaves, "any row fits a group");
+    const uint32_t turn = blockIdx.x / kXcd;  // workgroup blockIdx.x runs on XCD blockIdx.x % kXcd
+    const uint32_t slot = turn / kTileGroup * kXcd + blockIdx.x % kXcd;
+    if (slot >= (n_tiles + kTileGroup - 1) / kTileGroup) return;
+    const uint32_t tile = order[slot] * kTileGroup + turn % kTileGroup;
+    if (tile >= n_tiles) return;
     const uint64_t c0 = (uint64_t)tile * kTileCols;
     const uint64_t base = tile_base[tile];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const TileRows T{s_before, s_word, s_wave};
     V* __restrict__ cval = (V*)cval_out;
     for (int i = tid; i < kTileCols; i += kPlaceThreads) {
         s_next[i] = 0u;
         s_mask[0][i] = 0u;
         s_mask[1][i] = 0u;
     }
-    __syncthreads();
-    // entries per column: each wavefront takes every kWaves-th block of rows
-    for (uint64_t r0 = (uint64_t)wave * kBlockRows; r0 < R; r0 += (uint64_t)kWaves * kBlockRows) {
-        uint64_t start;
-        uint32_t len;
-        block_segments(r0, R, n_tiles, tile, tiles, rowptr, start, len);
-        constexpr int Q = 8;  // rows in flight
-        for (uint64_t todo = __ballot(len != 0); todo;) {
-            uint32_t n[Q], col[Q];
-            uint64_t e0[Q];
+    // entries per column
+    uint64_t r_next = 0;
+    uint32_t n_list = 0;
+    bool whole = true;  // the list holds every row that reaches the tile
+    do {
+        n_list = list_rows(T, r_next, R, n_tiles, tile, tiles);
+        whole = whole && r_next >= R;
+        for (uint32_t g = 0; g < n_list;) {
+            const RowGroup G = row_group(T, rowptr, g, n_list, ~0u);
+            for (uint32_t u0 = wave; u0 < G.units; u0 += kUnits) {
+                uint32_t col[8];
 #pragma unroll
-            for (int q = 0; q < Q; q++) {
-                const int l = todo ? __ffsll((unsigned long long)todo) - 1 : 0;
-                n[q] = todo ? lane_u32(len, l) : 0u;
-                e0[q] = lane_u64(start, l);
-                todo &= todo - 1;  // 0 stays 0
-                col[q] = (uint32_t)lane < n[q] ? (uint32_t)(columns[e0[q] + lane] - c0) : ~0u;
-            }
+                for (int q = 0; q < 8; q++) {
+                    const uint32_t u = u0 + kWaves * q;
+                    uint64_t e0 = 0;
+                    uint32_t n = 0;
+                    if (u < G.units) G.unit(u, e0, n);
+                    col[q] = (uint32_t)lane < n ? (uint32_t)(columns[e0 + lane] - c0) : ~0u;
+                }
 #pragma unroll
-            for (int q = 0; q < Q; q++) {
-                if (col[q] != ~0u) atomicAdd(&s_next[col[q]], 1u);
-                for (uint32_t i = 64 + lane; i < n[q]; i += 64) atomicAdd(&s_next[columns[e0[q] + i] - c0], 1u);
+                for (int q = 0; q < 8; q++)
+                    if (col[q] != ~0u) atomicAdd(&s_next[col[q]], 1u);
             }
+            g += (uint32_t)G.taken;
         }
-    }
-    __syncthreads();
+        __syncthreads();
+    } while (r_next < R);
     // column pointers, and offsets within the tile: thread tid owns columns kCols tid ...
     {
         uint32_t n[kCols], sum = 0;
@@ -244,74 +351,59 @@ __global__ __launch_bounds__(kPlaceThreads) void place_tile_kernel(
         if (tid == kPlaceThreads - 1 && tile == n_tiles - 1) colptr[C] = base + run;
     }
     __syncthreads();
-    uint64_t start_next;
-    uint32_t len_next;
-    block_segments(0, R, n_tiles, tile, tiles, rowptr, start_next, len_next);
-    for (uint64_t r0 = 0; r0 < R; r0 += kBlockRows) {
-        const uint64_t start = start_next;
-        const uint32_t len = len_next;
-        block_segments(r0 + kBlockRows, R, n_tiles, tile, tiles, rowptr, start_next, len_next);
-        const uint64_t some = __ballot(len != 0);
-        const int n_some = __popcll(some);  // the same in every wavefront
-        if (n_some == 0) continue;
-        // the rows that reach the tile are dealt to the wavefronts; the first 64 entries of each stay
-        // in registers
-        const uint32_t rank = (uint32_t)__popcll(some & ((1ull << lane) - 1ull));
-        auto block = [&](auto slots) {
-            constexpr int Q = decltype(slots)::value;
-            uint32_t col[Q];
-            float val[Q];
-            int row[Q];
-            uint32_t n[Q];
-            uint64_t e0[Q];
+    if (!whole) r_next = 0;
+    do {
+        if (!whole) n_list = list_rows(T, r_next, R, n_tiles, tile, tiles);
+        for (uint32_t g = 0; g < n_list;) {
+            const RowGroup G = row_group(T, rowptr, g, n_list, kUnits);
+            auto group = [&](auto slots) {
+                constexpr int Q = decltype(slots)::value;
+                uint32_t col[Q], r[Q];
+                float val[Q];
+                int at[Q];  // the row's place in the group: its bit in the masks
 #pragma unroll
-            for (int q = 0; q < Q; q++) {
-                const uint64_t at = __ballot(len != 0 && rank == (uint32_t)(wave + kWaves * q));
-                row[q] = at ? __ffsll((unsigned long long)at) - 1 : 0;
-                e0[q] = lane_u64(start, row[q]);
-                n[q] = at ? lane_u32(len, row[q]) : 0u;
-                const bool on = (uint32_t)lane < n[q];
-                col[q] = on ? (uint32_t)(columns[e0[q] + lane] - c0) : ~0u;
-                val[q] = on ? values[e0[q] + lane] : 0.0f;
-            }
+                for (int q = 0; q < Q; q++) {
+                    const uint32_t u = wave + kWaves * q;
+                    uint64_t e0 = 0;
+                    uint32_t n = 0;
+                    at[q] = u < G.units ? G.unit(u, e0, n) : 0;
+                    r[q] = lane_u32(G.word, at[q]) & ((1u << kRowBits) - 1u);
+                    const bool on = (uint32_t)lane < n;
+                    col[q] = on ? (uint32_t)(columns[e0 + lane] - c0) : ~0u;
+                    val[q] = on ? values[e0 + lane] : 0.0f;
+                }
 #pragma unroll
-            for (int q = 0; q < Q; q++) {
-                const uint32_t bit = 1u << (row[q] & 31);
-                uint32_t* mask = s_mask[row[q] >> 5];
-                if (col[q] != ~0u) atomicOr(&mask[col[q]], bit);
-                for (uint32_t i = 64 + lane; i < n[q]; i += 64) atomicOr(&mask[columns[e0[q] + i] - c0], bit);
-            }
+                for (int q = 0; q < Q; q++)
+                    if (col[q] != ~0u) atomicOr(&s_mask[at[q] >> 5][col[q]], 1u << (at[q] & 31));
+                __syncthreads();
+#pragma unroll
+                for (int q = 0; q < Q; q++) {
+                    if (col[q] == ~0u) continue;
+                    const uint32_t below = (1u << (at[q] & 31)) - 1u;
+                    const uint32_t lo = s_mask[0][col[q]];
+                    const uint32_t before =
+                        at[q] < 32 ? __popc(lo & below) : __popc(lo) + __popc(s_mask[1][col[q]] & below);
+                    const uint64_t pos = base + s_next[col[q]] + before;
+                    crow[pos] = r[q];
+                    cval[pos] = stored<VT>(val[q], scale, r[q]);
+                }
+            };
+            if (G.units > 2 * kWaves)
+                group(std::integral_constant<int, 8>{});
+            else
+                group(std::integral_constant<int, 2>{});
             __syncthreads();
 #pragma unroll
-            for (int q = 0; q < Q; q++) {
-                const uint32_t below = (1u << (row[q] & 31)) - 1u;
-                auto place = [&](uint32_t c, float v) {
-                    const uint32_t lo = s_mask[0][c];
-                    const uint32_t before =
-                        row[q] < 32 ? __popc(lo & below) : __popc(lo) + __popc(s_mask[1][c] & below);
-                    const uint64_t pos = base + s_next[c] + before;
-                    crow[pos] = (uint32_t)(r0 + row[q]);
-                    cval[pos] = stored<VT>(v, scale, r0 + row[q]);
-                };
-                if (col[q] != ~0u) place(col[q], val[q]);
-                for (uint32_t i = 64 + lane; i < n[q]; i += 64)
-                    place((uint32_t)(columns[e0[q] + i] - c0), values[e0[q] + i]);
+            for (int i = 0; i < kCols; i++) {
+                const int c = tid + kPlaceThreads * i;
+                s_next[c] += __popc(s_mask[0][c]) + __popc(s_mask[1][c]);
+                s_mask[0][c] = 0u;
+                s_mask[1][c] = 0u;
             }
-        };
-        if (n_some > 2 * kWaves)
-            block(std::integral_constant<int, kPerWave>{});
-        else
-            block(std::integral_constant<int, 2>{});
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < kCols; i++) {
-            const int c = tid + kPlaceThreads * i;
-            s_next[c] += __popc(s_mask[0][c]) + __popc(s_mask[1][c]);
-            s_mask[0][c] = 0u;
-            s_mask[1][c] = 0u;
+            __syncthreads();
+            g += (uint32_t)G.taken;
         }
-        __syncthreads();
-    }
+    } while (!whole && r_next < R);
 }
 
 // ---- The general path (columns in any order, or rows too short for the tile table).
@@ -548,6 +640,7 @@ hipError_t launch_pack_rows(uint64_t R, const uint64_t* rowptr, const float* val
 }
 
 uint64_t csc_tiles(uint64_t C) { return (C + kTileCols - 1) / kTileCols; }
+uint64_t csc_tile_groups(uint64_t C) { return (csc_tiles(C) + kTileGroup - 1) / kTileGroup; }
 
 hipError_t launch_row_tiles(uint64_t R, const uint64_t* rowptr, const uint64_t* columns, const float* values,
                             uint64_t C, uint32_t* tiles, float* scale, uint32_t* unsorted, hipStream_t stream) {
@@ -568,20 +661,18 @@ hipError_t launch_tile_totals(uint64_t R, uint64_t C, const uint32_t* tiles, uin
 
 hipError_t launch_place_tiles(int vtype, uint64_t R, uint64_t C, const uint32_t* tiles, const uint64_t* rowptr,
                               const uint64_t* columns, const float* values, const float* scale,
-                              const uint64_t* tile_base, uint64_t* colptr, uint32_t* crow, void* cval,
-                              hipStream_t stream) {
+                              const uint64_t* tile_base, uint32_t* order, uint64_t* colptr, uint32_t* crow,
+                              void* cval, hipStream_t stream) {
     if (C == 0) return hipSuccess;
     const uint32_t n_tiles = (uint32_t)csc_tiles(C);
-    const dim3 g(n_tiles), b(kPlaceThreads);
-    if (vtype == FD_VAL_F32)
-        hipLaunchKernelGGL(place_tile_kernel<FD_VAL_F32>, g, b, 0, stream, R, C, n_tiles, tiles, rowptr, columns,
-                           values, scale, tile_base, colptr, crow, cval);
-    else if (vtype == FD_VAL_BF16)
-        hipLaunchKernelGGL(place_tile_kernel<FD_VAL_BF16>, g, b, 0, stream, R, C, n_tiles, tiles, rowptr, columns,
-                           values, scale, tile_base, colptr, crow, cval);
-    else
-        hipLaunchKernelGGL(place_tile_kernel<FD_VAL_FP16>, g, b, 0, stream, R, C, n_tiles, tiles, rowptr, columns,
-                           values, scale, tile_base, colptr, crow, cval);
+    const uint32_t n_groups = (uint32_t)csc_tile_groups(C);
+    hipLaunchKernelGGL(tile_order_kernel, dim3(1), dim3(1024), 0, stream, n_tiles, tile_base, order);
+    const dim3 g((n_groups + kXcd - 1) / kXcd * kXcd * kTileGroup), b(kPlaceThreads);
+    const auto kernel = vtype == FD_VAL_F32    ? place_tile_kernel<FD_VAL_F32>
+                        : vtype == FD_VAL_BF16 ? place_tile_kernel<FD_VAL_BF16>
+                                               : place_tile_kernel<FD_VAL_FP16>;
+    hipLaunchKernelGGL(kernel, g, b, 0, stream, R, C, n_tiles, tiles, rowptr, columns, values, scale, tile_base, order,
+                       colptr, crow, cval);
     return hipGetLastError();
 }
 

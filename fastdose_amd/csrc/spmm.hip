@@ -64,9 +64,9 @@ int hip_result(hipError_t e) {
 int build_by_tiles(const fd_dosemat* m, fd_spmm& p, const uint64_t* rowptr, hipStream_t s, bool* built) {
     const uint64_t nt = csc_tiles(p.cols), R = p.rows;
     DevBuf<uint64_t> base;    // exclusive scan of the tiles' totals (nt + 1), then the scan's scratch
-    DevBuf<uint32_t> total;   // entries of each tile (nt), unsorted flag, the tile table
+    DevBuf<uint32_t> total;   // entries of each tile (nt), unsorted flag, the tile table, the tiles' order
     int r = base.reserve(nt + 1 + scan_scratch_size(nt));
-    if (r == FD_OK) r = total.reserve(nt + 1 + R * (nt + 1));
+    if (r == FD_OK) r = total.reserve(nt + 1 + R * (nt + 1) + csc_tile_groups(p.cols));
     auto enqueue = [&]() -> hipError_t {
         uint32_t unsorted = 0;
         uint32_t* tiles = total.ptr + nt + 1;
@@ -82,7 +82,7 @@ int build_by_tiles(const fd_dosemat* m, fd_spmm& p, const uint64_t* rowptr, hipS
         if (e == hipSuccess) e = launch_scan_u32(total.ptr, nt, base.ptr, base.ptr + nt, base.ptr + nt + 1, s);
         if (e == hipSuccess)
             e = launch_place_tiles(p.vtype, R, p.cols, tiles, rowptr, m->columns.ptr, m->values.ptr, p.scale.ptr,
-                                   base.ptr, p.colptr.ptr, p.crow.ptr, p.cval.ptr, s);
+                                   base.ptr, tiles + R * (nt + 1), p.colptr.ptr, p.crow.ptr, p.cval.ptr, s);
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         *built = e == hipSuccess;
         return e;

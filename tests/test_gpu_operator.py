@@ -117,6 +117,34 @@ def test_general_path_gives_the_same_operator(torch_cuda):
     assert np.all(np.abs(got - want) <= 4 * U * want)
 
 
+@pytest.mark.parametrize("R,cols", [(1472, 2048), (1473, 2049), (1985, 4096), (4100, 40 * 2048 + 1)])
+def test_rows_beyond_one_list(torch_cuda, R, cols):
+    """Up to 1984 rows that reach a tile are listed at once, 512 rows of the matrix at a time: all rows
+    reach the first tile here, most with a few entries and some with all its columns (32 units of 64).
+    The general path, which takes them in another order, is the reference: same bits."""
+    torch = torch_cuda
+    rng = np.random.default_rng([R, cols])
+    rows = []
+    for r in range(R):
+        c = np.concatenate([rng.integers(0, 2048, 4), rng.integers(0, cols, 3)])
+        if r % 200 == 77:
+            c = np.arange(min(cols, 2048))
+        rows.append(np.unique(c))
+    off = np.concatenate([[0], np.cumsum([len(c) for c in rows])])
+    c = np.concatenate(rows).astype(np.int64)
+    v = rng.uniform(0.01, 1.0, len(c)).astype(np.float32)
+    back = np.concatenate([np.arange(off[r], off[r + 1])[::-1] for r in range(R)])
+    x = torch.rand((R, 3), device="cuda")
+    y = []
+    for m in ((off, c, v), (off, c[back], v[back])):
+        with fd.Spmm(dose_mat(torch, cols, [m])) as op:
+            y.append(op.run(x).cpu().numpy())
+    assert np.array_equal(*y)
+    D = np.zeros(cols)
+    np.add.at(D, c, v.astype(np.float64) * np.repeat(x[:, 0].cpu().numpy().astype(np.float64), np.diff(off)))
+    assert np.allclose(y[0][:, 0], D, rtol=R * U)
+
+
 @pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 7, 8, 12, 16, 20, 31, 33, 64, 65, 100, 128, 130, 132, 256, 260])
 def test_product_over_lane_arrangements(torch_cuda, k):
     """Sparse, medium and crowded stretches of columns (each picks its own lanes per column, the crowded
