@@ -98,7 +98,7 @@ hipError_t launch_resample_compact(int n, int Z, const uint64_t* cand_off, const
                                    hipStream_t stream);
 
 // Exclusive scan of count[0..N) (u32) into off[0..N) (u64) plus total[0] = sum.  With scratch
-// (scan_scratch_size(N) u64, nullable) large inputs take a three-pass multi-workgroup scan.
+// (scan_scratch_size(N) u64, nullable) large inputs take a scan by many workgroups.
 hipError_t launch_scan_u32(const uint32_t* count, uint64_t N, uint64_t* off, uint64_t* total, uint64_t* scratch,
                            hipStream_t stream);
 uint64_t scan_scratch_size(uint64_t N);

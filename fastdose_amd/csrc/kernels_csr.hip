@@ -15,41 +15,10 @@ namespace {
 
 constexpr int kScanThreads = 1024;
 
-// Single-workgroup exclusive scan: thread i owns a contiguous chunk of the input.
-__global__ __launch_bounds__(kScanThreads) void scan_u32_kernel(const uint32_t* __restrict__ count, uint64_t N,
-                                                                uint64_t* __restrict__ off,
-                                                                uint64_t* __restrict__ total) {
-    __shared__ uint64_t s_part[kScanThreads];
-    const uint64_t chunk = (N + kScanThreads - 1) / kScanThreads;
-    const uint64_t lo = (uint64_t)threadIdx.x * chunk;
-    const uint64_t hi = lo + chunk < N ? lo + chunk : N;
-    uint64_t sum = 0;
-    for (uint64_t i = lo; i < hi; i++) sum += count[i];
-    s_part[threadIdx.x] = sum;
-    __syncthreads();
-    // Hillis-Steele over the 1024 partial sums
-    for (int o = 1; o < kScanThreads; o <<= 1) {
-        uint64_t v = threadIdx.x >= (unsigned)o ? s_part[threadIdx.x - o] : 0;
-        __syncthreads();
-        s_part[threadIdx.x] += v;
-        __syncthreads();
-    }
-    uint64_t run = s_part[threadIdx.x] - sum;
-    for (uint64_t i = lo; i < hi; i++) {
-        off[i] = run;
-        run += count[i];
-    }
-    if (threadIdx.x == kScanThreads - 1) total[0] = s_part[kScanThreads - 1];
-}
-
-// Three-pass scan for large inputs: tile sums, a scan of the tile sums, tile scans.  A tile is
-// 4096 elements, 16 consecutive ones per thread.
-constexpr int kTileThreads = 256;
-constexpr int kTileItems = 16;
-constexpr uint64_t kTile = (uint64_t)kTileThreads * kTileItems;
-
+// Exclusive scan of a value per thread of a workgroup of WAVES wavefronts, and the total.
+template <int WAVES>
 __device__ __forceinline__ uint64_t block_excl_scan_u64(uint64_t v, uint64_t* s_wave, uint64_t& total) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     uint64_t x = v;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -58,70 +27,130 @@ __device__ __forceinline__ uint64_t block_excl_scan_u64(uint64_t v, uint64_t* s_
     }
     if (lane == 63) s_wave[wave] = x;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        uint64_t acc = 0;
-        for (int w = 0; w < nw; w++) {
-            const uint64_t t = s_wave[w];
-            s_wave[w] = acc;
-            acc += t;
-        }
-        s_wave[nw] = acc;
+    uint64_t before = 0;
+    total = 0;
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) {  // independent reads, unlike one thread's running sum
+        const uint64_t t = s_wave[w];
+        before += w < wave ? t : 0;
+        total += t;
     }
     __syncthreads();
-    const uint64_t res = s_wave[wave] + x - v;
-    total = s_wave[nw];
-    __syncthreads();
-    return res;
+    return before + x - v;
 }
+
+// Thread's kScanItems consecutive elements from `at` on, and their exclusive sums from run on
+constexpr int kScanItems = 16;
+__device__ __forceinline__ uint64_t load_items(const uint32_t* __restrict__ count, uint64_t at, uint64_t N,
+                                               uint32_t (&c)[kScanItems]) {
+    uint64_t sum = 0;
+    if (at + kScanItems <= N && (reinterpret_cast<uintptr_t>(count) & 15) == 0) {  // at is a multiple of 16
+#pragma unroll
+        for (int i = 0; i < kScanItems / 4; i++) {
+            const uint4 q = reinterpret_cast<const uint4*>(count + at)[i];
+            c[4 * i] = q.x;
+            c[4 * i + 1] = q.y;
+            c[4 * i + 2] = q.z;
+            c[4 * i + 3] = q.w;
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < kScanItems; i++) c[i] = at + i < N ? count[at + i] : 0u;
+    }
+#pragma unroll
+    for (int i = 0; i < kScanItems; i++) sum += c[i];
+    return sum;
+}
+__device__ __forceinline__ void store_items(uint64_t* __restrict__ off, uint64_t at, uint64_t N, uint64_t run,
+                                            const uint32_t (&c)[kScanItems]) {
+    if (at + kScanItems <= N && (reinterpret_cast<uintptr_t>(off) & 15) == 0) {
+#pragma unroll
+        for (int i = 0; i < kScanItems / 2; i++) {
+            const uint64_t second = run + c[2 * i];
+            reinterpret_cast<ulonglong2*>(off + at)[i] = make_ulonglong2(run, second);
+            run = second + c[2 * i + 1];
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < kScanItems; i++) {
+            if (at + i < N) off[at + i] = run;
+            run += c[i];
+        }
+    }
+}
+
+// Exclusive scan by one workgroup, kScanPass elements at a time.
+constexpr uint64_t kScanPass = (uint64_t)kScanThreads * kScanItems;
+__global__ __launch_bounds__(kScanThreads) void scan_u32_kernel(const uint32_t* __restrict__ count, uint64_t N,
+                                                                uint64_t* __restrict__ off,
+                                                                uint64_t* __restrict__ total) {
+    __shared__ uint64_t s_wave[kScanThreads / 64];
+    uint64_t carry = 0;
+    for (uint64_t base = 0; base < N; base += kScanPass) {
+        const uint64_t at = base + (uint64_t)threadIdx.x * kScanItems;
+        uint32_t c[kScanItems];
+        uint64_t sum;
+        const uint64_t run = block_excl_scan_u64<kScanThreads / 64>(load_items(count, at, N, c), s_wave, sum);
+        store_items(off, at, N, carry + run, c);
+        carry += sum;
+    }
+    if (threadIdx.x == 0) total[0] = carry;
+}
+
+// Larger inputs in two kernels: the sums of tiles of 4096 elements, then every tile's scan from the sum
+// of the tiles before it, which its workgroup adds up itself (up to kScanTiles of them; beyond, a third
+// kernel scans the tile sums in between).
+constexpr int kTileThreads = 256;
+constexpr uint64_t kTile = (uint64_t)kTileThreads * kScanItems;
+constexpr uint64_t kScanTiles = 4096;
 
 __global__ __launch_bounds__(kTileThreads) void scan_tile_sums_kernel(const uint32_t* __restrict__ count, uint64_t N,
                                                                       uint64_t* __restrict__ sums) {
-    __shared__ uint64_t s_wave[kTileThreads / 64 + 1];
-    const uint64_t base = (uint64_t)blockIdx.x * kTile + (uint64_t)threadIdx.x * kTileItems;
-    uint64_t v = 0;
-#pragma unroll
-    for (int i = 0; i < kTileItems; i++)
-        if (base + i < N) v += count[base + i];
+    __shared__ uint64_t s_wave[kTileThreads / 64];
+    const uint64_t at = (uint64_t)blockIdx.x * kTile + (uint64_t)threadIdx.x * kScanItems;
+    uint32_t c[kScanItems];
     uint64_t total;
-    block_excl_scan_u64(v, s_wave, total);
+    block_excl_scan_u64<kTileThreads / 64>(load_items(count, at, N, c), s_wave, total);
     if (threadIdx.x == 0) sums[blockIdx.x] = total;
 }
 
 // exclusive scan of the tile sums in place (one workgroup), grand total to total[0]
 __global__ __launch_bounds__(1024) void scan_sums_kernel(uint64_t* __restrict__ sums, uint64_t nb,
                                                          uint64_t* __restrict__ total) {
-    __shared__ uint64_t s_wave[1024 / 64 + 1];
+    __shared__ uint64_t s_wave[1024 / 64];
     uint64_t carry = 0;
     for (uint64_t i0 = 0; i0 < nb; i0 += blockDim.x) {
         const uint64_t i = i0 + threadIdx.x;
         const uint64_t v = i < nb ? sums[i] : 0;
         uint64_t tot;
-        const uint64_t ex = block_excl_scan_u64(v, s_wave, tot);
+        const uint64_t ex = block_excl_scan_u64<1024 / 64>(v, s_wave, tot);
         if (i < nb) sums[i] = carry + ex;
         carry += tot;
     }
     if (threadIdx.x == 0) total[0] = carry;
 }
 
+// SCANNED: sums holds exclusive sums (and total is written already)
+template <bool SCANNED>
 __global__ __launch_bounds__(kTileThreads) void scan_tiles_kernel(const uint32_t* __restrict__ count, uint64_t N,
                                                                   const uint64_t* __restrict__ sums,
-                                                                  uint64_t* __restrict__ off) {
-    __shared__ uint64_t s_wave[kTileThreads / 64 + 1];
-    const uint64_t base = (uint64_t)blockIdx.x * kTile + (uint64_t)threadIdx.x * kTileItems;
-    uint32_t c[kTileItems];
-    uint64_t v = 0;
-#pragma unroll
-    for (int i = 0; i < kTileItems; i++) {
-        c[i] = base + i < N ? count[base + i] : 0u;
-        v += c[i];
+                                                                  uint64_t* __restrict__ off,
+                                                                  uint64_t* __restrict__ total) {
+    __shared__ uint64_t s_wave[kTileThreads / 64];
+    const uint64_t at = (uint64_t)blockIdx.x * kTile + (uint64_t)threadIdx.x * kScanItems;
+    uint32_t c[kScanItems];
+    const uint64_t v = load_items(count, at, N, c);
+    uint64_t before = 0, sum;
+    if (SCANNED) {
+        before = sums[blockIdx.x];
+    } else {
+        uint64_t mine = 0;
+        for (uint32_t b = threadIdx.x; b < blockIdx.x; b += kTileThreads) mine += sums[b];
+        block_excl_scan_u64<kTileThreads / 64>(mine, s_wave, before);
     }
-    uint64_t total;
-    uint64_t run = sums[blockIdx.x] + block_excl_scan_u64(v, s_wave, total);
-#pragma unroll
-    for (int i = 0; i < kTileItems; i++) {
-        if (base + i < N) off[base + i] = run;
-        run += c[i];
-    }
+    const uint64_t run = before + block_excl_scan_u64<kTileThreads / 64>(v, s_wave, sum);
+    store_items(off, at, N, run, c);
+    if (!SCANNED && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) total[0] = before + sum;
 }
 
 // Dense -> CSR works on segments: runs of consecutive elements of one row, one wavefront each.  A beam's
@@ -211,14 +240,21 @@ uint64_t scan_scratch_size(uint64_t N) { return (N + kTile - 1) / kTile + 1; }
 
 hipError_t launch_scan_u32(const uint32_t* count, uint64_t N, uint64_t* off, uint64_t* total, uint64_t* scratch,
                            hipStream_t stream) {
-    if (!scratch || N <= kTile) {
+    // one workgroup takes 5 us for up to a pass, and 7 for every further one; two kernels take 9
+    if (!scratch || N <= kScanPass) {
         hipLaunchKernelGGL(scan_u32_kernel, dim3(1), dim3(kScanThreads), 0, stream, count, N, off, total);
         return hipGetLastError();
     }
     const uint64_t nb = (N + kTile - 1) / kTile;
     hipLaunchKernelGGL(scan_tile_sums_kernel, dim3((unsigned)nb), dim3(kTileThreads), 0, stream, count, N, scratch);
+    if (nb <= kScanTiles) {
+        hipLaunchKernelGGL(scan_tiles_kernel<false>, dim3((unsigned)nb), dim3(kTileThreads), 0, stream, count, N,
+                           scratch, off, total);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(scan_sums_kernel, dim3(1), dim3(1024), 0, stream, scratch, nb, total);
-    hipLaunchKernelGGL(scan_tiles_kernel, dim3((unsigned)nb), dim3(kTileThreads), 0, stream, count, N, scratch, off);
+    hipLaunchKernelGGL(scan_tiles_kernel<true>, dim3((unsigned)nb), dim3(kTileThreads), 0, stream, count, N, scratch,
+                       off, total);
     return hipGetLastError();
 }
 

@@ -117,6 +117,25 @@ def test_general_path_gives_the_same_operator(torch_cuda):
     assert np.all(np.abs(got - want) <= 4 * U * want)
 
 
+@pytest.mark.parametrize("cols", [16383, 16384, 16385, 40961, 4096 ** 2, 4096 ** 2 + 1])
+def test_scan_of_column_counts(torch_cuda, cols):
+    """The general path scans one count per column: by one workgroup, in two kernels, in three."""
+    torch = torch_cuda
+    rng = np.random.default_rng(cols)
+    R = 300
+    c = np.sort(rng.choice(cols, (R, 2)), 1).astype(np.int64)
+    c[0] = [0, cols - 1]
+    c[:, 0] = np.where(c[:, 0] == c[:, 1], (c[:, 0] + 1) % cols, c[:, 0])
+    c = c[:, ::-1].copy()  # not ascending
+    v = rng.uniform(0.01, 1.0, 2 * R).astype(np.float32)
+    with fd.Spmm(dose_mat(torch, cols, [(np.arange(0, 2 * R + 1, 2), c.reshape(-1), v)])) as op:
+        x = torch.rand((R, 1), device="cuda")
+        got = op.run(x).cpu().numpy()[:, 0].astype(np.float64)
+    want = np.zeros(cols)
+    np.add.at(want, c.reshape(-1), v.astype(np.float64) * np.repeat(x.cpu().numpy()[:, 0].astype(np.float64), 2))
+    assert np.all(np.abs(got - want) <= 2 * R * U * want)
+
+
 @pytest.mark.parametrize("R,cols", [(1472, 2048), (1473, 2049), (1985, 4096), (4100, 40 * 2048 + 1)])
 def test_rows_beyond_one_list(torch_cuda, R, cols):
     """Up to 1984 rows that reach a tile are listed at once, 512 rows of the matrix at a time: all rows
