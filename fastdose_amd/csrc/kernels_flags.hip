@@ -2,17 +2,20 @@
 //
 // d_beamletFlagInit (IMRTOpt/src/IMRTBeamBundle.cu:130-316): a beamlet of a bundle is active if
 // any of its 3 x 3 lateral sample rays, at any of the central beam's long_dim depths, lands where
-// the linearly filtered PTV mask is positive.  One wavefront per (beamlet, bundle): lanes take the
-// (depth, sample) points in the host loop's order 64 at a time and stop at the first chunk with a
-// hit (the flag is an OR, so the early exit does not change it).  The point arithmetic is the host
+// the linearly filtered PTV mask is positive.  One wavefront per (beamlet, bundle): each lane keeps one
+// of the nine rays and takes every seventh depth, and the wavefront stops after the seven depths with a
+// hit (the flag is an OR, so neither order nor early exit changes it).  The point arithmetic is the host
 // code's FP32 sequence (explicit fmaf, IEEE division, no contraction), so flags are bit-identical
 // to fd_beamlet_flags_host.
 //
 // A plan's target fills a small part of the volume and most candidate beamlets miss it, which took the
 // walk of every point with its eight texel reads.  A first kernel finds the mask's bounding box
 // (reading the mask once); a beamlet then walks only the depths at which one of its nine rays can be
-// inside it, and a point reads texels only if its base texel is.  180 beams of 400 beamlets on
-// 200 x 200 x 160: 1.35 -> 0.13 ms.
+// inside it, and a point reads texels only if its base texel is.  What is left is the arithmetic of the
+// points in the box around the target, so a lane computes its ray once and divides by multiplying with
+// the reciprocal and correcting (Divisor).  180 beams of 400 beamlets on 200 x 200 x 160: 1.35 ms for
+// every point, 0.13 ms for those in the box, 0.065 ms with the texels of a point read at once (serial
+// reads with a branch each before: the loops took as many scalar instructions as vector ones).
 #include <hip/hip_runtime.h>
 
 #include "kernels.h"
@@ -49,11 +52,34 @@ __global__ __launch_bounds__(256) void mask_box_kernel(const uint8_t* __restrict
     }
     for (uint64_t i = head + 16 * quads + id; i < n; i += all)
         if (mask[i]) add(i);
+    __shared__ uint32_t s_lo[6];
+    if (threadIdx.x < 6) s_lo[threadIdx.x] = ~0u;
+    __syncthreads();
     for (int d = 0; d < 6; d++) {
         for (int o = 32; o > 0; o >>= 1) lo[d] = min(lo[d], (uint32_t)__shfl_xor((int)lo[d], o, 64));
-        if ((threadIdx.x & 63) == 0 && lo[d] != ~0u) atomicMin(&box[d], lo[d]);
+        if ((threadIdx.x & 63) == 0 && lo[d] != ~0u) atomicMin(&s_lo[d], lo[d]);
     }
+    __syncthreads();
+    if (threadIdx.x < 6 && s_lo[threadIdx.x] != ~0u) atomicMin(&box[threadIdx.x], s_lo[threadIdx.x]);
 }
+
+// x / v as the IEEE division rounds it, in three instructions: with r = 1 / v rounded, x r corrected by
+// its exact remainder times r is the rounded quotient (Markstein's theorem) unless v's significand is
+// all ones or a step leaves the normal range; such divisors are divided by.  (Quotients out of range,
+// infinities and NaN fail the box test either way; quotients below 2^-60 or so are rounded away by the
+// half texel subtracted from them.)
+struct Divisor {
+    float v, r;
+    bool plain;
+    __device__ __forceinline__ explicit Divisor(float d) : v(d), r(1.0f / d) {
+        plain = (__float_as_uint(d) & 0x7FFFFFu) != 0x7FFFFFu && d > 0x1p-40f && d < 0x1p40f;
+    }
+    __device__ __forceinline__ float of(float x) const {
+        if (!plain) return x / v;
+        const float q = x * r;
+        return fmaf(fmaf(-q, v, x), r, q);
+    }
+};
 
 // The box as signed texel bounds [lo, hi] (lo > hi when empty).
 struct MaskBox {
@@ -70,33 +96,46 @@ __device__ __forceinline__ MaskBox read_box(const uint32_t* __restrict__ box) {
 }
 
 // Linear-filtered binary mask > 0 at unnormalised texture coordinates (texel i spans [i, i+1),
-// border 0): true iff a texel with nonzero weight is set.
+// border 0): true iff a texel with nonzero weight is set.  The up to eight texels are read as four pairs
+// along x, all in flight, at coordinates moved into the volume; what was moved or has no weight is
+// masked off.
 __device__ bool mask_hit_dev(const uint8_t* __restrict__ mask, int X, int Y, int Z, const MaskBox& box, float cx,
                              float cy, float cz) {
     const float t[3] = {cx - 0.5f, cy - 0.5f, cz - 0.5f};
-    int base[3], reach[3];
+    int base[3];
+    bool two[3];  // the texel after the base texel has weight
 #pragma unroll
     for (int d = 0; d < 3; d++) {
         const float f = floorf(t[d]);
         // texels base and base + 1 at most: one of them lies in the box
         if (!(f >= (float)(box.lo[d] - 1) && f <= (float)box.hi[d])) return false;
         base[d] = (int)f;
-        reach[d] = (t[d] - f) > 0.0f ? 2 : 1;
+        two[d] = (t[d] - f) > 0.0f;
     }
-    for (int k = 0; k < reach[2]; k++) {
-        const int z = base[2] + k;
-        if (z < 0 || z >= Z) continue;
-        for (int j = 0; j < reach[1]; j++) {
-            const int y = base[1] + j;
-            if (y < 0 || y >= Y) continue;
-            for (int i = 0; i < reach[0]; i++) {
-                const int x = base[0] + i;
-                if (x < 0 || x >= X) continue;
-                if (mask[(size_t)x + (size_t)X * ((size_t)y + (size_t)Y * z)]) return true;
-            }
+    const int x = base[0];
+    // the pair's bytes: texels x and x + 1, or the volume's first or last two where x is -1 or X - 1
+    const int at = min(max(x, 0), max(X - 2, 0));
+    uint32_t low = 0, high = 0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int y = base[1] + (k & 1), z = base[2] + (k >> 1);
+        const bool row = y >= 0 && y < Y && z >= 0 && z < Z && (!(k & 1) || two[1]) && (!(k >> 1) || two[2]);
+        const size_t o = (size_t)at + (size_t)X * ((size_t)min(max(y, 0), Y - 1) + (size_t)Y * min(max(z, 0), Z - 1));
+        uint32_t w;
+        if (X >= 2) {
+            uint16_t pair;
+            __builtin_memcpy(&pair, mask + o, 2);
+            w = pair;
+        } else {
+            w = mask[o];
         }
+        w = row ? w : 0u;
+        low |= w & 255u;
+        high |= w >> 8;
     }
-    return false;
+    const uint32_t first = x < 0 ? 0u : (x > at ? high : low);
+    const uint32_t second = x < 0 ? low : (x == at ? high : 0u);  // x = X - 1: none
+    return first != 0u || (two[0] && second != 0u);
 }
 
 // BEV -> PVCS direction of sample ray r (j, k) of beamlet (bx, by), the host's FP32 sequence.
@@ -110,35 +149,41 @@ __device__ __forceinline__ void sample_ray(const FlagBeamDev& d, int bx, int by,
     p[2] = fmaf(d.Ri[8], dz, fmaf(d.Ri[7], dy, d.Ri[6] * dx));
 }
 
+// 1 / x to about 1e-14 (the hardware's FP64 reciprocal and one Newton step).
+__device__ __forceinline__ double reciprocal(double x) {
+    const double r = __builtin_amdgcn_rcp(x);
+    return fma(fma(-x, r, 1.0), r, r);
+}
+
 // Depth indices [i0, i1) of the ray with direction p at which a point (src + p depth / sad) / v can have
 // its base texel within [lo - 1, hi] of the box: the ray's interval in FP64, widened by 0.05 texel plus
 // 1e-5 of the coordinates' magnitude (the FP32 points are within a few 1e-7 of it) and by one index
-// either way.  All depths for values too large to bound so.  (FP32 intervals take 5 % less time.)
+// either way.  All depths for values too large to bound so.  Most beamlets end here, so there is one
+// reciprocal per axis and no branch on the direction's sign (with divisions and branches the kernel took
+// 2 % longer; FP64 multiply-adds run at the rate of FP32 ones).
 __device__ __forceinline__ void ray_depths(const FlagBeamDev& d, const MaskBox& box, const float p[3],
                                            const float v[3], int& i0, int& i1) {
     double lo = 0.0, hi = 1e30;  // scale = depth / sad
-    const double far_scale = ((double)d.lim_min + (double)d.L * d.ls) / d.sad;
-    bool odd = !(far_scale < 1e9 && far_scale > 0.0);
+    const double far_scale = fma((double)d.L, (double)d.ls, (double)d.lim_min) * reciprocal(d.sad);
+    bool odd = !(far_scale < 1e9 && far_scale > 0.0 && d.ls > 0.0f);
+#pragma unroll
     for (int a = 0; a < 3; a++) {
         const double s = d.src[a], q = p[a], u = v[a];
         odd |= !(fabs(s) < 1e9 && fabs(q) < 1e9 && u > 1e-9);
         const double m = u * 0.05 + 1e-5 * (fabs(s) + fabs(q) * far_scale);
         // base texel in [lo - 1, hi]: coordinate / v in [lo - 0.5, hi + 1.5)
         const double x0 = (box.lo[a] - 0.5) * u - m - s, x1 = (box.hi[a] + 1.5) * u + m - s;
-        if (q > 0.0) {
-            lo = fmax(lo, x0 / q);
-            hi = fmin(hi, x1 / q);
-        } else if (q < 0.0) {
-            lo = fmax(lo, x1 / q);
-            hi = fmin(hi, x0 / q);
-        } else if (x0 > 0.0 || x1 < 0.0) {
-            hi = -1.0;
-        }
+        // a direction component below 1e-20 moves by less than the margin over the whole depth
+        const bool still = fabs(q) < 1e-20;
+        const double r = reciprocal(still ? 1.0 : q), t0 = x0 * r, t1 = x1 * r;
+        lo = still ? lo : fmax(lo, fmin(t0, t1));
+        hi = still ? (x0 > 0.0 || x1 < 0.0 ? -1.0 : hi) : fmin(hi, fmax(t0, t1));
     }
     i0 = 0;
     i1 = d.L;
     if (odd) return;
-    const double L = d.L, a0 = (lo * d.sad - d.lim_min) / d.ls - 1.0, a1 = (hi * d.sad - d.lim_min) / d.ls + 2.0;
+    const double L = d.L, r = reciprocal(d.ls);
+    const double a0 = (lo * d.sad - d.lim_min) * r - 1.0, a1 = (hi * d.sad - d.lim_min) * r + 2.0;
     if (!(lo <= hi) || a0 >= L || a1 <= 0.0) {
         i1 = 0;
         return;
@@ -161,37 +206,29 @@ __global__ __launch_bounds__(64 * kFlagWaves) void beamlet_flags_kernel(const Fl
     const int bx = idx % d.fx, by = idx / d.fx;
     const MaskBox box = read_box(mask_box);
     const float v[3] = {vx, vy, vz};
-    // the depths at which one of the nine rays can be inside the mask's box
-    int first = d.L, last = 0;
-    if (lane < kFlagSS * kFlagSS && box.lo[0] <= box.hi[0]) {
-        float p[3];
-        int i0, i1;
-        sample_ray(d, bx, by, lane, p);
-        ray_depths(d, box, p, v, i0, i1);
-        if (i0 < i1) {
-            first = i0;
-            last = i1;
-        }
-    }
+    // my ray, and the depths at which it and the wavefront's nine rays can be inside the mask's box
+    constexpr int kRays = kFlagSS * kFlagSS, kDepths = 64 / kRays;
+    float p[3];
+    sample_ray(d, bx, by, lane % kRays, p);
+    int i0 = d.L, i1 = 0;
+    if (box.lo[0] <= box.hi[0]) ray_depths(d, box, p, v, i0, i1);
+    int first = i0 < i1 ? i0 : d.L, last = i0 < i1 ? i1 : 0;
     for (int o = 8; o > 0; o >>= 1) {  // lanes 0 ... 15 hold the nine rays
         first = min(first, __shfl_xor(first, o, 64));
         last = max(last, __shfl_xor(last, o, 64));
     }
     first = __builtin_amdgcn_readfirstlane(first);
     last = __builtin_amdgcn_readfirstlane(last);
-    const int total = last * kFlagSS * kFlagSS;
+    if (lane >= kRays * kDepths) i1 = 0;  // the 64th lane has no depth of its own
+    const Divisor by_sad(d.sad), by_vx(vx), by_vy(vy), by_vz(vz);
     bool on = false;
-    for (int t0 = first * kFlagSS * kFlagSS; t0 < total && !on; t0 += 64) {
-        const int t = t0 + lane;
+    for (int i = first + lane / kRays; first < last && !on; i += kDepths, first += kDepths) {
         bool hit = false;
-        if (t < total) {
-            const uint32_t i = (uint32_t)(t / (kFlagSS * kFlagSS));
+        if (i >= i0 && i < i1) {
             const float depth = d.lim_min + (float)i * d.ls;
-            const float scale = depth / d.sad;
-            float p[3];
-            sample_ray(d, bx, by, t - (int)i * kFlagSS * kFlagSS, p);
-            hit = mask_hit_dev(mask, X, Y, Z, box, fmaf(p[0], scale, d.src[0]) / vx,
-                               fmaf(p[1], scale, d.src[1]) / vy, fmaf(p[2], scale, d.src[2]) / vz);
+            const float scale = by_sad.of(depth);
+            hit = mask_hit_dev(mask, X, Y, Z, box, by_vx.of(fmaf(p[0], scale, d.src[0])),
+                               by_vy.of(fmaf(p[1], scale, d.src[1])), by_vz.of(fmaf(p[2], scale, d.src[2])));
         }
         on = __any(hit);
     }

@@ -72,3 +72,33 @@ def test_flags_equal_the_host(torch_cuda, name):
                 assert np.array_equal(w, g)
     if name in ("full", "plane"):
         assert any(w.any() for w in want)
+
+
+@pytest.mark.parametrize("voxel", [0.25, 0.3, float(np.uint32(0x3E7FFFFF).view(np.float32))])
+@pytest.mark.parametrize("dim", [(1, 29, 23), (2, 1, 23), (3, 29, 1), (24, 17, 2)])
+def test_flags_in_thin_volumes(torch_cuda, dim, voxel):
+    """Volumes one to three voxels wide, where the pair of texels read along x does not fit or is the whole
+    row, and voxel sizes whose division is exact, corrected, and (all ones in the significand) done as a
+    division; beams shifted so that sample points fall on texel boundaries among others."""
+    torch = torch_cuda
+    vol = synth.make_volume(dim, voxel)
+    rng = np.random.default_rng(list(dim))
+    masks = [(rng.random(dim[::-1]) < f).astype(np.uint8) for f in (0.02, 0.3)] + [np.ones(dim[::-1], np.uint8)]
+    iso = [voxel * d / 2 for d in dim]
+    bundles = []
+    for a in [(0, 0, 0), (90, 0, 0), (90, 90, 0)] + [tuple(rng.uniform(0, 360, 3)) for _ in range(9)]:
+        at = [c + float(rng.integers(-2, 3)) * voxel / 2 for c in iso]
+        bundles.append(synth.make_bundle(at, a, fluence_dim=int(rng.integers(1, 12)), beamlet_size=3 * voxel,
+                                         long_spacing=voxel))
+    some = 0
+    with fd.Context(vol, np.ones(dim[::-1], np.float32), synth.synthetic_spectrum(1), synth.synthetic_kernel(1)) as ctx:
+        for m in masks:
+            got = ctx.beamlet_flags(torch.from_numpy(m.reshape(-1)).cuda(), bundles)
+            for b, g in zip(bundles, got):
+                try:
+                    w = fd.beamlet_flag_init(b, m, vol)
+                except fd.FastDoseError:
+                    w = np.zeros(b.fluence_dim[0] ** 2, np.uint8)
+                assert np.array_equal(w, g)
+                some += int(w.any())
+    assert some > 0
