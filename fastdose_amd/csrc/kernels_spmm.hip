@@ -472,11 +472,17 @@ __global__ void col_sort_kernel(uint64_t C, const uint64_t* __restrict__ colptr,
     }
 }
 
+// An entry's stored number, and its value (16-bit numbers are fractions of the row maximum)
 template <int VT>
-__device__ __forceinline__ float entry_value(const void* cval, uint64_t e, const float* scale, uint32_t r) {
+__device__ __forceinline__ float stored_number(const void* cval, uint64_t e) {
     if (VT == FD_VAL_F32) return ((const float*)cval)[e];
     const uint16_t h = ((const uint16_t*)cval)[e];
-    return (VT == FD_VAL_BF16 ? bf16_to_f32(h) : fp16_to_f32(h)) * scale[r];
+    return VT == FD_VAL_BF16 ? bf16_to_f32(h) : fp16_to_f32(h);
+}
+template <int VT>
+__device__ __forceinline__ float entry_value(const void* cval, uint64_t e, const float* scale, uint32_t r) {
+    const float q = stored_number<VT>(cval, e);
+    return VT == FD_VAL_F32 ? q : q * scale[r];
 }
 
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -535,18 +541,27 @@ __global__ __launch_bounds__(256) void spmm_wide_kernel(uint64_t C, const uint64
 // entries is split over the four wavefronts (the longest tile would otherwise outlast the rest).
 // One BF16 vector product over 49 M entries (6.4 M voxels, 2 660 rows) takes 0.17 ms where one column
 // per wavefront with lanes along k took 5.4 ms; reading the entries and column pointers (350 MB) is
-// 0.07 ms of it, the rest latency of the x gathers.  Limits of E and kSplitEntries: a factor of two
-// either way costs 5-10 %.
+// 0.07 ms of it, the rest the gathers of rows, scales and x, whose lines keep the L1 busy.  Limits of E
+// and kSplitEntries: a factor of two either way costs 5-10 %.
+// SCALED (16-bit values, one vector): the workgroup holds scale times x of all rows in LDS, one gather
+// instead of two, and takes kScaledGroups times 256 columns to be worth it: 0.17 -> 0.15 ms (512 columns the
+// same, 2048 0.17).  With FP32 values, which have no scale, x in LDS takes 10 % longer, and with
+// four vectors the table's size costs what it saves.  Its length: 16 KiB leave eight workgroups to a CU.
 constexpr uint32_t kSplitEntries = 1024;  // entries of a 64-column tile that is worth splitting
+constexpr uint64_t kScaledRows = 4096, kScaledGroups = 4;
 
-template <int VT, int V, int G>
+template <int VT, int V, int G, bool SCALED = false>
 __global__ __launch_bounds__(256) void spmm_narrow_kernel(uint64_t C, const uint64_t* __restrict__ colptr,
                                                           const uint32_t* __restrict__ crow,
                                                           const void* __restrict__ cval,
                                                           const float* __restrict__ scale,
-                                                          const float* __restrict__ X, int k,
+                                                          const float* __restrict__ X, int k, uint64_t R,
                                                           float* __restrict__ Y) {
     typedef float vec __attribute__((ext_vector_type(V)));
+    static_assert(!SCALED || (V == 1 && G == 1 && VT != FD_VAL_F32), "one vector, 16-bit values");
+    extern __shared__ float s_scaled[];  // SCALED: scale[r] X[r]
+    if (SCALED)  // complete before the first barrier below
+        for (uint64_t r = threadIdx.x; r < R; r += blockDim.x) s_scaled[r] = scale[r] * X[r];
     constexpr int N = 64 / G;  // entry lanes of a wavefront
     constexpr int kUnroll = 4;
     __shared__ uint64_t s_ptr[257];
@@ -593,8 +608,10 @@ __global__ __launch_bounds__(256) void spmm_narrow_kernel(uint64_t C, const uint
 #pragma unroll
                             for (int u = 0; u < kUnroll; u++) {
                                 const uint64_t eu = e + (uint64_t)u * E;
-                                v[u] = entry_value<VT>(cval, eu < b ? eu : b - 1, scale, r[u]);
-                                x[u] = *(const vec*)(X + (uint64_t)r[u] * k + jj);
+                                const uint64_t at = eu < b ? eu : b - 1;
+                                v[u] = SCALED ? stored_number<VT>(cval, at) : entry_value<VT>(cval, at, scale, r[u]);
+                                x[u] = SCALED ? *(const vec*)(s_scaled + r[u])
+                                              : *(const vec*)(X + (uint64_t)r[u] * k + jj);
                             }
 #pragma unroll
                             for (int u = 0; u < kUnroll; u++) {
@@ -711,11 +728,20 @@ namespace {
 
 template <int VT, int V>
 void launch_narrow(int G, const dim3& g, const dim3& b, hipStream_t stream, uint64_t C, const uint64_t* colptr,
-                   const uint32_t* crow, const void* cval, const float* scale, const float* X, int k, float* Y) {
+                   const uint32_t* crow, const void* cval, const float* scale, const float* X, int k, uint64_t R,
+                   float* Y) {
+    if constexpr (VT != FD_VAL_F32 && V == 1)
+        if (G == 1 && R <= kScaledRows) {
+            const dim3 few(blocks_for((C + kScaledGroups - 1) / kScaledGroups, 65536));
+            hipLaunchKernelGGL((spmm_narrow_kernel<VT, 1, 1, true>), few, b, R * sizeof(float), stream, C, colptr, crow,
+                               cval, scale, X, k, R, Y);
+            return;
+        }
     switch (G) {
 #define FD_NARROW(g_)                                                                                             \
     case g_:                                                                                                      \
-        hipLaunchKernelGGL((spmm_narrow_kernel<VT, V, g_>), g, b, 0, stream, C, colptr, crow, cval, scale, X, k, Y); \
+        hipLaunchKernelGGL((spmm_narrow_kernel<VT, V, g_>), g, b, 0, stream, C, colptr, crow, cval, scale, X, k, \
+                           R, Y);                                                                              \
         break
         FD_NARROW(1);
         FD_NARROW(2);
@@ -731,7 +757,7 @@ void launch_narrow(int G, const dim3& g, const dim3& b, hipStream_t stream, uint
 
 template <int VT>
 hipError_t launch_spmm_typed(uint64_t C, const uint64_t* colptr, const uint32_t* crow, const void* cval,
-                             const float* scale, const float* X, int k, float* Y, hipStream_t stream) {
+                             const float* scale, const float* X, int k, uint64_t R, float* Y, hipStream_t stream) {
     const dim3 b(256);
     // beyond 128 vectors a column's lanes are all along them and its entries are wave-uniform
     if (k % 4 == 0 && k > 128) {
@@ -744,20 +770,20 @@ hipError_t launch_spmm_typed(uint64_t C, const uint64_t* colptr, const uint32_t*
     int G = 1;
     while (G < 64 && G * V < k) G *= 2;
     if (V == 4)
-        launch_narrow<VT, 4>(G, g, b, stream, C, colptr, crow, cval, scale, X, k, Y);
+        launch_narrow<VT, 4>(G, g, b, stream, C, colptr, crow, cval, scale, X, k, R, Y);
     else
-        launch_narrow<VT, 1>(G, g, b, stream, C, colptr, crow, cval, scale, X, k, Y);
+        launch_narrow<VT, 1>(G, g, b, stream, C, colptr, crow, cval, scale, X, k, R, Y);
     return hipGetLastError();
 }
 
 }  // namespace
 
 hipError_t launch_spmm(int vtype, uint64_t C, const uint64_t* colptr, const uint32_t* crow, const void* cval,
-                       const float* scale, const float* X, int k, float* Y, hipStream_t stream) {
+                       const float* scale, const float* X, int k, uint64_t R, float* Y, hipStream_t stream) {
     if (C == 0 || k <= 0) return hipSuccess;
-    if (vtype == FD_VAL_F32) return launch_spmm_typed<FD_VAL_F32>(C, colptr, crow, cval, scale, X, k, Y, stream);
-    if (vtype == FD_VAL_BF16) return launch_spmm_typed<FD_VAL_BF16>(C, colptr, crow, cval, scale, X, k, Y, stream);
-    return launch_spmm_typed<FD_VAL_FP16>(C, colptr, crow, cval, scale, X, k, Y, stream);
+    if (vtype == FD_VAL_F32) return launch_spmm_typed<FD_VAL_F32>(C, colptr, crow, cval, scale, X, k, R, Y, stream);
+    if (vtype == FD_VAL_BF16) return launch_spmm_typed<FD_VAL_BF16>(C, colptr, crow, cval, scale, X, k, R, Y, stream);
+    return launch_spmm_typed<FD_VAL_FP16>(C, colptr, crow, cval, scale, X, k, R, Y, stream);
 }
 
 }  // namespace fdi

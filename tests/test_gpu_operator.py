@@ -164,6 +164,23 @@ def test_rows_beyond_one_list(torch_cuda, R, cols):
     assert np.allclose(y[0][:, 0], D, rtol=R * U)
 
 
+@pytest.mark.parametrize("R,cols", [(1, 1), (255, 257), (4096, 1025), (4097, 1025)])
+def test_one_vector_and_16_bit_values(torch_cuda, R, cols):
+    """Up to 4096 rows the products of scales and vector lie in LDS, shared by 1024 columns."""
+    torch = torch_cuda
+    rng = np.random.default_rng([R, cols])
+    mats = [random_rows(rng, R, cols, 4.0 / cols, long_row=True)]
+    x = rng.uniform(-1.0, 1.0, (R, 1)).astype(np.float32)
+    dm = dose_mat(torch, cols, mats)
+    for vtype in (fd.FD_VAL_BF16, fd.FD_VAL_FP16):
+        D = rounded(dense(mats, cols), vtype)
+        with fd.Spmm(dm, vtype) as op:
+            y = op.run(torch.as_tensor(x).cuda()).cpu().numpy()
+        want, mag = D.T @ x.astype(np.float64), np.abs(D).T @ np.abs(x.astype(np.float64))
+        n = (D != 0).sum(0)[:, None]
+        assert np.all(np.abs(y - want) <= (n + 3) * U * mag), vtype
+
+
 @pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 7, 8, 12, 16, 20, 31, 33, 64, 65, 100, 128, 130, 132, 256, 260])
 def test_product_over_lane_arrangements(torch_cuda, k):
     """Sparse, medium and crowded stretches of columns (each picks its own lanes per column, the crowded
