@@ -447,13 +447,39 @@ __device__ __forceinline__ bool pick_dst(uint64_t total, const CsrDst& d0, const
     return false;
 }
 
+// Row offsets, and what the host waits for, written straight into its pinned memory (three or four
+// small copies took about as long as a kernel each) by the compacting kernel, which has at least n
+// workgroups of 256: everything here is known when it starts.
+struct RowOut {
+    const uint32_t* flags;
+    uint64_t* offsets;
+    uint64_t* host_offsets;  // nullable
+    uint64_t* host_totals;
+};
+__device__ __forceinline__ void write_rows(int Z, const uint64_t* __restrict__ cand_off,
+                                           const uint64_t* __restrict__ nnz_off, const RowOut& out) {
+    const uint64_t b = ((uint64_t)blockIdx.y * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x, n = gridDim.y;
+    if (b <= n) {
+        const uint64_t o = nnz_off[b * Z];  // n Z entries, then the total
+        out.offsets[b] = o;
+        if (out.host_offsets) out.host_offsets[b] = o;
+    }
+    if (b == 0) {
+        out.host_totals[0] = cand_off[n * Z];
+        out.host_totals[1] = nnz_off[n * Z];
+        out.host_totals[2] = out.flags[0];
+        out.host_totals[3] = out.flags[2];
+    }
+}
+
 // Ordered copy of the entries that pass the threshold into the CSR arrays.
 __global__ __launch_bounds__(256) void resample_compact_threshold_kernel(
     int Z, const uint64_t* __restrict__ cand_off, const uint64_t* __restrict__ nnz_off,
     const uint32_t* __restrict__ nnz_count, const uint64_t* __restrict__ tmp_cols, const float* __restrict__ tmp_vals,
     const uint32_t* __restrict__ rowmax_bits, float thr, const uint64_t* __restrict__ total, CsrDst dst0,
-    CsrDst dst1) {
+    CsrDst dst1, RowOut out) {
     __shared__ uint32_t s_wave[256 / 64 + 1];
+    write_rows(Z, cand_off, nnz_off, out);
     uint64_t* columns;
     float* values;
     if (!pick_dst(total[0], dst0, dst1, columns, values)) return;
@@ -489,7 +515,8 @@ __global__ __launch_bounds__(256) void resample_compact_kernel(int Z, const uint
                                                                const uint64_t* __restrict__ tmp_cols,
                                                                const float* __restrict__ tmp_vals,
                                                                const uint64_t* __restrict__ total, CsrDst dst0,
-                                                               CsrDst dst1) {
+                                                               CsrDst dst1, RowOut out) {
+    write_rows(Z, cand_off, nnz_off, out);
     uint64_t* columns;
     float* values;
     if (!pick_dst(total[0], dst0, dst1, columns, values)) return;
@@ -518,26 +545,6 @@ __global__ __launch_bounds__(256) void rcp_check_kernel(int exp0, uint32_t* __re
     const float r0 = __builtin_amdgcn_rcpf(b);
     const float r = fmaf(r0, fmaf(-b, r0, 1.0f), r0);
     if (r != 1.0f / b) atomicAdd(mismatches, 1u);
-}
-
-// Row offsets, and what the host waits for, written straight into its pinned memory: three or four
-// small copies after the last kernel took about as long as the kernel itself each.
-__global__ void row_offsets_kernel(int n, int Z, const uint64_t* __restrict__ cand_off,
-                                   const uint64_t* __restrict__ nnz_off, const uint32_t* __restrict__ flags,
-                                   uint64_t* __restrict__ offsets, uint64_t* __restrict__ host_offsets,
-                                   uint64_t* __restrict__ host_totals) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b <= n) {
-        const uint64_t o = nnz_off[(size_t)b * Z];  // b = n: the total
-        offsets[b] = o;
-        if (host_offsets) host_offsets[b] = o;
-    }
-    if (b == 0) {
-        host_totals[0] = cand_off[(size_t)n * Z];
-        host_totals[1] = nnz_off[(size_t)n * Z];
-        host_totals[2] = flags[0];
-        host_totals[3] = flags[2];
-    }
 }
 
 }  // namespace
@@ -591,24 +598,20 @@ hipError_t launch_resample_compact(int n, int Z, const uint64_t* cand_off, const
                                    hipStream_t stream) {
     if (n <= 0) return hipSuccess;
     dim3 grid(Z, n), block(256);
+    const RowOut out{flags, offsets, host_offsets, host_totals};
     const uint64_t* total = nnz_off + (size_t)n * Z;
     if (!dst0.columns || !dst0.values) dst0.capacity = 0;
     if (!dst1.columns || !dst1.values) dst1.capacity = 0;
     if (rowmax_bits && thr > 0.0f) {
         hipLaunchKernelGGL(resample_compact_threshold_kernel, grid, block, 0, stream, Z, cand_off, nnz_off, nnz_count,
-                           tmp_cols, tmp_vals, rowmax_bits, thr, total, dst0, dst1);
+                           tmp_cols, tmp_vals, rowmax_bits, thr, total, dst0, dst1, out);
     } else if ((uint64_t)n * (uint64_t)Z >= kCompactGroupSegments) {
         hipLaunchKernelGGL(resample_compact_kernel<kCompactPlanes>, dim3((Z + kCompactPlanes - 1) / kCompactPlanes, n),
-                           block, 0, stream, Z, cand_off, nnz_off, nnz_count, tmp_cols, tmp_vals, total, dst0, dst1);
+                           block, 0, stream, Z, cand_off, nnz_off, nnz_count, tmp_cols, tmp_vals, total, dst0, dst1, out);
     } else {
         hipLaunchKernelGGL(resample_compact_kernel<1>, grid, block, 0, stream, Z, cand_off, nnz_off, nnz_count,
-                           tmp_cols, tmp_vals, total, dst0, dst1);
+                           tmp_cols, tmp_vals, total, dst0, dst1, out);
     }
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    // nnz_off has n*Z entries followed by the total at index n*Z
-    hipLaunchKernelGGL(row_offsets_kernel, dim3((n + 1 + 255) / 256), dim3(256), 0, stream, n, Z, cand_off, nnz_off,
-                       flags, offsets, host_offsets, host_totals);
     return hipGetLastError();
 }
 
