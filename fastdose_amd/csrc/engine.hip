@@ -233,6 +233,11 @@ uint64_t candidate_estimate(const fd_ctx* ctx, Workspace& w, const fd_beam* beam
     return std::max<uint64_t>((uint64_t)std::ceil(w.cand_per_beamlet * *frustum), 1024);
 }
 
+// Partial CCCS volumes of a batch of n beamlets per BEV value, at least 4: the Terma kernel's scratch.
+static int partial_volumes(const fd_ctx* ctx, int n) {
+    return std::max(cccs_volumes(n, ctx->n_fwd, ctx->cones.n_phi), 4);
+}
+
 size_t batch_footprint(const fd_ctx* ctx, const fd_beam* beams, int n) {
     if (n <= 0) return 0;
     uint64_t bev = 0;  // BEV floats of the batch (packed volumes)
@@ -242,7 +247,7 @@ size_t batch_footprint(const fd_ctx* ctx, const fd_beam* beams, int n) {
         cand += frustum_voxels(beams[i], ctx->vol);
     }
     const size_t segs = (size_t)n * ctx->vol.dim[2];
-    return (size_t)bev * sizeof(float) * (3 + std::max(ctx->n_fwd, 4)) + (size_t)n * kNpix * sizeof(float) +
+    return (size_t)bev * sizeof(float) * (3 + partial_volumes(ctx, n)) + (size_t)n * kNpix * sizeof(float) +
            (size_t)(2.0 * cand) * (2 * sizeof(uint64_t) + 2 * sizeof(float)) + segs * 32 + (size_t)n * 128;
 }
 
@@ -270,7 +275,7 @@ int upload_beams(Workspace& w, const fd_beam* beams, int n, uint64_t stride, hip
     return FD_OK;
 }
 
-int reserve_cccs(const fd_ctx* ctx, Workspace& w, uint64_t bev_floats);
+int reserve_cccs(const fd_ctx* ctx, Workspace& w, int n, uint64_t bev_floats);
 
 int run_terma(const fd_ctx* ctx, Workspace& w, int options, int n, const float* fluence, float* terma, float* dens,
               uint64_t bev_floats, hipStream_t stream) {
@@ -280,7 +285,7 @@ int run_terma(const fd_ctx* ctx, Workspace& w, int options, int n, const float* 
                             : (options & FD_OPT_RPL_FP64) ? kLongRayVoxels * vmin
                                                           : INFINITY;
     // the per-cone partial buffer (4 floats per BEV value at least) is free until the CCCS stage
-    FD_TRY(reserve_cccs(ctx, w, bev_floats));
+    FD_TRY(reserve_cccs(ctx, w, n, bev_floats));
     w.mark(FD_T_TERMA, 0, stream);
     hipError_t e = launch_terma(w.desc.ptr, n, fluence, ctx->density_pad, ctx->vol, ctx->spec_dev, rpl64_len, terma,
                                 dens, w.partial.ptr, ctx->tune.terma_segments, stream);
@@ -292,10 +297,9 @@ int run_terma(const fd_ctx* ctx, Workspace& w, int options, int n, const float* 
     return FD_OK;
 }
 
-// The per-cone partials of a batch whose BEV buffers hold bev_floats floats (n_fwd of them per BEV
-// value, and at least 4: the Terma kernel's scratch).
-int reserve_cccs(const fd_ctx* ctx, Workspace& w, uint64_t bev_floats) {
-    FD_TRY(w.partial.reserve((size_t)bev_floats * std::max(ctx->n_fwd, 4)));
+// The partials of a batch whose BEV buffers hold bev_floats floats.
+int reserve_cccs(const fd_ctx* ctx, Workspace& w, int n, uint64_t bev_floats) {
+    FD_TRY(w.partial.reserve((size_t)bev_floats * partial_volumes(ctx, n)));
     return FD_OK;
 }
 
@@ -313,7 +317,7 @@ int run_cccs_tables(const fd_ctx* ctx, Workspace& w, const CccsTables& tab, hipS
 int run_cccs(const fd_ctx* ctx, Workspace& w, int options, int n, int max_L, const float* terma, const float* dens,
              float* dose, uint64_t bev_floats, hipStream_t stream, const CccsTables* tab, bool tab_built,
              bool vec4) {
-    FD_TRY(reserve_cccs(ctx, w, bev_floats));
+    FD_TRY(reserve_cccs(ctx, w, n, bev_floats));
     if (tab && !tab_built) FD_TRY(run_cccs_tables(ctx, w, *tab, stream));
     hipEvent_t evs[3];
     const bool t = w.timing && w.ev[0];
@@ -583,7 +587,7 @@ int run_batch(const fd_ctx* ctx, Workspace& w, int options, const fd_beam* beams
     FD_TRY(w.out_cols.reserve(cap));
     FD_TRY(w.out_vals.reserve(cap));
 
-    FD_TRY(reserve_cccs(ctx, w, bev));
+    FD_TRY(reserve_cccs(ctx, w, n, bev));
     FD_TRY(reserve_host_rowoff(w, n));
     FD_TRY(plan_tables(ctx, w, options, beams, n));
     FD_TRY(stage_inputs(w, beams, n, 0, w.bev_offs.data(), fluence, overlap));

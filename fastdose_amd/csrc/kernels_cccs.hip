@@ -37,11 +37,11 @@ namespace {
 
 constexpr int kSlots = kRaysPerLane;  // voxels (rows) per lane
 
-// Per-cone partial dose of beamlet B for forward-cone slot t: the beamlet's n_fwd volumes of
-// L x 256 floats start at n_fwd x its BEV offset, so the partial buffer has the BEV layout of the
-// batch scaled by the cone count (n_fwd x the BEV floats of the batch).
-__device__ __forceinline__ float* cone_partial(float* partial, const BeamletDev& B, int n_fwd, int t) {
-    return partial + (uint64_t)B.bev_off * (uint64_t)n_fwd + (uint64_t)t * (uint64_t)B.L * kNpix;
+// Partial volume v of beamlet B's n_vol volumes of L x 256 floats (one per forward cone, more when the
+// widest cone is split, split_volumes): they start at n_vol x its BEV offset, so the partial buffer has
+// the BEV layout of the batch scaled by n_vol (n_vol x the BEV floats of the batch).
+__device__ __forceinline__ float* cone_partial(float* partial, const BeamletDev& B, int n_vol, int v) {
+    return partial + (uint64_t)B.bev_off * (uint64_t)n_vol + (uint64_t)v * (uint64_t)B.L * kNpix;
 }
 
 // Distance to the next voxel boundary along one axis, in units of the direction's parameter
@@ -577,11 +577,12 @@ __host__ __device__ constexpr size_t march_lds_bytes(int n_phi) {
 static_assert(march_lds_bytes(kMaxMarchPhi) <= 65536, "march kernel LDS beyond 64 KiB");
 static_assert(kMaxMarchPhi <= kTabHdr - 2, "a march table chunk header holds every azimuth's count");
 
-__device__ __forceinline__ CcLds carve_lds(float4* base, int n_phi) {
+// n_lanes: azimuths the march wavefront walks (one more than n_phi when it also needs azimuth 0's)
+__device__ __forceinline__ CcLds carve_lds(float4* base, int n_phi, int n_lanes) {
     CcLds S;
     S.rec = base;
     S.pos = base + 2 * n_phi * kRecStride;
-    S.carry = reinterpret_cast<int2*>(S.pos + n_phi * (kRecCap + 1));
+    S.carry = reinterpret_cast<int2*>(S.pos + n_lanes * (kRecCap + 1));
     float* f = reinterpret_cast<float*>(S.carry + 2 * n_phi);
     S.slab = f;
     S.sC = f + 2 * kSlab;
@@ -617,6 +618,8 @@ struct CcBlock {
     const float* Rg;
     float* P;
     int L, wave, n_waves, n_phi;
+    int half;                // SPLIT: which half of the widest cone's azimuths
+    uint32_t volume;         // SPLIT: floats of a partial volume
     float A_a, B_b, na, nb;  // cone constants the slab is scaled with
 };
 
@@ -628,9 +631,16 @@ __device__ __forceinline__ int lds_place(int lane) { return ((lane & 15) << 2) |
 // The slab's eight groups are numbered density 0-3, Terma 4-7; wavefront w loads group w and, when
 // there are fewer than eight wavefronts, group w + n_waves.  So wavefront w < 4, which also combines
 // group w, holds that group's density in a register.  Workgroups with less than four wavefronts load
-// each slab when its slice starts, with all wavefronts.  WIDE: at least eight wavefronts.
-template <bool WIDE>
-__device__ __forceinline__ bool loads_ahead(const CcBlock& K) { return WIDE || K.n_waves >= 4; }
+// each slab when its slice starts, with all wavefronts.
+// kWide: at least eight wavefronts.  kSplit: half of the azimuths of the widest cone, at least four
+// wavefronts; what the combine needs goes to volumes of its own and the cone sum does the rest.
+enum Shape { kNarrow, kWide, kSplit };
+// Partial volumes beyond one per cone when the widest cone is split: a dose for each azimuth of the
+// second half, and the last one's length.
+__host__ __device__ constexpr int split_volumes(int n_phi) { return n_phi / 2 + 1; }
+constexpr uint64_t kSplitGroups = 256;  // most workgroups of a batch with a split cone (cccs_split_kernel)
+template <Shape SHAPE>
+__device__ __forceinline__ bool loads_ahead(const CcBlock& K) { return SHAPE != kNarrow || K.n_waves >= 4; }
 
 // Element lane of a wavefront-uniform address (kept in scalars).
 using GlobalF = __attribute__((address_space(1))) float;
@@ -651,23 +661,27 @@ __device__ __forceinline__ void store_slab(const CcBlock& K, const CcLds& S, int
 struct CcAhead {
     float v0 = 0.0f, v1 = 0.0f;
 };
-template <bool WIDE>
+template <Shape SHAPE>
 __device__ __forceinline__ void slab_regs(const CcBlock& K, int z, CcAhead& A) {
     if (K.wave < 8) A.v0 = slab_value(K, z, K.wave);
-    if (!WIDE && K.wave + K.n_waves < 8) A.v1 = slab_value(K, z, K.wave + K.n_waves);
+    if (SHAPE != kWide && K.wave + K.n_waves < 8) A.v1 = slab_value(K, z, K.wave + K.n_waves);
 }
-template <bool WIDE>
+template <Shape SHAPE>
 __device__ __forceinline__ void store_ahead(const CcBlock& K, const CcLds& S, int si, const CcAhead& A) {
     if (K.wave < 8) store_slab(K, S, si, K.wave, A.v0);
-    if (!WIDE && K.wave + K.n_waves < 8) store_slab(K, S, si, K.wave + K.n_waves, A.v1);
+    if (SHAPE != kWide && K.wave + K.n_waves < 8) store_slab(K, S, si, K.wave + K.n_waves, A.v1);
 }
 // The whole slab of slice z, ordinal si, by all wavefronts.
 __device__ __forceinline__ void load_slab(const CcBlock& K, const CcLds& S, int z, int si) {
     for (int q = K.wave; q < 8; q += K.n_waves) store_slab(K, S, si, q, slab_value(K, z, q));
 }
+template <Shape SHAPE>
 __device__ __forceinline__ void zero_slice(const CcBlock& K, int z) {
+    const int volumes = SHAPE == kSplit && K.half ? K.n_phi + 1 : 1;
     for (int q = K.wave; q < 4; q += K.n_waves)
-        uniform_base(K.P, (uint32_t)z * kNpix + (uint32_t)(q * kWave))[threadIdx.x & 63] = 0.0f;
+        for (int v = 0; v < volumes; v++)
+            uniform_base(K.P, (uint32_t)v * K.volume + (uint32_t)z * kNpix + (uint32_t)(q * kWave))[threadIdx.x & 63] =
+                0.0f;
 }
 
 // Where the march stands, in every wavefront alike.
@@ -675,11 +689,17 @@ struct CcSlice {
     int s = 0, si = 0, written = 0;  // slice being processed, its ordinal, slices written so far
     float rho = 0.0f;                // density of this wavefront's group of the slice (loads_ahead, wave < 4)
 };
-template <bool WIDE>
+template <Shape SHAPE>
 __device__ __forceinline__ CcSlice first_slice(const CcBlock& K) {
     CcSlice Z;
-    if (loads_ahead<WIDE>(K) && K.wave < 4) Z.rho = slab_value(K, 0, K.wave);
+    if (loads_ahead<SHAPE>(K) && K.wave < 4) Z.rho = slab_value(K, 0, K.wave);
     return Z;
+}
+
+// A slice's dose: rho times the dose in units of geometric length, summed over the azimuths, over (rho
+// times the cumulative length of the last azimuth + 1e-4), the quotient from the hardware reciprocal.
+__device__ __forceinline__ float slice_dose(float sum, float rho, float length) {
+    return sum * rho * __builtin_amdgcn_rcpf(fmaf(length, rho, kEps));
 }
 
 // End of a chunk, executed by every wavefront: store the prefetched slab, barrier, and after a
@@ -689,23 +709,28 @@ __device__ __forceinline__ CcSlice first_slice(const CcBlock& K) {
 // Runs once per slice and wavefront, against 1.5 to 12 lattice steps of about 60 vector instructions,
 // and a full GPU is bound by instructions issued and fetched (vector units over 95 % busy, 0.77
 // instruction cache fetches per cycle and CU pair): wavefront-uniform conditions and addresses are
-// kept in scalars, the common workgroup (WIDE) has no loops over groups, a lane's four voxels are one
+// kept in scalars, the common workgroup (kWide) has no loops over groups, a lane's four voxels are one
 // LDS access and the combine's density is a register.  Together with the step's X kept in place:
 // cccs_tab_kernel in a 20-beam plan 14.2 -> 13.6 ms, 400 beamlets of cccs_kernel 3.91 -> 3.60 ms,
 // 121 beamlets (one workgroup per CU and a half, latency) 1.20 -> 1.16 ms.
-template <bool WIDE>
+template <Shape SHAPE>
 __device__ __forceinline__ bool chunk_end(const CcBlock& K, const CcLds& S, int done, int sn, const CcAhead& A,
                                           CcSlice& Z, bool dma = false) {
-    if (done && sn < K.L && loads_ahead<WIDE>(K)) store_ahead<WIDE>(K, S, Z.si + 1, A);
+    if (done && sn < K.L && loads_ahead<SHAPE>(K)) store_ahead<SHAPE>(K, S, Z.si + 1, A);
     if (dma) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (!done) return true;
-    // slice s: rho sum over azimuths (in azimuth order) of the dose in units of geometric length /
-    // (rho cumulative length of the last azimuth + 1e-4); the quotient from the hardware reciprocal
+    // slice s: slice_dose of the sum over azimuths, in their order
     const int lane = threadIdx.x & 63;
     for (int q = K.wave; q < 4; q += K.n_waves) {
         const int i = q * kWave + lds_place(lane);
         const float* d = S.sD + (Z.si & 1) * K.n_phi * kNpix + i;
+        auto to = [&] { return (uint32_t)Z.s * kNpix + (uint32_t)(q * kWave); };
+        if (SHAPE == kSplit && K.half) {  // the later azimuths' doses and the last one's length
+            for (int f = 0; f < K.n_phi; f++) uniform_base(K.P, (uint32_t)f * K.volume + to())[lane] = d[f * kNpix];
+            uniform_base(K.P, (uint32_t)K.n_phi * K.volume + to())[lane] = S.sC[(Z.si & 1) * kNpix + i];
+            continue;
+        }
         float sum = 0.0f;
         int f = 0;
         for (; f + 4 <= K.n_phi; f += 4) {  // four reads in flight, summed in azimuth order
@@ -713,15 +738,18 @@ __device__ __forceinline__ bool chunk_end(const CcBlock& K, const CcLds& S, int 
             sum = (((sum + v0) + v1) + v2) + v3;
         }
         for (; f < K.n_phi; f++) sum += d[f * kNpix];
-        const float rho = loads_ahead<WIDE>(K) ? Z.rho : slab_value(K, Z.s, q);
-        uniform_base(K.P, (uint32_t)Z.s * kNpix + (uint32_t)(q * kWave))[lane] =
-            sum * rho * __builtin_amdgcn_rcpf(fmaf(S.sC[(Z.si & 1) * kNpix + i], rho, kEps));
-        if (WIDE) break;
+        if (SHAPE == kSplit) {  // the sum of the earlier azimuths
+            uniform_base(K.P, to())[lane] = sum;
+            continue;
+        }
+        const float rho = loads_ahead<SHAPE>(K) ? Z.rho : slab_value(K, Z.s, q);
+        uniform_base(K.P, to())[lane] = slice_dose(sum, rho, S.sC[(Z.si & 1) * kNpix + i]);
+        if (SHAPE == kWide) break;
     }
-    for (int z = Z.s + 1; z < sn && z < K.L; z++) zero_slice(K, z);  // slices the phi-0 march stepped over
+    for (int z = Z.s + 1; z < sn && z < K.L; z++) zero_slice<SHAPE>(K, z);  // slices the phi-0 march stepped over
     Z.written = sn < K.L ? sn : K.L;
     if (sn >= K.L) return false;
-    if (!loads_ahead<WIDE>(K)) {  // small workgroups load the next slab here
+    if (!loads_ahead<SHAPE>(K)) {  // small workgroups load the next slab here
         __syncthreads();
         load_slab(K, S, sn, Z.si + 1);
         __syncthreads();
@@ -732,8 +760,9 @@ __device__ __forceinline__ bool chunk_end(const CcBlock& K, const CcLds& S, int 
     return true;
 }
 
+template <Shape SHAPE>
 __device__ __forceinline__ void zero_tail(const CcBlock& K, int written) {
-    for (int z = written; z < K.L; z++) zero_slice(K, z);
+    for (int z = written; z < K.L; z++) zero_slice<SHAPE>(K, z);
 }
 
 // March wavefront, in two phases per chunk.  Phase 1: lane f < n_phi marches azimuth f with the
@@ -751,6 +780,7 @@ struct MarchLane {
 struct MarchConst {
     float bsx, bsy, ls, lim_min, inv_sad;
     int lane, kper, lf, lk;  // phase 2: lane -> azimuth lf, step lk of each group of kper steps
+    int lanes, lead;         // phase 1: lanes that march (n_phi, or one more), the one with azimuth 0
 };
 
 // Where phase 2 puts a chunk's records: the march kernel's LDS records (TABLE false), or a march
@@ -768,7 +798,7 @@ __device__ __forceinline__ bool march_chunk(MarchLane& M, const MarchConst& C, i
                                             const TabOut& T = TabOut{}) {
     const int lane = C.lane;
     if (new_slice) {
-        M.act = lane < n_phi;
+        M.act = lane < C.lanes;
         M.nsteps = 0;
     }
     // phase 1: lattice points; pos[f][0] is where the chunk starts.  A serial chain of FP32 steps per
@@ -776,7 +806,7 @@ __device__ __forceinline__ bool march_chunk(MarchLane& M, const MarchConst& C, i
     // branch on the slice end (both candidates are computed, lanes that have reached theirs keep
     // their position and write past their last point, which nothing reads), two steps per test.
     int cnt = 0, k = 0;
-    if (lane < n_phi) {
+    if (lane < C.lanes) {
         float4* mypos = S.pos + lane * (kRecCap + 1);
         mypos[0] = make_float4(M.bxp, M.byp, M.bzp, 0.0f);
         auto step = [&](int at) {
@@ -811,7 +841,7 @@ __device__ __forceinline__ bool march_chunk(MarchLane& M, const MarchConst& C, i
     k = __builtin_amdgcn_readfirstlane(k);
     const bool done = __ballot(M.act) == 0;
     if (lane < n_phi) hdr[lane] = cnt;
-    if (lane == 0) {
+    if (lane == C.lead) {
         hdr[kMaxPhi] = done ? 1 : 0;
         hdr[kMaxPhi + 1] = max((int)rintf(M.bzp), s_cur + 1);  // the phi-0 march decides the next slice
     }
@@ -922,9 +952,9 @@ __device__ __forceinline__ bool march_chunk(MarchLane& M, const MarchConst& C, i
 // March state of this lane (azimuth lane, if below n_phi) at the start of the walk of cone t, for a
 // beamlet with BEV pitch (bs0, bs1) and longitudinal spacing ls; phase-2 lane assignment.
 __device__ __forceinline__ void march_init(MarchLane& M, MarchConst& C, const ConeTable* __restrict__ cones, int t,
-                                           int n_phi, float bs0, float bs1, float ls) {
+                                           int n_phi, float bs0, float bs1, float ls, int first = 0) {
     const int lane = threadIdx.x & 63;
-    const int f = lane < n_phi ? lane : 0;
+    const int f = lane < n_phi ? first + lane : 0;  // lane n_phi: azimuth 0, which decides the slices
     {
         // grid direction of (theta, phi_f): unit vector scaled to voxel units, renormalised
         const float ux = cones->ux[t][f], uy = cones->uy[t][f], uz = cones->uz[t][f];
@@ -949,18 +979,20 @@ __device__ __forceinline__ void march_init(MarchLane& M, MarchConst& C, const Co
     C.bsy = uniform(bs1);
     C.ls = uniform(ls);
     C.lane = lane;
+    C.lead = first ? n_phi : 0;
+    C.lanes = n_phi + (first ? 1 : 0);
     C.kper = 64 / n_phi;
     C.lk = lane / n_phi;
     C.lf = C.lk < C.kper ? lane - C.lk * n_phi : n_phi;  // n_phi: idle in phase 2
 }
 
-template <bool WIDE>
+template <Shape SHAPE>
 __device__ __forceinline__ void cccs_march(const BeamletDev& B, const ConeTable* __restrict__ cones, int t,
                                            const CcBlock& K, const CcLds& S) {
     const int lane = threadIdx.x & 63;
     MarchLane M;
     MarchConst C;
-    march_init(M, C, cones, t, K.n_phi, B.bs[0], B.bs[1], B.ls);
+    march_init(M, C, cones, t, K.n_phi, B.bs[0], B.bs[1], B.ls, SHAPE == kSplit && K.half ? K.n_phi : 0);
     C.inv_sad = uniform(1.0f / B.sad);
     C.lim_min = uniform(B.lim_min);
     if (lane < K.n_phi) S.carry[lane] = make_int2(0, 0);  // the midpoint voxel starts at (0, 0)
@@ -968,19 +1000,19 @@ __device__ __forceinline__ void cccs_march(const BeamletDev& B, const ConeTable*
 
     march_chunk<false>(M, C, K.n_phi, S, S.rec, S.hdr, 0, true);
     __syncthreads();
-    CcSlice Z = first_slice<WIDE>(K);
+    CcSlice Z = first_slice<SHAPE>(K);
     int buf = 0;
     for (;;) {
         const int done = S.hdr[buf * kHdr + kMaxPhi], sn = S.hdr[buf * kHdr + kMaxPhi + 1];
         CcAhead ahead;
-        if (done && sn < K.L && loads_ahead<WIDE>(K)) slab_regs<WIDE>(K, sn, ahead);
+        if (done && sn < K.L && loads_ahead<SHAPE>(K)) slab_regs<SHAPE>(K, sn, ahead);
         if (!(done && sn >= K.L))
             march_chunk<false>(M, C, n_phi, S, S.rec + (buf ^ 1) * n_phi * kRecStride, S.hdr + (buf ^ 1) * kHdr,
                                done ? sn : Z.s, done != 0);
-        if (!chunk_end<WIDE>(K, S, done, sn, ahead, Z)) break;
+        if (!chunk_end<SHAPE>(K, S, done, sn, ahead, Z)) break;
         buf ^= 1;
     }
-    zero_tail(K, Z.written);
+    zero_tail<SHAPE>(K, Z.written);
 }
 
 // March tables: one wavefront per (march geometry, forward cone) walks the lattice of every azimuth
@@ -1092,7 +1124,7 @@ static_assert(2 * kRecCap == kWave, "a table block is one 16-byte load per lane"
 // X states are kept pre-scaled by A/a and B/b, and the dose and cumulative length are summed in
 // units of the geometric length s (p = s rho), multiplied by rho in the combine.  TAB: the chunks
 // come from a march table (cccs_tab_kernel), else from the march wavefront's LDS records.
-template <bool EXACT_G, bool WIDE, bool CUMU, bool TAB, bool FEW>
+template <bool EXACT_G, Shape SHAPE, bool CUMU, bool TAB, bool FEW>
 __device__ __forceinline__ void cccs_compute(const CcBlock& K, const CcLds& S, int wave,
                                              const TabRead& TR = TabRead{}) {
     const int lane = threadIdx.x & 63;
@@ -1123,7 +1155,7 @@ __device__ __forceinline__ void cccs_compute(const CcBlock& K, const CcLds& S, i
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
     __syncthreads();  // chunk 0's header, block 0 and slab 0 are in LDS
-    CcSlice Z = first_slice<WIDE>(K);
+    CcSlice Z = first_slice<SHAPE>(K);
     int buf = 0;
     // TAB: chunk, stream position after the previous chunk, block finished last (-1: none)
     uint32_t tc = 0, tofs = 0;
@@ -1177,7 +1209,7 @@ __device__ __forceinline__ void cccs_compute(const CcBlock& K, const CcLds& S, i
             rp = S.rec + (buf * n_phi + wave) * kRecStride;
         }
         CcAhead ahead;
-        if (done && sn < K.L && loads_ahead<WIDE>(K)) slab_regs<WIDE>(K, sn, ahead);
+        if (done && sn < K.L && loads_ahead<SHAPE>(K)) slab_regs<SHAPE>(K, sn, ahead);
         if (fresh) {
             const float4* slab = reinterpret_cast<const float4*>(S.slab + (Z.si & 1) * kSlab) + lane;
             const float4 ta = slab[0], tb = slab[kWave], ra = slab[2 * kWave], rb = slab[3 * kWave];
@@ -1198,10 +1230,12 @@ __device__ __forceinline__ void cccs_compute(const CcBlock& K, const CcLds& S, i
             const int ddx = ((int)(w << 27)) >> 27;
             const int ddy = ((int)(w << 22)) >> 27;
             // steps with no shift of the midpoint voxel (and with no reset below) skip the decision
-            // trees with one scalar test each
-            if (w & kShiftBits) {
+            // trees with one scalar test each.  The weights keep the rare shifts and resets out of line: a
+            // wavefront alone on its SIMD pays for every jump (3 % of a small batch's time; FEW only, with more
+            // wavefronts to a SIMD they gain nothing).
+            if (FEW ? __builtin_expect((w & kShiftBits) != 0, 1) : (w & kShiftBits) != 0) {
                 // rotate the X state (and my rays' x offsets) to follow the midpoint voxel
-                if (w & kUnitX) {
+                if (FEW ? __builtin_expect((w & kUnitX) != 0, 1) : (w & kUnitX) != 0) {
                     if (w & 0x10u) {  // ddx = -1
                         if (apart(w) & kZeroFillX) {  // with the previous step's reset of column 0
 #pragma unroll
@@ -1233,11 +1267,11 @@ __device__ __forceinline__ void cccs_compute(const CcBlock& K, const CcLds& S, i
                         }
                         fix = row_from_left(fix);
                     }
-                } else if (w & 0x1Fu) {
+                } else if (FEW ? __builtin_expect((w & 0x1Fu) != 0, 0) : (w & 0x1Fu) != 0) {
                     shift_x(XA, XB, ddx);
                     fix = (float)((vx - (int)((w >> 10) & 15)) & 15);
                 }
-                if (w & kUnitY) {
+                if (FEW ? __builtin_expect((w & kUnitY) != 0, 1) : (w & kUnitY) != 0) {
                     if (w & 0x200u) {  // ddy = -1
                         const float ta = wave_from(XA[0], down_lane);
                         const float tb = wave_from(XB[0], down_lane);
@@ -1253,7 +1287,7 @@ __device__ __forceinline__ void cccs_compute(const CcBlock& K, const CcLds& S, i
                         slots_down(XB, tb);
                         slots_down(fiy, tz);
                     }
-                } else if (w & 0x3E0u) {
+                } else if (FEW ? __builtin_expect((w & 0x3E0u) != 0, 0) : (w & 0x3E0u) != 0) {
                     shift_y3(XA, XB, fiy, ddy, up_lane, down_lane);
                 }
             }
@@ -1306,7 +1340,7 @@ __device__ __forceinline__ void cccs_compute(const CcBlock& K, const CcLds& S, i
                             XB[r] = m ? 0.0f : XB[r];
                         }
                 }
-                if (w & kGeneralReset) {
+                if (FEW ? __builtin_expect((w & kGeneralReset) != 0, 0) : (w & kGeneralReset) != 0) {
                     const int mx = (int)((w >> 10) & 15), my = (int)((w >> 14) & 15);
                     const float2 gw = rp2[4 * k + 3];
                     const int gxw = __builtin_amdgcn_readfirstlane(__float_as_int(gw.x));
@@ -1363,11 +1397,11 @@ __device__ __forceinline__ void cccs_compute(const CcBlock& K, const CcLds& S, i
             if (CUMU)
                 reinterpret_cast<float4*>(S.sC + (Z.si & 1) * kNpix)[lane] = make_float4(Cs[0], Cs[1], Cs[2], Cs[3]);
         }
-        if (!chunk_end<WIDE>(K, S, done, sn, ahead, Z, TAB)) break;
+        if (!chunk_end<SHAPE>(K, S, done, sn, ahead, Z, TAB)) break;
         fresh = done != 0;
         buf ^= 1;
     }
-    zero_tail(K, Z.written);
+    zero_tail<SHAPE>(K, Z.written);
 }
 
 // 72 VGPRs (7 wavefronts per SIMD) and 47.0 KiB of LDS fit three workgroups of 9 wavefronts on a CU
@@ -1375,7 +1409,7 @@ __device__ __forceinline__ void cccs_compute(const CcBlock& K, const CcLds& S, i
 // FEW: at most two workgroups per CU, where a slice takes as long as its slowest wavefront's serial
 // chain: up to 96 VGPRs, and the wavefronts of a SIMD take turns (cccs_compute).  16 beamlets of a slab
 // beam (64 workgroups) 476 -> 459 us, 121 (484) 1157 -> 1115; with 196 (784) the turns cost 2 %.
-template <bool EXACT_G, bool WIDE, bool FEW>
+template <bool EXACT_G, Shape SHAPE, bool FEW>
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(FEW ? 5 : 7, 8))) void cccs_kernel(
     const BeamletDev* __restrict__ beams, int n, const ConeTable* __restrict__ cones, int n_fwd,
     const float* __restrict__ terma, const float* __restrict__ dens_bev, float* __restrict__ partial) {
@@ -1393,7 +1427,7 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(FEW ? 5 : 
     K.Tg = terma + B.bev_off;
     K.Rg = dens_bev + B.bev_off;
     K.P = cone_partial(partial, B, n_fwd, t);
-    const CcLds S = carve_lds(lds4, K.n_phi);
+    const CcLds S = carve_lds(lds4, K.n_phi, K.n_phi);
 
     K.A_a = cones->A_a[t];
     K.B_b = cones->B_b[t];
@@ -1401,17 +1435,17 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(FEW ? 5 : 
     K.nb = cones->nb[t];
     load_slab(K, S, 0, 0);
     if (wave == K.n_phi)
-        cccs_march<WIDE>(B, cones, t, K, S);
+        cccs_march<SHAPE>(B, cones, t, K, S);
     else if (wave == K.n_phi - 1)
-        cccs_compute<EXACT_G, WIDE, true, false, FEW>(K, S, wave);
+        cccs_compute<EXACT_G, SHAPE, true, false, FEW>(K, S, wave);
     else
-        cccs_compute<EXACT_G, WIDE, false, false, FEW>(K, S, wave);
+        cccs_compute<EXACT_G, SHAPE, false, false, FEW>(K, S, wave);
 }
 
 // cccs_kernel without the march wavefront: the workgroup's n_phi compute wavefronts read their
 // chunks from the march table of the beamlet's geometry (cccs_table_kernel) and finish the
 // records with the beamlet's lim_min and sad themselves.  Same arithmetic, same results.
-template <bool EXACT_G, bool WIDE>
+template <bool EXACT_G, Shape SHAPE>
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(6, 8))) void cccs_tab_kernel(
     const BeamletDev* __restrict__ beams, int n, const ConeTable* __restrict__ cones, int n_fwd,
     const float* __restrict__ terma, const float* __restrict__ dens_bev, float* __restrict__ partial,
@@ -1450,9 +1484,9 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(6, 8))) vo
     TR.ls = B.ls;
     load_slab(K, S, 0, 0);
     if (wave == K.n_phi - 1)
-        cccs_compute<EXACT_G, WIDE, true, true, false>(K, S, wave, TR);
+        cccs_compute<EXACT_G, SHAPE, true, true, false>(K, S, wave, TR);
     else
-        cccs_compute<EXACT_G, WIDE, false, true, false>(K, S, wave, TR);
+        cccs_compute<EXACT_G, SHAPE, false, true, false>(K, S, wave, TR);
 }
 
 // dose[b][s][p] = sum over forward cones of partial[b][t][s][p], cone slots in order.
@@ -1492,7 +1526,93 @@ __global__ __launch_bounds__(256) void cone_sum4_kernel(const BeamletDev* __rest
     reinterpret_cast<float4*>(dose + B.bev_off)[i] = acc;
 }
 
+// cccs_kernel for the smallest batches, with the widest cone's azimuths in two workgroups per beamlet
+// (workgroups 0 ... 2 n - 1, the first half of the azimuths even): its segments are 60 % of a beamlet's,
+// so its workgroup sets the time when every workgroup has a CU to itself, and with half the azimuths no
+// two compute wavefronts share a SIMD and the march takes one pass per slice for its records.  The
+// second half's march also walks azimuth 0, which decides the slices.  Wavefronts a half does not
+// need end at once.  The sums are finished by cone_sum_split_kernel, in azimuth order: same bits.
+// 4 beamlets of a slab beam 371 -> 354 us, 16 beamlets 460 -> 438.  64 (320 workgroups) would gain 2 % and
+// pay for it with a partial buffer of more than twice the size; with 196 it would cost 36 %.  What is
+// left is one wavefront's serial chain of 650 to 750 cycles per lattice step.
+template <bool EXACT_G>
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 8))) void cccs_split_kernel(
+    const BeamletDev* __restrict__ beams, int n, const ConeTable* __restrict__ cones, int n_fwd,
+    const float* __restrict__ terma, const float* __restrict__ dens_bev, float* __restrict__ partial) {
+    extern __shared__ float4 lds4[];
+    const int n_phi = cones->n_phi, n_half = n_phi / 2, n_vol = n_fwd + split_volumes(n_phi);
+    const bool whole = (int)blockIdx.x >= 2 * n;
+    const int t = whole ? 1 + ((int)blockIdx.x - 2 * n) / n : 0;
+    const int b = whole ? ((int)blockIdx.x - 2 * n) % n : (int)blockIdx.x >> 1;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const BeamletDev& B = beams[b];
+    CcBlock K;
+    K.L = B.L;
+    if (K.L <= 0) return;
+    K.half = whole ? 0 : (int)blockIdx.x & 1;
+    K.wave = wave;
+    K.n_phi = whole ? n_phi : n_half;
+    K.n_waves = K.n_phi + 1;
+    if (wave >= K.n_waves) return;
+    K.Tg = terma + B.bev_off;
+    K.Rg = dens_bev + B.bev_off;
+    K.volume = (uint32_t)B.L * kNpix;
+    K.P = cone_partial(partial, B, n_vol, whole ? n_half + 1 + t : K.half);
+    K.A_a = cones->A_a[t];
+    K.B_b = cones->B_b[t];
+    K.na = cones->na[t];
+    K.nb = cones->nb[t];
+    const CcLds S = carve_lds(lds4, K.n_phi, K.n_phi + K.half);
+    load_slab(K, S, 0, 0);
+    const bool last = wave == K.n_phi - 1;
+    if (whole) {
+        if (wave == K.n_phi)
+            cccs_march<kWide>(B, cones, t, K, S);
+        else if (last)
+            cccs_compute<EXACT_G, kWide, true, false, true>(K, S, wave);
+        else
+            cccs_compute<EXACT_G, kWide, false, false, true>(K, S, wave);
+    } else {
+        if (wave == K.n_phi)
+            cccs_march<kSplit>(B, cones, t, K, S);
+        else if (last)
+            cccs_compute<EXACT_G, kSplit, true, false, true>(K, S, wave);
+        else
+            cccs_compute<EXACT_G, kSplit, false, false, true>(K, S, wave);
+    }
+}
+
+// cone_sum_kernel after cccs_split_kernel: the widest cone's dose first, from the sum of its earlier
+// azimuths, the doses of the later ones and the last one's length.
+__global__ __launch_bounds__(256) void cone_sum_split_kernel(const BeamletDev* __restrict__ beams,
+                                                             const ConeTable* __restrict__ cones, int n_fwd,
+                                                             const float* __restrict__ partial,
+                                                             const float* __restrict__ dens_bev,
+                                                             float* __restrict__ dose) {
+    const BeamletDev& B = beams[blockIdx.y];
+    const int n_half = cones->n_phi / 2;
+    const uint64_t count = (uint64_t)B.L * kNpix;
+    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= count) return;
+    const float* src = partial + (uint64_t)B.bev_off * (uint64_t)(n_fwd + split_volumes(cones->n_phi)) + i;
+    float sum = src[0];
+    for (int f = 1; f <= n_half; f++) sum += src[(uint64_t)f * count];
+    src += (uint64_t)(n_half + 1) * count;
+    float acc = 0.0f;
+    acc += slice_dose(sum, dens_bev[B.bev_off + i], src[0]);
+    for (int t = 1; t < n_fwd; t++) acc += src[(uint64_t)t * count];
+    dose[B.bev_off + i] = acc;
+}
+
 }  // namespace
+
+int cccs_volumes(int n, int n_fwd, int n_phi) {
+    // an even number of azimuths, at least eight wavefronts in the other cones' workgroups (kWide), a CU
+    // for each workgroup
+    const bool split = n_phi % 2 == 0 && n_phi >= 8 && n_phi <= kMaxMarchPhi && n_fwd > 0 &&
+                       (uint64_t)n * (uint64_t)(n_fwd + 1) <= kSplitGroups;
+    return n_fwd + (split ? split_volumes(n_phi) : 0);
+}
 
 int cccs_table_max_phi() { return kMaxMarchPhi; }
 int cccs_chunk_steps() { return kRecCap; }
@@ -1512,12 +1632,20 @@ hipError_t launch_cccs(const BeamletDev* beams, int n, int max_L, const ConeTabl
                        float* dose, bool vec4, hipStream_t stream, hipEvent_t* ev, const CccsTables* tab) {
     if (n <= 0) return hipSuccess;
     if (ev) (void)hipEventRecord(ev[0], stream);
-    if (n_fwd > 0 && tab && n_phi <= kMaxMarchPhi) {
+    const bool split = !tab && cccs_volumes(n, n_fwd, n_phi) > n_fwd;
+    if (split) {
+        const dim3 grid((unsigned)(n * (n_fwd + 1))), block((n_phi + 1) * kWave);
+        const auto kernel = exact_g ? cccs_split_kernel<true> : cccs_split_kernel<false>;
+        hipLaunchKernelGGL(kernel, grid, block, march_lds_bytes(n_phi), stream, beams, n, cones_dev, n_fwd, terma,
+                           dens_bev, partial);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    } else if (n_fwd > 0 && tab && n_phi <= kMaxMarchPhi) {
         // compute wavefronts only, reading their chunks from the tables
         const dim3 grid((unsigned)(n * n_fwd)), block(n_phi * kWave);
         const size_t shm = tab_lds_bytes(n_phi);
-        const auto kernel = n_phi >= 8 ? (exact_g ? cccs_tab_kernel<true, true> : cccs_tab_kernel<false, true>)
-                                       : (exact_g ? cccs_tab_kernel<true, false> : cccs_tab_kernel<false, false>);
+        const auto kernel = n_phi >= 8 ? (exact_g ? cccs_tab_kernel<true, kWide> : cccs_tab_kernel<false, kWide>)
+                                       : (exact_g ? cccs_tab_kernel<true, kNarrow> : cccs_tab_kernel<false, kNarrow>);
         hipLaunchKernelGGL(kernel, grid, block, shm, stream, beams, n, cones_dev, n_fwd, terma, dens_bev, partial,
                            tab->ent, tab->rec, tab->hdr);
         hipError_t e = hipGetLastError();
@@ -1530,9 +1658,9 @@ hipError_t launch_cccs(const BeamletDev* beams, int n, int max_L, const ConeTabl
             const size_t shm = march_lds_bytes(n_phi);
             const bool few = grid.x <= kFewGroups;
             const auto kernel =
-                n_phi + 1 < 8 ? (exact_g ? cccs_kernel<true, false, false> : cccs_kernel<false, false, false>)
-                : few         ? (exact_g ? cccs_kernel<true, true, true> : cccs_kernel<false, true, true>)
-                              : (exact_g ? cccs_kernel<true, true, false> : cccs_kernel<false, true, false>);
+                n_phi + 1 < 8 ? (exact_g ? cccs_kernel<true, kNarrow, false> : cccs_kernel<false, kNarrow, false>)
+                : few         ? (exact_g ? cccs_kernel<true, kWide, true> : cccs_kernel<false, kWide, true>)
+                              : (exact_g ? cccs_kernel<true, kWide, false> : cccs_kernel<false, kWide, false>);
             hipLaunchKernelGGL(kernel, grid, block, shm, stream, beams, n, cones_dev, n_fwd, terma, dens_bev, partial);
         } else {
             // one azimuth per wavefront up to 16 azimuths (1024 threads), two beyond
@@ -1560,7 +1688,10 @@ hipError_t launch_cccs(const BeamletDev* beams, int n, int max_L, const ConeTabl
         if (e != hipSuccess) return e;
     }
     if (ev) (void)hipEventRecord(ev[1], stream);
-    if (vec4 && reinterpret_cast<uintptr_t>(dose) % 16 == 0 && reinterpret_cast<uintptr_t>(partial) % 16 == 0) {
+    if (split) {
+        dim3 g2((unsigned)(((uint64_t)max_L * kNpix + 255) / 256), (unsigned)n), b2(256);
+        hipLaunchKernelGGL(cone_sum_split_kernel, g2, b2, 0, stream, beams, cones_dev, n_fwd, partial, dens_bev, dose);
+    } else if (vec4 && reinterpret_cast<uintptr_t>(dose) % 16 == 0 && reinterpret_cast<uintptr_t>(partial) % 16 == 0) {
         dim3 g2((unsigned)(((uint64_t)max_L * (kNpix / 4) + 255) / 256), (unsigned)n), b2(256);
         hipLaunchKernelGGL(cone_sum4_kernel, g2, b2, 0, stream, beams, n_fwd, partial, dose);
     } else {

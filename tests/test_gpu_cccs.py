@@ -48,6 +48,32 @@ def test_workgroup_sizes(torch_cuda, n_phi, exact_g):
     assert same_matrix(mats[0].matrix(0), mats[1].matrix(0))
 
 
+@pytest.mark.parametrize("n_phi", [8, 10])
+@pytest.mark.parametrize("exact_g", [False, True])
+def test_split_widest_cone(torch_cuda, n_phi, exact_g):
+    """Up to 51 beamlets (four forward cones: 255 workgroups) the widest cone's azimuths take two workgroups
+    each; 56 beamlets in one call (no split) and in calls of 51, 4 and 1 (all split): the same bits, also
+    with a slice spacing at which the march of azimuth 0 skips slices and others take several chunks."""
+    cfg = synth.small_config(seed=95 + n_phi, dim=(30, 26, 28), fluence_dim=8, angles=(20.0, 15.0, 0.0))
+    cfg.kernel = synth.synthetic_kernel(1095, n_phi=n_phi)
+    all_beams, flu = beamlets_of(cfg)
+    for spacing in (1.0, 6.0, 0.2):
+        beams = fd.beam_array(list(all_beams)[:56])
+        for b in beams:
+            b.long_spacing *= spacing
+            b.long_dim = max(1, int(np.ceil(b.long_dim / spacing)))
+        log(f"split cone, {n_phi} azimuths, exact_g={exact_g}, slice spacing x {spacing}")
+        options = fd.FD_OPT_EXACT_G if exact_g else 0
+        with fd.Context(cfg.volume, cfg.density, cfg.spectrum, cfg.kernel, options=options) as ctx:
+            dose = gpu_stages(ctx, beams, flu[:56], cfg.extent)["dose"]
+            k = 0
+            for a, b in ((0, 51), (51, 55), (55, 56)):
+                for d in gpu_stages(ctx, fd.beam_array(beams[a:b]), flu[a:b], cfg.extent)["dose"]:
+                    L = beams[k].long_dim
+                    assert np.array_equal(d[:L], dose[k, :L]) and d[:L].max() > 0
+                    k += 1
+
+
 def test_few_and_many_workgroups(torch_cuda):
     """144 beamlets (four forward cones: 576 workgroups) in one call and in calls of 128 and 16: the
     instances for few and for many workgroups, the first at its largest."""
