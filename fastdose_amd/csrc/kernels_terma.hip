@@ -14,7 +14,7 @@
 // share cache lines.
 //
 // It is bound by vector instructions on small batches (1.0 issued per CU and cycle at 256 beamlets of
-// 175 slices) and by the record reads on large ones (the data path of vector memory 99 % busy in a
+// 137 slices) and by the record reads on large ones (the data path of vector memory 99 % busy in a
 // 20-beam plan: a read is issued for nearly every sample, since some lane of the wavefront changes its
 // base voxel).  So a sample has few instructions: base voxel and fraction are one conversion and one
 // v_fract per axis, the record offset is two 24-bit multiply-adds and three bit selects.  45.4 -> 37.2 M
