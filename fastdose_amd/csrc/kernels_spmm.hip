@@ -11,6 +11,7 @@
 //     entries and columns according to k and the columns' lengths.
 #include <hip/hip_runtime.h>
 
+#include <cfloat>
 #include <type_traits>
 
 #include "kernels.h"
@@ -547,6 +548,8 @@ __global__ __launch_bounds__(256) void spmm_wide_kernel(uint64_t C, const uint64
 // instead of two, and takes kScaledGroups times 256 columns to be worth it: 0.17 -> 0.15 ms (512 columns the
 // same, 2048 0.17).  With FP32 values, which have no scale, x in LDS takes 10 % longer, and with
 // four vectors the table's size costs what it saves.  Its length: 16 KiB leave eight workgroups to a CU.
+// Where scale times x is not finite (the row's other entries times x may be), the product is taken entry by
+// entry as without the table.
 constexpr uint32_t kSplitEntries = 1024;  // entries of a 64-column tile that is worth splitting
 constexpr uint64_t kScaledRows = 4096, kScaledGroups = 4;
 
@@ -560,76 +563,91 @@ __global__ __launch_bounds__(256) void spmm_narrow_kernel(uint64_t C, const uint
     typedef float vec __attribute__((ext_vector_type(V)));
     static_assert(!SCALED || (V == 1 && G == 1 && VT != FD_VAL_F32), "one vector, 16-bit values");
     extern __shared__ float s_scaled[];  // SCALED: scale[r] X[r]
-    if (SCALED)  // complete before the first barrier below
-        for (uint64_t r = threadIdx.x; r < R; r += blockDim.x) s_scaled[r] = scale[r] * X[r];
     constexpr int N = 64 / G;  // entry lanes of a wavefront
     constexpr int kUnroll = 4;
     __shared__ uint64_t s_ptr[257];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int j = lane % G, slot = lane / G;
     const uint64_t groups = (C + 255) / 256;
-    for (uint64_t grp = blockIdx.x; grp < groups; grp += gridDim.x) {
-        const uint64_t c0 = grp * 256;
-        const int ncol = (int)(C - c0 < 256 ? C - c0 : 256);
-        __syncthreads();
-        s_ptr[tid] = colptr[tid < ncol ? c0 + tid : C];
-        if (tid == 0) s_ptr[256] = colptr[ncol == 256 ? c0 + 256 : C];
-        __syncthreads();
-        for (int t = 0; t < 4; t++) {
-            const uint64_t n64 = s_ptr[64 * t + 64] - s_ptr[64 * t];
-            const uint32_t n = __builtin_amdgcn_readfirstlane((uint32_t)(n64 < 0xFFFFFFFFull ? n64 : 0xFFFFFFFFull));
-            const bool split = n > kSplitEntries;
-            if (!split && t != wave) continue;
-            const int first = 64 * t + (split ? 16 * wave : 0);
-            const int last = min(first + (split ? 16 : 64), ncol);
-            const uint32_t mean = n / 64;
-            const int want = mean < 12 ? 1 : (mean < 48 ? 4 : (mean < 192 ? 16 : 64));
-            const int E = min(want, N), S = N / E;
-            const int e0 = slot % E, s = slot / E;
-            for (int cb = first; cb < last; cb += S) {
-                const bool on = cb + s < last;
-                const int cc = on ? cb + s : cb;
-                const uint64_t a = s_ptr[cc], b = on ? s_ptr[cc + 1] : a;
-                for (int j0 = 0; j0 < k; j0 += V * G) {
-                    const int jj = j0 + V * j;
-                    vec acc = {};
-                    if (jj < k) {
-                        // kUnroll entries in flight; those past the column's end read its last entry
-                        // and count as 0 x 0
-                        for (uint64_t e = a + e0; e < b; e += (uint64_t)kUnroll * E) {
-                            uint32_t r[kUnroll];
-                            float v[kUnroll];
-                            vec x[kUnroll];
+    auto product = [&](auto scaled) {
+        constexpr bool kScaled = decltype(scaled)::value;
+        for (uint64_t grp = blockIdx.x; grp < groups; grp += gridDim.x) {
+            const uint64_t c0 = grp * 256;
+            const int ncol = (int)(C - c0 < 256 ? C - c0 : 256);
+            __syncthreads();
+            s_ptr[tid] = colptr[tid < ncol ? c0 + tid : C];
+            if (tid == 0) s_ptr[256] = colptr[ncol == 256 ? c0 + 256 : C];
+            __syncthreads();
+            for (int t = 0; t < 4; t++) {
+                const uint64_t n64 = s_ptr[64 * t + 64] - s_ptr[64 * t];
+                const uint32_t n = __builtin_amdgcn_readfirstlane((uint32_t)(n64 < 0xFFFFFFFFull ? n64 : 0xFFFFFFFFull));
+                const bool split = n > kSplitEntries;
+                if (!split && t != wave) continue;
+                const int first = 64 * t + (split ? 16 * wave : 0);
+                const int last = min(first + (split ? 16 : 64), ncol);
+                const uint32_t mean = n / 64;
+                const int want = mean < 12 ? 1 : (mean < 48 ? 4 : (mean < 192 ? 16 : 64));
+                const int E = min(want, N), S = N / E;
+                const int e0 = slot % E, s = slot / E;
+                for (int cb = first; cb < last; cb += S) {
+                    const bool on = cb + s < last;
+                    const int cc = on ? cb + s : cb;
+                    const uint64_t a = s_ptr[cc], b = on ? s_ptr[cc + 1] : a;
+                    for (int j0 = 0; j0 < k; j0 += V * G) {
+                        const int jj = j0 + V * j;
+                        vec acc = {};
+                        if (jj < k) {
+                            // kUnroll entries in flight; those past the column's end read its last entry
+                            // and count as 0 x 0
+                            for (uint64_t e = a + e0; e < b; e += (uint64_t)kUnroll * E) {
+                                uint32_t r[kUnroll];
+                                float v[kUnroll];
+                                vec x[kUnroll];
 #pragma unroll
-                            for (int u = 0; u < kUnroll; u++) {
-                                const uint64_t eu = e + (uint64_t)u * E;
-                                r[u] = crow[eu < b ? eu : b - 1];
-                            }
+                                for (int u = 0; u < kUnroll; u++) {
+                                    const uint64_t eu = e + (uint64_t)u * E;
+                                    r[u] = crow[eu < b ? eu : b - 1];
+                                }
 #pragma unroll
-                            for (int u = 0; u < kUnroll; u++) {
-                                const uint64_t eu = e + (uint64_t)u * E;
-                                const uint64_t at = eu < b ? eu : b - 1;
-                                v[u] = SCALED ? stored_number<VT>(cval, at) : entry_value<VT>(cval, at, scale, r[u]);
-                                x[u] = SCALED ? *(const vec*)(s_scaled + r[u])
-                                              : *(const vec*)(X + (uint64_t)r[u] * k + jj);
-                            }
+                                for (int u = 0; u < kUnroll; u++) {
+                                    const uint64_t eu = e + (uint64_t)u * E;
+                                    const uint64_t at = eu < b ? eu : b - 1;
+                                    v[u] = kScaled ? stored_number<VT>(cval, at) : entry_value<VT>(cval, at, scale, r[u]);
+                                    x[u] = kScaled ? *(const vec*)(s_scaled + r[u])
+                                                  : *(const vec*)(X + (uint64_t)r[u] * k + jj);
+                                }
 #pragma unroll
-                            for (int u = 0; u < kUnroll; u++) {
-                                const bool in = e + (uint64_t)u * E < b;
+                                for (int u = 0; u < kUnroll; u++) {
+                                    const bool in = e + (uint64_t)u * E < b;
 #pragma unroll
-                                for (int i = 0; i < V; i++)
-                                    acc[i] = fmaf(in ? v[u] : 0.0f, in ? x[u][i] : 0.0f, acc[i]);
+                                    for (int i = 0; i < V; i++)
+                                        acc[i] = fmaf(in ? v[u] : 0.0f, in ? x[u][i] : 0.0f, acc[i]);
+                                }
                             }
                         }
-                    }
-                    for (int o = E / 2; o > 0; o >>= 1)
+                        for (int o = E / 2; o > 0; o >>= 1)
 #pragma unroll
-                        for (int i = 0; i < V; i++) acc[i] += __shfl_xor(acc[i], o * G, 64);
-                    if (on && e0 == 0 && jj < k)
-                        __builtin_nontemporal_store(acc, (vec*)(Y + (c0 + (uint64_t)(cb + s)) * (uint64_t)k + jj));
+                            for (int i = 0; i < V; i++) acc[i] += __shfl_xor(acc[i], o * G, 64);
+                        if (on && e0 == 0 && jj < k)
+                            __builtin_nontemporal_store(acc, (vec*)(Y + (c0 + (uint64_t)(cb + s)) * (uint64_t)k + jj));
+                    }
                 }
             }
         }
+    };
+    if constexpr (SCALED) {
+        bool over = false;
+        for (uint64_t r = threadIdx.x; r < R; r += blockDim.x) {
+            const float sx = scale[r] * X[r];
+            over |= !(fabsf(sx) <= FLT_MAX);
+            s_scaled[r] = sx;
+        }
+        if (__syncthreads_or(over))
+            product(std::false_type{});
+        else
+            product(std::true_type{});
+    } else {
+        product(std::false_type{});
     }
 }
 

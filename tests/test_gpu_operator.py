@@ -204,3 +204,27 @@ def test_product_over_lane_arrangements(torch_cuda, k):
         want, mag = D.T @ x.astype(np.float64), np.abs(D).T @ np.abs(x.astype(np.float64))
         n = (D != 0).sum(0)[:, None]
         assert np.all(np.abs(y.cpu().numpy() - want) <= (n + 2) * U * mag), (k, vtype)
+
+
+@pytest.mark.parametrize("vtype", [fd.FD_VAL_BF16, fd.FD_VAL_FP16])
+@pytest.mark.parametrize("x1", [1e10, float("inf"), float("nan"), 0.0])
+def test_one_vector_beyond_the_float_range(torch_cuda, vtype, x1):
+    """A row whose maximum times x is not finite while its other entries' products are: one vector gives
+    what the same vector beside a second one gives (columns of at most three entries: same order)."""
+    torch = torch_cuda
+    cols = 5000
+    rng = np.random.default_rng(3)
+    v = rng.uniform(1e25, 1e27, (3, cols)).astype(np.float32)
+    v[:, 100] = 1e30
+    off = np.arange(4) * cols
+    c = np.tile(np.arange(cols, dtype=np.int64), 3)
+    with fd.Spmm(dose_mat(torch, cols, [(off, c, v.reshape(-1))]), vtype) as op:
+        x = torch.tensor([[1.0], [x1], [1e-3]], device="cuda")
+        one = op.run(x).cpu().numpy()[:, 0]
+        two = op.run(torch.cat([x, torch.ones_like(x)], 1).contiguous()).cpu().numpy()[:, 0]
+    if x1 == 1e10:
+        assert np.isinf(two[100]) and np.isfinite(np.delete(two, 100)).all()
+    if x1 == 0.0:  # the table's path: q (s x) against (q s) x, three terms of one sign
+        assert np.all(np.abs(one.astype(np.float64) - two) <= 8 * U * np.abs(two))
+    else:
+        assert np.array_equal(one, two, equal_nan=True)
