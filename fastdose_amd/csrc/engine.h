@@ -54,6 +54,7 @@ struct DevBuf {
                               : hipMalloc((void**)&ptr, want * sizeof(T));
         if (e != hipSuccess) {
             ptr = nullptr;
+            (void)hipGetLastError();  // reported here: the next launch's check must not find it again
             set_error(std::string("hipMalloc: ") + hipGetErrorString(e));
             return FD_ERR_HIP;
         }

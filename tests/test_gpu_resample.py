@@ -112,3 +112,13 @@ def test_result_far_below_the_estimate(torch_cuda, case):
     assert cols.untyped_storage().nbytes() <= 8 * (2 * len(cols) + 1024)
     assert off[1] == len(cols) and (off[1:] == len(cols)).all() and (vals > 0).all()
     assert len(none[1]) == len(none[2]) == 0 and not none[0].any()
+
+
+def test_failed_allocation_is_reported_once(torch_cuda):
+    """A matrix whose operator would need 2 TB: the call fails, and the next launches are not blamed for it."""
+    torch = torch_cuda
+    with pytest.raises(fd.FastDoseError, match="out of memory"):
+        fd.Spmm(fd.DoseMat(1 << 38))
+    d = torch.ones((3, 5), device="cuda")
+    off, cols, vals = fd.host.dense_to_csr(d)
+    assert off.tolist() == [0, 5, 10, 15] and cols.tolist() == list(range(5)) * 3 and (vals == 1.0).all()
