@@ -210,7 +210,8 @@ class Context:
              C.c_void_p(dose_dev.data_ptr()), stride, _stream_arg(stream))
 
     def resample_csr(self, beams, dose_dev, stride: int, extent: float = 2.0, stream=None):
-        """Returns (offsets, columns, values) as device tensors."""
+        """Returns (offsets, columns, values) as device tensors; columns and values may be views of memory for up
+        to twice their entries plus 1024 (clone them to hold on to no more than they need)."""
         import torch
 
         arr = beam_array(beams)
@@ -219,21 +220,41 @@ class Context:
         offsets = torch.empty(n + 1, dtype=torch.int64, device=dev)
         cap = C.c_uint64()
         call("fd_resample_capacity", self._h, arr, n, C.byref(cap))
-        # room for the estimate, so that one call does; twice only when it was too small
-        while True:
-            room = max(cap.value, 1)
-            cols = torch.empty(room, dtype=torch.int64, device=dev)
-            vals = torch.empty(room, dtype=torch.float32, device=dev)
-            csr = CSR(0, 0, room, offsets.data_ptr(), cols.data_ptr(), vals.data_ptr())
+
+        def arrays(room):
+            return (torch.empty(room, dtype=torch.int64, device=dev), torch.empty(room, dtype=torch.float32, device=dev))
+
+        def resample(cols, vals):
+            room = 0 if cols is None else len(cols)
+            csr = CSR(0, 0, room, offsets.data_ptr(), cols.data_ptr() if room else None,
+                      vals.data_ptr() if room else None)
             rc = load().fd_resample_csr(self._h, arr, n, C.c_void_p(dose_dev.data_ptr()), stride, extent,
                                         C.byref(csr), _stream_arg(stream))
-            nnz = int(csr.nnz)
-            if rc != _lib.FD_ERR_CAPACITY:
-                break
-            cap.value = nnz
+            return rc, int(csr.nnz)
+
+        # room for the estimate, so that one call does; where that room, or the call's scratch beside it, does
+        # not fit on the device, a call without room first, and arrays of the exact size after it
+        try:
+            cols, vals = arrays(max(cap.value, 1))
+        except torch.OutOfMemoryError:
+            cols = vals = None
+        rc, nnz = resample(cols, vals)
+        if rc == _lib.FD_ERR_HIP and cols is not None and b"out of memory" in load().fd_last_error():
+            cols = vals = None
+            if dev.type == "cuda":
+                torch.cuda.empty_cache()  # the library allocates beside torch
+            rc, nnz = resample(None, None)
+        if rc == _lib.FD_ERR_CAPACITY or (rc == _lib.FD_OK and cols is None):
+            cols = vals = None
+            cols, vals = arrays(max(nnz, 1))
+            if nnz:
+                rc, nnz = resample(cols, vals)
         _lib.check(rc, "fd_resample_csr")
-        if room > 2 * nnz + 1024:  # the result should not hold on to much more memory than it needs
-            return offsets, cols[:nnz].clone(), vals[:nnz].clone()
+        if len(cols) > 2 * nnz + 1024:  # the result should not hold on to much more memory than it needs
+            try:
+                return offsets, cols[:nnz].clone(), vals[:nnz].clone()
+            except torch.OutOfMemoryError:
+                pass
         return offsets, cols[:nnz], vals[:nnz]
 
     def cccs_segments(self, beams) -> np.ndarray:

@@ -114,6 +114,25 @@ def test_result_far_below_the_estimate(torch_cuda, case):
     assert len(none[1]) == len(none[2]) == 0 and not none[0].any()
 
 
+def test_estimate_beyond_the_device(torch_cuda, case, monkeypatch):
+    """An estimate for which there is no memory: the result comes from a sizing call and arrays of its size."""
+    context, beams, dose, stride = case
+    with context() as ctx:
+        want = rows(ctx.resample_csr(beams, dose, stride))
+        real = fd.host.call
+
+        def call(name, *args):
+            real(name, *args)
+            if name == "fd_resample_capacity":
+                args[-1]._obj.value = 1 << 45
+            return _lib.FD_OK
+
+        monkeypatch.setattr(fd.host, "call", call)
+        got = rows(ctx.resample_csr(beams, dose, stride))
+    for a, b in zip(want, got):
+        assert np.array_equal(a, b)
+
+
 def test_failed_allocation_is_reported_once(torch_cuda):
     """A matrix whose operator would need 2 TB: the call fails, and the next launches are not blamed for it."""
     torch = torch_cuda
