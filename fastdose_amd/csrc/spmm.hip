@@ -60,13 +60,17 @@ int hip_result(hipError_t e) {
 }
 
 // The voxel-major copy tile by tile (launch_place_tiles); *built is false when a row's columns do
-// not ascend, and nothing of the copy is written then.
+// not ascend or the tile table does not fit in memory (the general path's scratch can be smaller: 4 bytes
+// per column, and 2 per entry of 16-bit values), and nothing of the copy is written then.
 int build_by_tiles(const fd_dosemat* m, fd_spmm& p, const uint64_t* rowptr, hipStream_t s, bool* built) {
     const uint64_t nt = csc_tiles(p.cols), R = p.rows;
     DevBuf<uint64_t> base;    // exclusive scan of the tiles' totals (nt + 1), then the scan's scratch
     DevBuf<uint32_t> total;   // entries of each tile (nt), unsorted flag, the tile table, the tiles' order
-    int r = base.reserve(nt + 1 + scan_scratch_size(nt));
-    if (r == FD_OK) r = total.reserve(nt + 1 + R * (nt + 1) + csc_tile_groups(p.cols));
+    if (base.reserve(nt + 1 + scan_scratch_size(nt)) != FD_OK ||
+        total.reserve(nt + 1 + R * (nt + 1) + csc_tile_groups(p.cols)) != FD_OK) {
+        base.release();
+        return FD_OK;
+    }
     auto enqueue = [&]() -> hipError_t {
         uint32_t unsorted = 0;
         uint32_t* tiles = total.ptr + nt + 1;
@@ -87,7 +91,7 @@ int build_by_tiles(const fd_dosemat* m, fd_spmm& p, const uint64_t* rowptr, hipS
         *built = e == hipSuccess;
         return e;
     };
-    if (r == FD_OK) r = hip_result(enqueue());
+    const int r = hip_result(enqueue());
     base.release();
     total.release();
     return r;
