@@ -270,7 +270,7 @@ int max_long_dim(const fd_beam* beams, int n);
 // beamlet's BEV offset is a multiple of four floats (the packed layout; a stride of 4k floats).
 int upload_beams(Workspace& w, const fd_beam* beams, int n, uint64_t stride, hipStream_t stream);
 int run_terma(const fd_ctx* ctx, Workspace& w, int options, int n, const float* fluence, float* terma, float* dens,
-              uint64_t bev_floats, hipStream_t stream);
+              uint64_t bev_floats, hipStream_t stream, bool tables = false);
 // The march tables `tab` (timing slot FD_T_CCCS_TABLES) on `stream`.
 int run_cccs_tables(const fd_ctx* ctx, Workspace& w, const CccsTables& tab, hipStream_t stream);
 int run_cccs(const fd_ctx* ctx, Workspace& w, int options, int n, int max_L, const float* terma, const float* dens,
@@ -301,7 +301,7 @@ int run_batch(const fd_ctx* ctx, Workspace& w, int options, const fd_beam* beams
               bool overlap = false);
 
 // Device bytes a batch of these beamlets needs (BEV volumes, cone partials, resampler staging).
-size_t batch_footprint(const fd_ctx* ctx, const fd_beam* beams, int n);
+size_t batch_footprint(const fd_ctx* ctx, int options, const fd_beam* beams, int n);
 
 // Appends one matrix of `rows` rows and `nnz` nonzeros; returns where its arrays go.
 int append_matrix(fd_dosemat* m, uint64_t rows, uint64_t nnz, hipStream_t stream, uint64_t** off_dst,

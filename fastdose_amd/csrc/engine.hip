@@ -233,12 +233,71 @@ uint64_t candidate_estimate(const fd_ctx* ctx, Workspace& w, const fd_beam* beam
     return std::max<uint64_t>((uint64_t)std::ceil(w.cand_per_beamlet * *frustum), 1024);
 }
 
-// Partial CCCS volumes of a batch of n beamlets per BEV value, at least 4: the Terma kernel's scratch.
-static int partial_volumes(const fd_ctx* ctx, int n) {
-    return std::max(cccs_volumes(n, ctx->n_fwd, ctx->cones.n_phi), 4);
+namespace {
+
+// Partial CCCS volumes of a batch of n beamlets (with or without march tables).
+int partial_volumes(const fd_ctx* ctx, int n, uint64_t bev_floats, bool tables) {
+    return cccs_volumes(n, ctx->n_fwd, ctx->cones.n_phi, bev_floats, tables);
 }
 
-size_t batch_footprint(const fd_ctx* ctx, const fd_beam* beams, int n) {
+// The buffer of a batch's partials, at least 4 floats per BEV value: the Terma kernel's scratch.
+int reserve_cccs(const fd_ctx* ctx, Workspace& w, int n, uint64_t bev_floats, bool tables) {
+    return w.partial.reserve((size_t)bev_floats * std::max(partial_volumes(ctx, n, bev_floats, tables), 4));
+}
+
+// March geometries of a batch: beamlets of equal pitch and longitudinal spacing share their lattice walk.
+struct MarchGeom {
+    uint32_t bits[3];
+    int Lmax;
+};
+// geom_of (nullable): each beamlet's index into the result.
+std::vector<MarchGeom> march_geometries(const fd_beam* beams, int n, int32_t* geom_of) {
+    std::vector<MarchGeom> geoms;
+    // open-addressed index of the geometries by their bit patterns
+    size_t slots = 64;
+    while (slots < 2 * (size_t)n) slots *= 2;
+    std::vector<int> slot_geom(slots, -1);
+    for (int i = 0; i < n; i++) {
+        uint32_t k[3];
+        std::memcpy(&k[0], &beams[i].beamlet_size[0], 4);
+        std::memcpy(&k[1], &beams[i].beamlet_size[1], 4);
+        std::memcpy(&k[2], &beams[i].long_spacing, 4);
+        uint64_t hsh = ((uint64_t)k[0] * 0x9E3779B97F4A7C15ull) ^ ((uint64_t)k[1] * 0xC2B2AE3D27D4EB4Full) ^
+                       ((uint64_t)k[2] * 0x165667B19E3779F9ull);
+        size_t h = (size_t)(hsh ^ (hsh >> 29)) & (slots - 1);
+        int g;
+        for (;;) {
+            g = slot_geom[h];
+            if (g < 0 || std::memcmp(geoms[g].bits, k, sizeof(k)) == 0) break;
+            h = (h + 1) & (slots - 1);
+        }
+        if (g < 0) {
+            g = (int)geoms.size();
+            geoms.push_back(MarchGeom{{k[0], k[1], k[2]}, 0});
+            slot_geom[h] = g;
+        }
+        geoms[g].Lmax = std::max(geoms[g].Lmax, (int)beams[i].long_dim);
+        if (geom_of) geom_of[i] = g;
+    }
+    return geoms;
+}
+
+// Beamlets of a batch per march geometry at which the tables replace the march wavefronts by
+// default: below it, walking every geometry's longest beamlet costs about what it saves.
+constexpr int kTabMinShare = 4;
+
+// Whether the context and the options allow march tables, and whether a batch takes them (FD_OPT_TABLES,
+// or kTabMinShare beamlets per march geometry unless FD_OPT_NO_TABLES).
+bool tables_allowed(const fd_ctx* ctx, int options) {
+    return !(options & FD_OPT_NO_TABLES) && ctx->n_fwd > 0 && ctx->cones.n_phi <= cccs_table_max_phi();
+}
+bool tables_taken(int options, int n, size_t n_geoms) {
+    return (options & FD_OPT_TABLES) || n >= kTabMinShare * (int)n_geoms;
+}
+
+}  // namespace
+
+size_t batch_footprint(const fd_ctx* ctx, int options, const fd_beam* beams, int n) {
     if (n <= 0) return 0;
     uint64_t bev = 0;  // BEV floats of the batch (packed volumes)
     double cand = 0;
@@ -247,7 +306,10 @@ size_t batch_footprint(const fd_ctx* ctx, const fd_beam* beams, int n) {
         cand += frustum_voxels(beams[i], ctx->vol);
     }
     const size_t segs = (size_t)n * ctx->vol.dim[2];
-    return (size_t)bev * sizeof(float) * (3 + partial_volumes(ctx, n)) + (size_t)n * kNpix * sizeof(float) +
+    int volumes = partial_volumes(ctx, n, bev, false);
+    if (volumes > ctx->n_fwd && tables_allowed(ctx, options))
+        volumes = partial_volumes(ctx, n, bev, tables_taken(options, n, march_geometries(beams, n, nullptr).size()));
+    return (size_t)bev * sizeof(float) * (3 + std::max(volumes, 4)) + (size_t)n * kNpix * sizeof(float) +
            (size_t)(2.0 * cand) * (2 * sizeof(uint64_t) + 2 * sizeof(float)) + segs * 32 + (size_t)n * 128;
 }
 
@@ -275,17 +337,15 @@ int upload_beams(Workspace& w, const fd_beam* beams, int n, uint64_t stride, hip
     return FD_OK;
 }
 
-int reserve_cccs(const fd_ctx* ctx, Workspace& w, int n, uint64_t bev_floats);
-
 int run_terma(const fd_ctx* ctx, Workspace& w, int options, int n, const float* fluence, float* terma, float* dens,
-              uint64_t bev_floats, hipStream_t stream) {
+              uint64_t bev_floats, hipStream_t stream, bool tables) {
     // FP64 radiological path on rays longer than kLongRayVoxels voxels (or on all rays)
     const float vmin = std::min(ctx->vol.voxel_size[0], std::min(ctx->vol.voxel_size[1], ctx->vol.voxel_size[2]));
     const float rpl64_len = (options & FD_OPT_RPL_FP64_ALL) ? -1.0f
                             : (options & FD_OPT_RPL_FP64) ? kLongRayVoxels * vmin
                                                           : INFINITY;
-    // the per-cone partial buffer (4 floats per BEV value at least) is free until the CCCS stage
-    FD_TRY(reserve_cccs(ctx, w, n, bev_floats));
+    // the partial buffer (4 floats per BEV value at least) is free until the CCCS stage
+    FD_TRY(reserve_cccs(ctx, w, n, bev_floats, tables));
     w.mark(FD_T_TERMA, 0, stream);
     hipError_t e = launch_terma(w.desc.ptr, n, fluence, ctx->density_pad, ctx->vol, ctx->spec_dev, rpl64_len, terma,
                                 dens, w.partial.ptr, ctx->tune.terma_segments, stream);
@@ -294,12 +354,6 @@ int run_terma(const fd_ctx* ctx, Workspace& w, int options, int n, const float* 
         set_error(std::string("terma launch: ") + hipGetErrorString(e));
         return FD_ERR_HIP;
     }
-    return FD_OK;
-}
-
-// The partials of a batch whose BEV buffers hold bev_floats floats.
-int reserve_cccs(const fd_ctx* ctx, Workspace& w, int n, uint64_t bev_floats) {
-    FD_TRY(w.partial.reserve((size_t)bev_floats * partial_volumes(ctx, n)));
     return FD_OK;
 }
 
@@ -317,7 +371,8 @@ int run_cccs_tables(const fd_ctx* ctx, Workspace& w, const CccsTables& tab, hipS
 int run_cccs(const fd_ctx* ctx, Workspace& w, int options, int n, int max_L, const float* terma, const float* dens,
              float* dose, uint64_t bev_floats, hipStream_t stream, const CccsTables* tab, bool tab_built,
              bool vec4) {
-    FD_TRY(reserve_cccs(ctx, w, n, bev_floats));
+    const int volumes = partial_volumes(ctx, n, bev_floats, tab != nullptr);
+    FD_TRY(reserve_cccs(ctx, w, n, bev_floats, tab != nullptr));
     if (tab && !tab_built) FD_TRY(run_cccs_tables(ctx, w, *tab, stream));
     hipEvent_t evs[3];
     const bool t = w.timing && w.ev[0];
@@ -328,7 +383,7 @@ int run_cccs(const fd_ctx* ctx, Workspace& w, int options, int n, int max_L, con
         evs[1] = w.ev[2 * FD_T_CCCS + 1];
         evs[2] = w.ev[2 * FD_T_CONE_SUM + 1];
     }
-    hipError_t e = launch_cccs(w.desc.ptr, n, max_L, ctx->cones_dev, ctx->n_fwd, ctx->cones.n_phi,
+    hipError_t e = launch_cccs(w.desc.ptr, n, max_L, ctx->cones_dev, ctx->n_fwd, ctx->cones.n_phi, volumes,
                                (options & FD_OPT_EXACT_G) != 0, terma, dens, w.partial.ptr, dose, vec4, stream,
                                t ? evs : nullptr, tab);
     if (t) {
@@ -458,16 +513,11 @@ int run_resample_compact(const fd_ctx* ctx, Workspace& w, int n, float thr, uint
 
 namespace {
 
-// Beamlets of a batch per march geometry at which the tables replace the march wavefronts by
-// default: below it, walking every geometry's longest beamlet costs about what it saves.
-constexpr int kTabMinShare = 4;
-
-// March tables for a batch (FD_OPT_TABLES, or kTabMinShare beamlets per march geometry unless
-// FD_OPT_NO_TABLES): assigns w.tab_geom, stages one TabEntry per (geometry, forward cone) in
-// w.tab_stage and reserves the streams and headers.  Capacities: within one slice an azimuth
-// crosses at most ceil(|dx / dz|) + 1 x and ceil(|dy / dz|) + 1 y cell boundaries plus the slice
-// end (dx, dy, dz the lattice direction); twice that plus 4 bounds its steps per slice, a chunk
-// takes at most cccs_chunk_steps() of them, and a walk covers at most Lmax slices.  A chunk's
+// March tables for a batch, where it takes them (tables_taken): assigns w.tab_geom, stages one TabEntry
+// per (geometry, forward cone) in w.tab_stage and reserves the streams and headers.  Capacities: within
+// one slice an azimuth crosses at most ceil(|dx / dz|) + 1 x and ceil(|dy / dz|) + 1 y cell boundaries
+// plus the slice end (dx, dy, dz the lattice direction); twice that plus 4 bounds its steps per slice, a
+// chunk takes at most cccs_chunk_steps() of them, and a walk covers at most Lmax slices.  A chunk's
 // records never straddle a block of cccs_chunk_steps() records: the space skipped at a block end
 // is smaller than the chunk placed after it, so a stream needs at most twice its records (plus a
 // block).  Sets w.tab_n_gt (0: no tables).
@@ -479,41 +529,11 @@ int plan_tables(const fd_ctx* ctx, Workspace& w, int options, const fd_beam* bea
                   " azimuths");
         return FD_ERR_UNSUPPORTED;
     }
-    if ((options & FD_OPT_NO_TABLES) || n_fwd <= 0 || n_phi > cccs_table_max_phi()) return FD_OK;
-    struct Geom {
-        uint32_t bits[3];
-        int Lmax;
-    };
-    std::vector<Geom> geoms;
+    if (!tables_allowed(ctx, options)) return FD_OK;
     w.tab_geom.resize((size_t)n);
-    // open-addressed index of the geometries by their bit patterns
-    size_t slots = 64;
-    while (slots < 2 * (size_t)n) slots *= 2;
-    std::vector<int> slot_geom(slots, -1);
-    for (int i = 0; i < n; i++) {
-        uint32_t k[3];
-        std::memcpy(&k[0], &beams[i].beamlet_size[0], 4);
-        std::memcpy(&k[1], &beams[i].beamlet_size[1], 4);
-        std::memcpy(&k[2], &beams[i].long_spacing, 4);
-        uint64_t hsh = ((uint64_t)k[0] * 0x9E3779B97F4A7C15ull) ^ ((uint64_t)k[1] * 0xC2B2AE3D27D4EB4Full) ^
-                       ((uint64_t)k[2] * 0x165667B19E3779F9ull);
-        size_t h = (size_t)(hsh ^ (hsh >> 29)) & (slots - 1);
-        int g;
-        for (;;) {
-            g = slot_geom[h];
-            if (g < 0 || std::memcmp(geoms[g].bits, k, sizeof(k)) == 0) break;
-            h = (h + 1) & (slots - 1);
-        }
-        if (g < 0) {
-            g = (int)geoms.size();
-            geoms.push_back(Geom{{k[0], k[1], k[2]}, 0});
-            slot_geom[h] = g;
-        }
-        geoms[g].Lmax = std::max(geoms[g].Lmax, (int)beams[i].long_dim);
-        w.tab_geom[i] = g;
-    }
+    const std::vector<MarchGeom> geoms = march_geometries(beams, n, w.tab_geom.data());
     const int ng = (int)geoms.size();
-    if (!(options & FD_OPT_TABLES) && n < kTabMinShare * ng) return FD_OK;
+    if (!tables_taken(options, n, geoms.size())) return FD_OK;
     const size_t n_gt = (size_t)ng * n_fwd;
     FD_TRY(grow_pinned(w.tab_stage, w.tab_stage_cap, n_gt));
     const int chunk = cccs_chunk_steps();
@@ -587,9 +607,9 @@ int run_batch(const fd_ctx* ctx, Workspace& w, int options, const fd_beam* beams
     FD_TRY(w.out_cols.reserve(cap));
     FD_TRY(w.out_vals.reserve(cap));
 
-    FD_TRY(reserve_cccs(ctx, w, n, bev));
-    FD_TRY(reserve_host_rowoff(w, n));
     FD_TRY(plan_tables(ctx, w, options, beams, n));
+    FD_TRY(reserve_cccs(ctx, w, n, bev, w.tab_n_gt > 0));
+    FD_TRY(reserve_host_rowoff(w, n));
     FD_TRY(stage_inputs(w, beams, n, 0, w.bev_offs.data(), fluence, overlap));
     const CccsTables tabs{w.tab_ent.ptr, w.tab_rec.ptr, w.tab_hdr.ptr, w.flags.ptr + 2, w.tab_n_gt};
     if (overlap && !w.aux_stream) {
@@ -604,8 +624,9 @@ int run_batch(const fd_ctx* ctx, Workspace& w, int options, const fd_beam* beams
     if (w.tab_n_gt)
         for (int i = 0; i < n; i++) w.stage[i].geom = w.tab_geom[i];
 
-    // Everything from the uploads to the host copies of the totals is one stream-ordered sequence
-    // with no host synchronisation, so it can run as a captured HIP graph (FD_OPT_GRAPH).
+    // Everything from the uploads to the last kernel, which writes the totals into host memory, is one
+    // stream-ordered sequence with no host synchronisation, so it can run as a captured HIP graph
+    // (FD_OPT_GRAPH).
     auto enqueue = [&](hipStream_t st) -> int {
         FD_HIP(hipMemcpyAsync(w.desc.ptr, w.stage, (size_t)n * sizeof(BeamletDev), hipMemcpyHostToDevice, st));
         FD_HIP(hipMemcpyAsync(w.fluence.ptr, w.flu_stage, (size_t)n * kNpix * sizeof(float), hipMemcpyHostToDevice,
@@ -627,7 +648,8 @@ int run_batch(const fd_ctx* ctx, Workspace& w, int options, const fd_beam* beams
             FD_TRY(launch_count(ctx, w, n, w.aux_stream));
             FD_HIP(hipEventRecord(w.count_ev, w.aux_stream));
         }
-        FD_TRY(run_terma(ctx, w, options, n, w.fluence.ptr, w.terma.ptr, w.dens_bev.ptr, bev, st));
+        FD_TRY(run_terma(ctx, w, options, n, w.fluence.ptr, w.terma.ptr, w.dens_bev.ptr, bev, st,
+                         w.tab_n_gt > 0));
         if (overlap && w.tab_n_gt) FD_HIP(hipStreamWaitEvent(st, w.join_ev, 0));
         FD_TRY(run_cccs(ctx, w, options, n, maxL, w.terma.ptr, w.dens_bev.ptr, w.dose_bev.ptr, bev, st,
                         w.tab_n_gt ? &tabs : nullptr, overlap));

@@ -50,18 +50,20 @@ hipError_t launch_cccs_tables(const CccsTables& tab, const ConeTable* cones_dev,
 int cccs_table_max_phi();
 int cccs_chunk_steps();  // lattice steps of one azimuth per chunk at most
 
+// Partial volumes per beamlet for a batch of n whose BEV buffers hold bev_floats floats: n_fwd, or more
+// where the widest cone is split (never with march tables).
+int cccs_volumes(int n, int n_fwd, int n_phi, uint64_t bev_floats, bool tables);
+
 // CCCS over the forward cones (DoseComp.cu:217-392): per-cone partial BEV doses
-// partial[v * bev_off_b + t * L_b * 256 + s * 256 + p] with v = cccs_volumes volumes per beamlet (at least
-// v times the batch's BEV floats), then their sum into dose (four floats per thread when vec4: every
-// bev_off_b a multiple of four).
+// partial[v * bev_off_b + t * L_b * 256 + s * 256 + p] with v = n_vol volumes per beamlet, as cccs_volumes
+// gives them (at least v times the batch's BEV floats), then their sum into dose (four floats per thread
+// when vec4: every bev_off_b a multiple of four).
 // ev (nullable): events recorded before the CCCS kernel, between it and the cone sum, and after.
 // tab (nullable, n_phi <= cccs_table_max_phi()): the beamlets' march tables, built on this stream
 // beforehand (launch_cccs_tables), beams[b].geom indexing them; the CCCS reads its chunks from
 // them, with the results of the march wavefront.
-// Partial volumes per beamlet for a batch of n: n_fwd, or more where the widest cone is split.
-int cccs_volumes(int n, int n_fwd, int n_phi);
 hipError_t launch_cccs(const BeamletDev* beams, int n, int max_L, const ConeTable* cones_dev, int n_fwd,
-                       int n_phi, bool exact_g, const float* terma, const float* dens_bev, float* partial,
+                       int n_phi, int n_vol, bool exact_g, const float* terma, const float* dens_bev, float* partial,
                        float* dose, bool vec4, hipStream_t stream, hipEvent_t* ev = nullptr,
                        const CccsTables* tab = nullptr);
 

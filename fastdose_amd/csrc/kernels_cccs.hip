@@ -639,6 +639,7 @@ enum Shape { kNarrow, kWide, kSplit };
 // second half, and the last one's length.
 __host__ __device__ constexpr int split_volumes(int n_phi) { return n_phi / 2 + 1; }
 constexpr uint64_t kSplitGroups = 256;  // most workgroups of a batch with a split cone (cccs_split_kernel)
+constexpr uint64_t kSplitBytes = 1ull << 29;  // and most bytes of its partial buffer
 template <Shape SHAPE>
 __device__ __forceinline__ bool loads_ahead(const CcBlock& K) { return SHAPE != kNarrow || K.n_waves >= 4; }
 
@@ -1606,12 +1607,14 @@ __global__ __launch_bounds__(256) void cone_sum_split_kernel(const BeamletDev* _
 
 }  // namespace
 
-int cccs_volumes(int n, int n_fwd, int n_phi) {
+int cccs_volumes(int n, int n_fwd, int n_phi, uint64_t bev_floats, bool tables) {
     // an even number of azimuths, at least eight wavefronts in the other cones' workgroups (kWide), a CU
-    // for each workgroup
-    const bool split = n_phi % 2 == 0 && n_phi >= 8 && n_phi <= kMaxMarchPhi && n_fwd > 0 &&
-                       (uint64_t)n * (uint64_t)(n_fwd + 1) <= kSplitGroups;
-    return n_fwd + (split ? split_volumes(n_phi) : 0);
+    // for each workgroup, and not much more memory than without: 51 beamlets of 1100 slices reach the limit
+    const int volumes = n_fwd + split_volumes(n_phi);
+    const bool split = !tables && n_phi % 2 == 0 && n_phi >= 8 && n_phi <= kMaxMarchPhi && n_fwd > 0 &&
+                       (uint64_t)n * (uint64_t)(n_fwd + 1) <= kSplitGroups &&
+                       bev_floats <= kSplitBytes / sizeof(float) / (uint64_t)volumes;
+    return split ? volumes : n_fwd;
 }
 
 int cccs_table_max_phi() { return kMaxMarchPhi; }
@@ -1628,11 +1631,11 @@ hipError_t launch_cccs_tables(const CccsTables& tab, const ConeTable* cones_dev,
 }
 
 hipError_t launch_cccs(const BeamletDev* beams, int n, int max_L, const ConeTable* cones_dev, int n_fwd,
-                       int n_phi, bool exact_g, const float* terma, const float* dens_bev, float* partial,
+                       int n_phi, int n_vol, bool exact_g, const float* terma, const float* dens_bev, float* partial,
                        float* dose, bool vec4, hipStream_t stream, hipEvent_t* ev, const CccsTables* tab) {
     if (n <= 0) return hipSuccess;
     if (ev) (void)hipEventRecord(ev[0], stream);
-    const bool split = !tab && cccs_volumes(n, n_fwd, n_phi) > n_fwd;
+    const bool split = n_vol > n_fwd;
     if (split) {
         const dim3 grid((unsigned)(n * (n_fwd + 1))), block((n_phi + 1) * kWave);
         const auto kernel = exact_g ? cccs_split_kernel<true> : cccs_split_kernel<false>;

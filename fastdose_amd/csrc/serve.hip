@@ -166,7 +166,7 @@ void slot_loop(fd_server* s, int slot) {
                     beams.insert(beams.end(), r.req->beamlets.begin() + f, r.req->beamlets.begin() + f + c);
                     flu.insert(flu.end(), r.req->fluence.begin() + f * kNpix, r.req->fluence.begin() + (f + c) * kNpix);
                 }
-                bytes = batch_footprint(s->ctx, beams.data(), (int)beams.size());
+                bytes = batch_footprint(s->ctx, s->opts.options, beams.data(), (int)beams.size());
                 if (s->inflight_batches == 0 || s->inflight_bytes + bytes <= s->opts.hbm_budget) {
                     for (size_t k = 0; k < batch.size(); k++) s->queue.pop_front();
                     s->inflight_bytes += bytes;

@@ -92,3 +92,52 @@ def test_few_and_many_workgroups(torch_cuda):
                 L = beams[k].long_dim
                 assert np.array_equal(d[:L], dose[k, :L]) and d[:L].max() > 0
                 k += 1
+
+
+def test_split_partials_stay_small(torch_cuda):
+    """A split cone takes more partial volumes (nine instead of four here), but not beyond 512 MiB: one
+    beamlet of 50 000 slices is split (440 MiB), one of 60 000 (527) is not; the slices they share are the
+    same bits."""
+    torch = torch_cuda
+    cfg = synth.small_config(seed=77, dim=(22, 26, 23), fluence_dim=1, angles=(20.0, 15.0, 0.0))
+    cfg.kernel = synth.synthetic_kernel(1077, n_phi=8)
+    beams, _ = beamlets_of(cfg)
+    beams = fd.beam_array(list(beams)[:1])
+    depth = beams[0].long_spacing * beams[0].long_dim
+    slice_floats = 256
+    g = torch.Generator(device="cuda")
+    g.manual_seed(5)
+    T = torch.rand(60000 * slice_floats, device="cuda", generator=g)
+    R = torch.rand(60000 * slice_floats, device="cuda", generator=g) + 0.5
+    dose, taken = [], []
+    for L in (50000, 60000):
+        beams[0].long_dim, beams[0].long_spacing = L, depth / 60000
+        D = torch.zeros(L * slice_floats, device="cuda")
+        log(f"split partials, {L} slices")
+        with fd.Context(cfg.volume, cfg.density, cfg.spectrum, cfg.kernel) as ctx:
+            torch.cuda.synchronize()
+            free = torch.cuda.mem_get_info()[0]
+            ctx.cccs(beams, T[:D.numel()], R[:D.numel()], D, D.numel())
+            torch.cuda.synchronize()
+            taken.append(free - torch.cuda.mem_get_info()[0])
+        dose.append(D)
+    assert torch.equal(dose[0], dose[1][:dose[0].numel()]) and float(dose[0].max()) > 0
+    assert taken[0] > 8 * 50000 * slice_floats * 4      # the split's volumes
+    assert taken[1] < 5 * 60000 * slice_floats * 4
+
+
+def test_no_split_volumes_beside_march_tables(torch_cuda):
+    """A served batch of 16 beamlets: with march tables the widest cone is not split, and the batch counts
+    five volumes less."""
+    cfg = synth.small_config(seed=78, dim=(30, 26, 28), fluence_dim=4, angles=(20.0, 15.0, 0.0))
+    cfg.kernel = synth.synthetic_kernel(1078, n_phi=8)
+    beams, flu = beamlets_of(cfg)
+    peak, mats = [], []
+    with fd.Context(cfg.volume, cfg.density, cfg.spectrum, cfg.kernel) as ctx:
+        for how in (fd.FD_OPT_NO_TABLES, fd.FD_OPT_TABLES):
+            log(f"served batch, options {how}")
+            with fd.Server(ctx, n_slots=1, options=how) as server:
+                mats.append(server.fetch(server.submit(beams, flu, [len(beams)])))
+                peak.append(server.stats()["peak_inflight_bytes"])
+    assert peak[0] - peak[1] == 5 * 4 * 256 * sum(b.long_dim for b in beams)
+    assert same_matrix(mats[0].matrix(0), mats[1].matrix(0))
