@@ -550,10 +550,18 @@ __global__ __launch_bounds__(256) void spmm_wide_kernel(uint64_t C, const uint64
 // four vectors the table's size costs what it saves.  Its length: 16 KiB leave eight workgroups to a CU.
 // Where scale times x is not finite (the row's other entries times x may be), the product is taken entry by
 // entry as without the table.
+// M (k above 64, no multiple of four): a lane takes M vectors 64 apart, so a column's entries are read once
+// for 128 or 256 vectors.  Such rows of Y are no whole lines, and streamed out in parts they cost more than
+// the entries where columns are short: tiles without entries are written as one run of zeros, tiles with
+// few entries through L2, which merges the lines' parts; the others are streamed (through L2 they take 5-10 %
+// longer, the entries and X no longer stay there).  129 vectors, FP32: 262 144 columns with 32 000 entries
+// 79 us with four words per lane and a column per wavefront, 96 with a pass per 64 vectors, 59 so;
+// 2 097 152 columns with 65 000 entries 434, 543, 218; 128^3 voxels with 256 pencil rows 1087, 741, 384.
 constexpr uint32_t kSplitEntries = 1024;  // entries of a 64-column tile that is worth splitting
 constexpr uint64_t kScaledRows = 4096, kScaledGroups = 4;
+constexpr uint32_t kMergeEntries = 128;  // of a 64-column tile: below, its rows go through L2 (M > 1)
 
-template <int VT, int V, int G, bool SCALED = false>
+template <int VT, int V, int G, bool SCALED = false, int M = 1>
 __global__ __launch_bounds__(256) void spmm_narrow_kernel(uint64_t C, const uint64_t* __restrict__ colptr,
                                                           const uint32_t* __restrict__ crow,
                                                           const void* __restrict__ cval,
@@ -562,6 +570,7 @@ __global__ __launch_bounds__(256) void spmm_narrow_kernel(uint64_t C, const uint
                                                           float* __restrict__ Y) {
     typedef float vec __attribute__((ext_vector_type(V)));
     static_assert(!SCALED || (V == 1 && G == 1 && VT != FD_VAL_F32), "one vector, 16-bit values");
+    static_assert(M == 1 || (V == 1 && G == 64), "several parts of a row");
     extern __shared__ float s_scaled[];  // SCALED: scale[r] X[r]
     constexpr int N = 64 / G;  // entry lanes of a wavefront
     constexpr int kUnroll = 4;
@@ -583,6 +592,12 @@ __global__ __launch_bounds__(256) void spmm_narrow_kernel(uint64_t C, const uint
                 const uint32_t n = __builtin_amdgcn_readfirstlane((uint32_t)(n64 < 0xFFFFFFFFull ? n64 : 0xFFFFFFFFull));
                 const bool split = n > kSplitEntries;
                 if (!split && t != wave) continue;
+                if (M > 1 && n == 0 && 64 * t + 64 <= ncol && (reinterpret_cast<uintptr_t>(Y) & 15) == 0) {
+                    v4f* out = (v4f*)(Y + (c0 + 64 * (uint64_t)t) * (uint64_t)k);  // 64 rows of zeros, whole lines
+                    for (int i = lane; i < 16 * k; i += 64) __builtin_nontemporal_store(v4f{}, out + i);
+                    continue;
+                }
+                const bool merge = M > 1 && n < kMergeEntries;
                 const int first = 64 * t + (split ? 16 * wave : 0);
                 const int last = min(first + (split ? 16 : 64), ncol);
                 const uint32_t mean = n / 64;
@@ -593,16 +608,16 @@ __global__ __launch_bounds__(256) void spmm_narrow_kernel(uint64_t C, const uint
                     const bool on = cb + s < last;
                     const int cc = on ? cb + s : cb;
                     const uint64_t a = s_ptr[cc], b = on ? s_ptr[cc + 1] : a;
-                    for (int j0 = 0; j0 < k; j0 += V * G) {
+                    for (int j0 = 0; j0 < k; j0 += V * G * M) {
                         const int jj = j0 + V * j;
-                        vec acc = {};
+                        vec acc[M] = {};
                         if (jj < k) {
                             // kUnroll entries in flight; those past the column's end read its last entry
                             // and count as 0 x 0
                             for (uint64_t e = a + e0; e < b; e += (uint64_t)kUnroll * E) {
                                 uint32_t r[kUnroll];
                                 float v[kUnroll];
-                                vec x[kUnroll];
+                                vec x[kUnroll][M];
 #pragma unroll
                                 for (int u = 0; u < kUnroll; u++) {
                                     const uint64_t eu = e + (uint64_t)u * E;
@@ -613,23 +628,37 @@ __global__ __launch_bounds__(256) void spmm_narrow_kernel(uint64_t C, const uint
                                     const uint64_t eu = e + (uint64_t)u * E;
                                     const uint64_t at = eu < b ? eu : b - 1;
                                     v[u] = kScaled ? stored_number<VT>(cval, at) : entry_value<VT>(cval, at, scale, r[u]);
-                                    x[u] = kScaled ? *(const vec*)(s_scaled + r[u])
-                                                  : *(const vec*)(X + (uint64_t)r[u] * k + jj);
+#pragma unroll
+                                    for (int m = 0; m < M; m++) {
+                                        x[u][m] = vec{};
+                                        if (m == 0 || jj + m * V * G < k)
+                                            x[u][m] = kScaled ? *(const vec*)(s_scaled + r[u])
+                                                              : *(const vec*)(X + (uint64_t)r[u] * k + jj + m * V * G);
+                                    }
                                 }
 #pragma unroll
                                 for (int u = 0; u < kUnroll; u++) {
                                     const bool in = e + (uint64_t)u * E < b;
 #pragma unroll
-                                    for (int i = 0; i < V; i++)
-                                        acc[i] = fmaf(in ? v[u] : 0.0f, in ? x[u][i] : 0.0f, acc[i]);
+                                    for (int m = 0; m < M; m++)
+#pragma unroll
+                                        for (int i = 0; i < V; i++)
+                                            acc[m][i] = fmaf(in ? v[u] : 0.0f, in ? x[u][m][i] : 0.0f, acc[m][i]);
                                 }
                             }
                         }
-                        for (int o = E / 2; o > 0; o >>= 1)
+                        for (int o = E / 2; o > 0; o >>= 1)  // (one entry lane where M > 1)
 #pragma unroll
-                            for (int i = 0; i < V; i++) acc[i] += __shfl_xor(acc[i], o * G, 64);
-                        if (on && e0 == 0 && jj < k)
-                            __builtin_nontemporal_store(acc, (vec*)(Y + (c0 + (uint64_t)(cb + s)) * (uint64_t)k + jj));
+                            for (int i = 0; i < V; i++) acc[0][i] += __shfl_xor(acc[0][i], o * G, 64);
+#pragma unroll
+                        for (int m = 0; m < M; m++) {
+                            if (!(on && e0 == 0 && jj + m * V * G < k)) continue;
+                            vec* out = (vec*)(Y + (c0 + (uint64_t)(cb + s)) * (uint64_t)k + jj + m * V * G);
+                            if (merge)
+                                *out = acc[m];
+                            else
+                                __builtin_nontemporal_store(acc[m], out);
+                        }
                     }
                 }
             }
@@ -753,6 +782,13 @@ void launch_narrow(int G, const dim3& g, const dim3& b, hipStream_t stream, uint
             const dim3 few(blocks_for((C + kScaledGroups - 1) / kScaledGroups, 65536));
             hipLaunchKernelGGL((spmm_narrow_kernel<VT, 1, 1, true>), few, b, R * sizeof(float), stream, C, colptr, crow,
                                cval, scale, X, k, R, Y);
+            return;
+        }
+    if constexpr (V == 1)
+        if (k > 64) {
+            const auto kernel =
+                k > 128 ? spmm_narrow_kernel<VT, 1, 64, false, 4> : spmm_narrow_kernel<VT, 1, 64, false, 2>;
+            hipLaunchKernelGGL(kernel, g, b, 0, stream, C, colptr, crow, cval, scale, X, k, R, Y);
             return;
         }
     switch (G) {

@@ -206,6 +206,37 @@ def test_product_over_lane_arrangements(torch_cuda, k):
         assert np.all(np.abs(y.cpu().numpy() - want) <= (n + 2) * U * mag), (k, vtype)
 
 
+@pytest.mark.parametrize("k", [127, 129, 131, 255, 257, 515])
+def test_product_of_odd_numbers_of_vectors_around_128(torch_cuda, k):
+    """Beyond 128 vectors a wavefront takes one column at a time, also where k is no multiple of four."""
+    test_product_over_lane_arrangements(torch_cuda, k)
+
+
+@pytest.mark.parametrize("k", [65, 66, 127, 129, 131, 191, 255, 257, 515])
+def test_product_of_odd_numbers_of_vectors(torch_cuda, k):
+    """Beyond 64 vectors, where k is no multiple of four, a lane takes two or four vectors 64 apart and columns
+    without entries are written in one run; also into memory that is not aligned to 16 bytes."""
+    test_product_over_lane_arrangements(torch_cuda, k)
+    torch = torch_cuda
+    rng = np.random.default_rng(k)
+    R, cols = 40, 1500
+    off, c, v = random_rows(rng, R, cols, 0.01)
+    keep = (c < 300) | (c >= 700)  # 400 columns without entries
+    off = np.concatenate([[0], np.cumsum(keep)])[off]
+    mats = [(off, c[keep], v[keep])]
+    x = rng.uniform(-1.0, 1.0, (R, k)).astype(np.float32)
+    xd = torch.as_tensor(x).cuda()
+    with fd.Spmm(dose_mat(torch, cols, mats)) as op:
+        y = op.run(xd).cpu().numpy()
+        buf = torch.full((cols * k + 2,), -7.0, device="cuda")
+        _lib.call("fd_spmm_run", op._h, C.c_void_p(xd.data_ptr()), k, C.c_void_p(buf[1:].data_ptr()), None)
+        shifted = buf.cpu().numpy()
+    D = dense(mats, cols)
+    want, mag = D.T @ x.astype(np.float64), np.abs(D).T @ np.abs(x.astype(np.float64))
+    assert np.all(np.abs(y - want) <= ((D != 0).sum(0)[:, None] + 2) * U * mag)
+    assert np.array_equal(shifted[1:-1].reshape(cols, k), y) and shifted[0] == shifted[-1] == -7.0
+
+
 @pytest.mark.parametrize("vtype", [fd.FD_VAL_BF16, fd.FD_VAL_FP16])
 @pytest.mark.parametrize("x1", [1e10, float("inf"), float("nan"), 0.0])
 def test_one_vector_beyond_the_float_range(torch_cuda, vtype, x1):
