@@ -171,7 +171,7 @@ int fd_beamlet_flags(fd_ctx* ctx, const uint8_t* mask_dev, const fd_bundle* bund
     }
     if (n_bundles == 0) return FD_OK;
     std::vector<FlagBeamDev> d((size_t)n_bundles);
-    uint64_t total = 0;
+    uint64_t total = 0, points = 0;  // points: nine rays a beamlet
     int max_pixels = 0;
     for (int b = 0; b < n_bundles; b++) {
         const int fx = bundles[b].fluence_dim[0], fy = bundles[b].fluence_dim[1];
@@ -182,6 +182,7 @@ int fd_beamlet_flags(fd_ctx* ctx, const uint8_t* mask_dev, const fd_bundle* bund
         (void)flag_beam_setup(bundles[b], ctx->vol, d[b]);  // a miss leaves L = 0: all flags 0
         d[b].out_off = (uint32_t)total;
         total += (uint64_t)fx * fy;
+        points += (uint64_t)fx * fy * 9 * (uint64_t)std::max(d[b].L, 0);
         max_pixels = std::max(max_pixels, fx * fy);
     }
     if (total >= (1ull << 32)) {
@@ -189,12 +190,15 @@ int fd_beamlet_flags(fd_ctx* ctx, const uint8_t* mask_dev, const fd_bundle* bund
         return FD_ERR_ARG;
     }
     hipStream_t s = (hipStream_t)stream;
+    // the bounding box's six words, all ones, behind the descriptors: one copy sets both up
+    static_assert(sizeof(FlagBeamDev) >= 6 * sizeof(uint32_t) && alignof(FlagBeamDev) >= alignof(uint32_t), "room");
+    d.emplace_back();
+    std::memset(&d.back(), 0xFF, sizeof(FlagBeamDev));
     FD_TRY(ctx->flag_desc.reserve(d.size()));
     FD_TRY(ctx->flag_out.reserve(total));
-    FD_TRY(ctx->flag_box.reserve(6));
     FD_HIP(hipMemcpyAsync(ctx->flag_desc.ptr, d.data(), d.size() * sizeof(FlagBeamDev), hipMemcpyHostToDevice, s));
-    hipError_t e = launch_beamlet_flags(ctx->flag_desc.ptr, n_bundles, max_pixels, mask_dev, ctx->vol,
-                                        ctx->flag_box.ptr, ctx->flag_out.ptr, s);
+    hipError_t e = launch_beamlet_flags(ctx->flag_desc.ptr, n_bundles, max_pixels, points, mask_dev, ctx->vol,
+                                        (uint32_t*)(ctx->flag_desc.ptr + n_bundles), ctx->flag_out.ptr, s);
     if (e != hipSuccess) {
         set_error(std::string("beamlet flags launch: ") + hipGetErrorString(e));
         return FD_ERR_HIP;
@@ -436,7 +440,6 @@ int fd_ctx_destroy(fd_ctx* ctx) {
     ctx->ws.release();
     ctx->flag_desc.release();
     ctx->flag_out.release();
-    ctx->flag_box.release();
     for (auto& w : ctx->parked_ws) w.release();  // frees ordered on park_stream
     for (auto& c : ctx->parked_csr) {
         c.cols.release();

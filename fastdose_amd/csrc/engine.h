@@ -226,9 +226,8 @@ struct fd_ctx {
     bool rcp_exact = false;  // the resampler's reciprocal is the IEEE quotient on this device
     fd_tuning tune{8192, 0, 16, 0.0f};  // launch parameters (fd_autotune; Terma segments also plain)
     fdi::Workspace ws;
-    fdi::DevBuf<fdi::FlagBeamDev> flag_desc;  // beamlet-flag kernel inputs / outputs
+    fdi::DevBuf<fdi::FlagBeamDev> flag_desc;  // beamlet-flag kernel inputs (the mask's box behind them) / outputs
     fdi::DevBuf<uint8_t> flag_out;
-    fdi::DevBuf<uint32_t> flag_box;  // bounding box of the mask
     // Device scratch of stopped servers, kept for the next server on this context: the slots'
     // workspaces and the output pool's CSR buffers keep their sizes, so the next server's slots
     // start without allocating (an allocation while another slot's batch runs has stalled both for

@@ -15,8 +15,9 @@ struct CsrDst {
 };
 
 // Beamlet / PTV intersection flags of n bundles (d_beamletFlagInit, IMRTBeamBundle.cu:130-316);
-// flags[beams[b].out_off + pixel], max_pixels = the largest fluence_dim^2; box: six u32 of scratch.
-hipError_t launch_beamlet_flags(const FlagBeamDev* beams, int n, int max_pixels, const uint8_t* mask,
+// flags[beams[b].out_off + pixel], max_pixels = the largest fluence_dim^2; points: sample points of all
+// beamlets; box: six u32 of scratch, all ones.
+hipError_t launch_beamlet_flags(const FlagBeamDev* beams, int n, int max_pixels, uint64_t points, const uint8_t* mask,
                                 const fd_volume& vol, uint32_t* box, uint8_t* flags, hipStream_t stream);
 
 // Per-voxel trilinear corner records of the density (8 floats per base voxel of the zero-bordered

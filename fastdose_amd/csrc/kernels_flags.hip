@@ -10,12 +10,13 @@
 //
 // A plan's target fills a small part of the volume and most candidate beamlets miss it, which took the
 // walk of every point with its eight texel reads.  A first kernel finds the mask's bounding box
-// (reading the mask once); a beamlet then walks only the depths at which one of its nine rays can be
+// (reading the mask once; calls of a few beamlets take the volume for it, kBoxPoints); a beamlet then walks only the depths at which one of its nine rays can be
 // inside it, and a point reads texels only if its base texel is.  What is left is the arithmetic of the
 // points in the box around the target, so a lane computes its ray once and divides by multiplying with
 // the reciprocal and correcting (Divisor).  180 beams of 400 beamlets on 200 x 200 x 160: 1.35 ms for
 // every point, 0.13 ms for those in the box, 0.065 ms with the texels of a point read at once (serial
 // reads with a branch each before: the loops took as many scalar instructions as vector ones).
+#include <algorithm>
 #include <hip/hip_runtime.h>
 
 #include "kernels.h"
@@ -25,33 +26,45 @@ namespace {
 
 constexpr int kFlagSS = 3;
 
-// Bounding box of the mask's nonzero texels: box[0..2] the smallest x, y, z, box[3..5] the bitwise
-// complements of the largest (so that every entry is a minimum; ~0 in all of them: an empty mask).
-__global__ __launch_bounds__(256) void mask_box_kernel(const uint8_t* __restrict__ mask, uint32_t X, uint32_t Y,
-                                                       uint64_t n, uint32_t* __restrict__ box) {
+// Bounding box of the mask's n nonzero texels: box[0..2] the smallest x, y, z, box[3..5] the bitwise
+// complements of the largest (so that every entry is a minimum; ~0 in all of them, as before the call: an
+// empty mask).  n < 2^31: its divisions take 32 bits.  Bound by reading the mask: 105 M texels, a quarter
+// of them set, take 21 us of a call, and took 157 with every set texel's coordinates and an atomic per
+// workgroup and word.
+constexpr int kBoxThreads = 512;
+constexpr uint64_t kBoxBlocks = 512;
+__global__ __launch_bounds__(kBoxThreads) void mask_box_kernel(const uint8_t* __restrict__ mask, uint32_t X, uint32_t Y,
+                                                               uint32_t n, uint32_t* __restrict__ box) {
     uint32_t lo[6] = {~0u, ~0u, ~0u, ~0u, ~0u, ~0u};
-    auto add = [&](uint64_t i) {
-        const uint64_t r = i / X;
-        const uint32_t c[3] = {(uint32_t)(i - r * X), (uint32_t)(r % Y), (uint32_t)(r / Y)};
-        for (int d = 0; d < 3; d++) {
-            lo[d] = min(lo[d], c[d]);
-            lo[3 + d] = min(lo[3 + d], ~c[d]);
-        }
+    // texels [i, j] of row r, both ends set
+    auto add = [&](uint32_t r, uint32_t i, uint32_t j) {
+        const uint32_t x0 = r * X, z = r / Y, y = r - z * Y;
+        const uint32_t v[6] = {i - x0, y, z, ~(j - x0), ~y, ~z};
+        for (int d = 0; d < 6; d++) lo[d] = min(lo[d], v[d]);
     };
-    const uint64_t id = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, all = (uint64_t)gridDim.x * blockDim.x;
+    const uint32_t id = blockIdx.x * kBoxThreads + threadIdx.x, all = gridDim.x * kBoxThreads;
     // 16 texels at a time where the mask is aligned, single ones before and after
-    const uint64_t head = min((uint64_t)(-(uintptr_t)mask & 15), n), quads = (n - head) / 16;
-    for (uint64_t i = id; i < head; i += all)
-        if (mask[i]) add(i);
-    for (uint64_t q = id; q < quads; q += all) {
+    const uint32_t head = min((uint32_t)(-(uintptr_t)mask & 15), n), quads = (n - head) / 16;
+    for (uint32_t i = id; i < head; i += all)
+        if (mask[i]) add(i / X, i, i);
+    for (uint32_t q = id; q < quads; q += all) {
         const uint4 v = reinterpret_cast<const uint4*>(mask + head)[q];
-        if ((v.x | v.y | v.z | v.w) == 0u) continue;
-        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+        const uint64_t w[2] = {v.x | (uint64_t)v.y << 32, v.z | (uint64_t)v.w << 32};
+        if ((w[0] | w[1]) == 0u) continue;
+        // the first and the last of them bound the rest, unless the row ends in between
+        const uint32_t at = head + 16 * q;
+        const uint32_t i = at + (w[0] ? __builtin_ctzll(w[0]) >> 3 : 8 + (__builtin_ctzll(w[1]) >> 3));
+        const uint32_t j = at + (w[1] ? 15 - (__builtin_clzll(w[1]) >> 3) : 7 - (__builtin_clzll(w[0]) >> 3));
+        const uint32_t r = i / X;
+        if (j - r * X < X) {
+            add(r, i, j);
+            continue;
+        }
         for (int k = 0; k < 16; k++)
-            if ((w[k >> 2] >> (8 * (k & 3))) & 255u) add(head + 16 * q + k);
+            if ((w[k >> 3] >> (8 * (k & 7))) & 255u) add((at + k) / X, at + k, at + k);
     }
-    for (uint64_t i = head + 16 * quads + id; i < n; i += all)
-        if (mask[i]) add(i);
+    for (uint32_t i = head + 16 * quads + id; i < n; i += all)
+        if (mask[i]) add(i / X, i, i);
     __shared__ uint32_t s_lo[6];
     if (threadIdx.x < 6) s_lo[threadIdx.x] = ~0u;
     __syncthreads();
@@ -60,7 +73,10 @@ __global__ __launch_bounds__(256) void mask_box_kernel(const uint8_t* __restrict
         if ((threadIdx.x & 63) == 0 && lo[d] != ~0u) atomicMin(&s_lo[d], lo[d]);
     }
     __syncthreads();
-    if (threadIdx.x < 6 && s_lo[threadIdx.x] != ~0u) atomicMin(&box[threadIdx.x], s_lo[threadIdx.x]);
+    // one line of six words: a workgroup that lowers none of them any more leaves it alone
+    if (threadIdx.x < 6 && s_lo[threadIdx.x] < __hip_atomic_load(&box[threadIdx.x], __ATOMIC_RELAXED,
+                                                                 __HIP_MEMORY_SCOPE_AGENT))
+        atomicMin(&box[threadIdx.x], s_lo[threadIdx.x]);
 }
 
 // x / v as the IEEE division rounds it, in three instructions: with r = 1 / v rounded, x r corrected by
@@ -81,12 +97,13 @@ struct Divisor {
     }
 };
 
-// The box as signed texel bounds [lo, hi] (lo > hi when empty).
+// The box as signed texel bounds [lo, hi] (lo > hi when empty); without one, the whole volume.
 struct MaskBox {
     int lo[3], hi[3];
 };
-__device__ __forceinline__ MaskBox read_box(const uint32_t* __restrict__ box) {
-    MaskBox b;
+__device__ __forceinline__ MaskBox read_box(const uint32_t* __restrict__ box, int X, int Y, int Z) {
+    MaskBox b{{0, 0, 0}, {X - 1, Y - 1, Z - 1}};
+    if (!box) return b;
     for (int d = 0; d < 3; d++) {
         const bool any = box[d] != ~0u;
         b.lo[d] = any ? (int)box[d] : 1;
@@ -193,6 +210,11 @@ __device__ __forceinline__ void ray_depths(const FlagBeamDev& d, const MaskBox& 
 }
 
 constexpr int kFlagWaves = 4;  // beamlets per workgroup
+// Below kBoxPoints sample points, and one more per kBoxVoxels texels of the mask, the box is not looked for:
+// finding it takes 4 us and 0.15 us per million texels, which beamlets that soon hit the target do not earn
+// back (16 beamlets, all hits, on 200 x 200 x 160 31 us a call without and 41 with it; 400 beamlets 32 and
+// 41, but 51 and 35 with a target eight texels wide).
+constexpr uint64_t kBoxPoints = 200000, kBoxVoxels = 64;
 
 __global__ __launch_bounds__(64 * kFlagWaves) void beamlet_flags_kernel(const FlagBeamDev* __restrict__ beams,
                                                                         const uint8_t* __restrict__ mask, int X,
@@ -204,7 +226,7 @@ __global__ __launch_bounds__(64 * kFlagWaves) void beamlet_flags_kernel(const Fl
     const int idx = blockIdx.x * kFlagWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (idx >= d.fx * d.fy) return;
     const int bx = idx % d.fx, by = idx / d.fx;
-    const MaskBox box = read_box(mask_box);
+    const MaskBox box = read_box(mask_box, X, Y, Z);
     const float v[3] = {vx, vy, vz};
     // my ray, and the depths at which it and the wavefront's nine rays can be inside the mask's box
     constexpr int kRays = kFlagSS * kFlagSS, kDepths = 64 / kRays;
@@ -237,15 +259,19 @@ __global__ __launch_bounds__(64 * kFlagWaves) void beamlet_flags_kernel(const Fl
 
 }  // namespace
 
-hipError_t launch_beamlet_flags(const FlagBeamDev* beams, int n, int max_pixels, const uint8_t* mask,
+hipError_t launch_beamlet_flags(const FlagBeamDev* beams, int n, int max_pixels, uint64_t points, const uint8_t* mask,
                                 const fd_volume& vol, uint32_t* box, uint8_t* flags, hipStream_t stream) {
     if (n <= 0 || max_pixels <= 0) return hipSuccess;
     const uint64_t voxels = (uint64_t)vol.dim[0] * vol.dim[1] * vol.dim[2];
-    hipError_t e = launch_fill_u32(box, 6, ~0u, stream);
-    if (e != hipSuccess) return e;
-    const uint64_t blocks = (voxels / 16 + 255) / 256 + 1;
-    hipLaunchKernelGGL(mask_box_kernel, dim3((unsigned)(blocks < 1024 ? blocks : 1024)), dim3(256), 0, stream, mask,
-                       vol.dim[0], vol.dim[1], voxels, box);
+    if (points < kBoxPoints + voxels / kBoxVoxels || voxels >= (1ull << 31)) {
+        box = nullptr;
+    } else {
+        const uint64_t blocks = std::min(voxels / (16 * kBoxThreads) + 1, kBoxBlocks);
+        hipLaunchKernelGGL(mask_box_kernel, dim3((unsigned)blocks), dim3(kBoxThreads), 0, stream, mask, vol.dim[0],
+                           vol.dim[1], (uint32_t)voxels, box);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
     dim3 grid((unsigned)((max_pixels + kFlagWaves - 1) / kFlagWaves), (unsigned)n), block(64 * kFlagWaves);
     hipLaunchKernelGGL(beamlet_flags_kernel, grid, block, 0, stream, beams, mask, (int)vol.dim[0], (int)vol.dim[1],
                        (int)vol.dim[2], vol.voxel_size[0], vol.voxel_size[1], vol.voxel_size[2], box, flags);

@@ -102,3 +102,38 @@ def test_flags_in_thin_volumes(torch_cuda, dim, voxel):
                 assert np.array_equal(w, g)
                 some += int(w.any())
     assert some > 0
+
+
+@pytest.mark.parametrize("name", list(masks()))
+def test_flags_with_and_without_the_box(torch_cuda, name):
+    """One beamlet and 16 of them (fewer sample points than it pays to look for the mask's box) and 30 beams of
+    400 (more): the host's flags."""
+    torch = torch_cuda
+    m = masks()[name]
+    vol = synth.make_volume(DIM, 0.25)
+    rng = np.random.default_rng(sum(map(ord, name)) + 1)
+    at = [0.25 * (d / 2 + float(rng.uniform(-4, 4))) for d in DIM]
+    angles = [(0, 0, 0), (90, 0, 0)] + [tuple(rng.uniform(0, 360, 3)) for _ in range(4)]
+    with fd.Context(vol, np.ones(DIM[::-1], np.float32), synth.synthetic_spectrum(1), synth.synthetic_kernel(1)) as ctx:
+        for fluence, copies in ((1, 1), (4, 1), (20, 5)):
+            bundles = [synth.make_bundle(at, a, fluence_dim=fluence, beamlet_size=0.4, long_spacing=0.25) for a in angles]
+            want = [fd.beamlet_flag_init(b, m, vol) for b in bundles]
+            points = sum(9 * fd.calc_range(beam_of(b), vol).long_dim * fluence ** 2 for b in bundles) * copies
+            assert (points > 200_000 + m.size // 64) == (copies == 5)
+            for shift in (0, 5):
+                buf = torch.zeros(m.size + 16, dtype=torch.uint8, device="cuda")
+                buf[shift:shift + m.size] = torch.from_numpy(m.reshape(-1)).cuda()
+                got = ctx.beamlet_flags(buf[shift:], bundles * copies)
+                for w, g in zip(want * copies, got):
+                    assert np.array_equal(w, g)
+
+
+def beam_of(bundle):
+    beam = fd.Beam()
+    for f in ("isocenter", "angles", "beamlet_size"):
+        for i, v in enumerate(getattr(bundle, f)):
+            getattr(beam, f)[i] = v
+    beam.fmap_size[0], beam.fmap_size[1] = bundle.fluence_dim[0], bundle.fluence_dim[1]
+    beam.sad, beam.long_spacing = bundle.sad, bundle.long_spacing
+    return beam
+
