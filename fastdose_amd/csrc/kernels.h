@@ -133,19 +133,21 @@ hipError_t launch_global_rows(int n_mat, const uint64_t* row_first, const uint64
 // scale[r] = row maximum; q (nullable) = value / scale in BF16 or FP16
 hipError_t launch_pack_rows(uint64_t R, const uint64_t* rowptr, const float* values, int vtype, float* scale,
                             uint16_t* q, hipStream_t stream);
-// Voxel-major copy of rows whose columns ascend: tiles of consecutive columns (csc_tiles(C) of them).
-// launch_row_tiles: tiles[r (csc_tiles(C) + 1) + t] = row r's entries before tile t; scale (nullable)
+// Voxel-major copy of rows whose columns ascend: n = csc_tiles(C, tile_cols) tiles of tile_cols consecutive
+// columns (csc_tile_cols).  launch_row_tiles: tiles[r (n + 1) + t] = row r's entries before tile t; scale (nullable)
 // = row maxima; *unsorted (zeroed by the caller) = 1 when a row's columns do not ascend below C (the
 // table then must not be used).  launch_tile_totals: total[t] (zeroed by the caller) = entries of tile
 // t.  launch_place_tiles: colptr (C + 1), crow and cval from the table and tile_base, the exclusive
-// scan of total; order: csc_tile_groups(C) words of scratch.  C > 0, R <= 2^20 and every row's length
+// scan of total; order: csc_tile_groups(C, tile_cols) words of scratch.  C > 0, R <= 2^20 and every row's length
 // below 2^32.
-uint64_t csc_tiles(uint64_t C);
-uint64_t csc_tile_groups(uint64_t C);
+uint32_t csc_tile_cols(uint64_t R, uint64_t C, bool narrow);  // narrow: where narrow tiles are worth it
+uint64_t csc_tiles(uint64_t C, uint32_t tile_cols);
+uint64_t csc_tile_groups(uint64_t C, uint32_t tile_cols);
 hipError_t launch_row_tiles(uint64_t R, const uint64_t* rowptr, const uint64_t* columns, const float* values,
-                            uint64_t C, uint32_t* tiles, float* scale, uint32_t* unsorted, hipStream_t stream);
-hipError_t launch_tile_totals(uint64_t R, uint64_t C, const uint32_t* tiles, uint32_t* total, hipStream_t stream);
-hipError_t launch_place_tiles(int vtype, uint64_t R, uint64_t C, const uint32_t* tiles, const uint64_t* rowptr,
+                            uint64_t C, uint32_t tile_cols, uint32_t* tiles, float* scale, uint32_t* unsorted,
+                            hipStream_t stream);
+hipError_t launch_tile_totals(uint64_t R, uint64_t C, uint32_t tile_cols, const uint32_t* tiles, uint32_t* total, hipStream_t stream);
+hipError_t launch_place_tiles(int vtype, uint64_t R, uint64_t C, uint32_t tile_cols, const uint32_t* tiles, const uint64_t* rowptr,
                               const uint64_t* columns, const float* values, const float* scale,
                               const uint64_t* tile_base, uint32_t* order, uint64_t* colptr, uint32_t* crow,
                               void* cval, hipStream_t stream);

@@ -51,7 +51,7 @@ __global__ void global_rows_kernel(int n_mat, const uint64_t* __restrict__ row_f
 
 // ---- Voxel-major copy of rows with ascending columns.
 //
-// The columns are cut into tiles of kTileCols.  A row's entries of one tile are contiguous, so one
+// The columns are cut into tiles of kTileCols or kNarrowTile.  A row's entries of one tile are contiguous, so one
 // pass over the rows (row_tiles_kernel, HBM-bound on the 8-byte columns) writes where every tile
 // starts in every row, and one workgroup per tile then places the tile's entries: it lists the rows
 // that reach the tile (list_rows), counts the entries per column in LDS, scans the counts into the
@@ -67,7 +67,13 @@ __global__ void global_rows_kernel(int n_mat, const uint64_t* __restrict__ row_f
 // kTileCols: a beamlet's footprint is about ten voxels wide, so 2048 columns (ten x-rows of a
 // 200-voxel plane) hold about one wavefront of a row's entries, and the tile's LDS (39.5 KiB) lets
 // four workgroups of eight wavefronts share a CU.
-constexpr int kTileCols = 2048;
+// kNarrowTile: in small volumes, where the tiles are fewer than the CUs, and with enough rows for a tile's
+// serial part (the rounds over its rows) to weigh more than a tile table of four times the size: an
+// operator of 60 pencil rows on 61 x 63 x 65 voxels is built in 95 us instead of 111, of 400 rows in 222
+// instead of 267; 7 rows would take 82 instead of 77.  The general path still is up to a tenth faster for
+// rows of a few entries scattered over a small volume, but its sort of one crowded column can take seconds.
+constexpr int kTileCols = 2048, kNarrowTile = 512;
+constexpr uint64_t kNarrowBelow = 192 * (uint64_t)kTileCols, kNarrowRow = 8192;
 constexpr int kPlaceThreads = 512;
 
 // tiles[r * (n_tiles + 1) + t] = entries of row r before tile t (t = n_tiles: all of them), and for
@@ -76,8 +82,9 @@ constexpr int kPlaceThreads = 512;
 __global__ __launch_bounds__(256) void row_tiles_kernel(const uint64_t* __restrict__ rowptr,
                                                         const uint64_t* __restrict__ columns,
                                                         const float* __restrict__ values, uint64_t C,
-                                                        uint32_t n_tiles, uint32_t* __restrict__ tiles,
-                                                        float* __restrict__ scale, uint32_t* __restrict__ unsorted) {
+                                                        uint32_t shift, uint32_t n_tiles,
+                                                        uint32_t* __restrict__ tiles, float* __restrict__ scale,
+                                                        uint32_t* __restrict__ unsorted) {
     __shared__ float s_max[4];
     const uint64_t r = blockIdx.x;
     const uint64_t a = rowptr[r], n = rowptr[r + 1] - a;
@@ -89,8 +96,8 @@ __global__ __launch_bounds__(256) void row_tiles_kernel(const uint64_t* __restri
         const uint64_t p = i > 0 ? columns[a + i - 1] : 0;
         bad |= (i > 0 && p >= c) || (i < n && c >= C);
         // tiles after the previous entry's, up to this one's, start here
-        uint64_t t = i > 0 ? p / kTileCols + 1 : 0;
-        uint64_t t1 = i < n ? c / kTileCols : n_tiles;
+        uint64_t t = i > 0 ? (p >> shift) + 1 : 0;
+        uint64_t t1 = i < n ? c >> shift : n_tiles;
         t1 = t1 < n_tiles ? t1 : n_tiles;
         for (; t <= t1; t++) row[t] = (uint32_t)i;
         if (scale && i < n) m = fmaxf(m, values[a + i]);
@@ -104,19 +111,24 @@ __global__ __launch_bounds__(256) void row_tiles_kernel(const uint64_t* __restri
     if (threadIdx.x == 0) scale[r] = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]));
 }
 
-// total[t] (zeroed by the caller) += entries of tile t in the rows of this workgroup's range
-__global__ __launch_bounds__(256) void tile_totals_kernel(uint64_t R, uint32_t n_tiles, uint32_t rows_per,
+// total[t] (zeroed by the caller) += entries of tile t in this workgroup's kTotalRows rows, all in flight
+// (64 rows one after the other: 19 us against 8 for 3000 rows of 98 tiles)
+constexpr uint32_t kTotalRows = 16;
+__global__ __launch_bounds__(256) void tile_totals_kernel(uint64_t R, uint32_t n_tiles,
                                                           const uint32_t* __restrict__ tiles,
                                                           uint32_t* __restrict__ total) {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n_tiles) return;
-    const uint64_t r0 = (uint64_t)blockIdx.y * rows_per;
-    const uint64_t r1 = r0 + rows_per < R ? r0 + rows_per : R;
-    uint32_t sum = 0;
-    for (uint64_t r = r0; r < r1; r++) {
-        const uint32_t* row = tiles + r * (uint64_t)(n_tiles + 1) + t;
-        sum += row[1] - row[0];
+    uint32_t lo[kTotalRows], hi[kTotalRows], sum = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < kTotalRows; i++) {
+        const uint64_t r = (uint64_t)blockIdx.y * kTotalRows + i;
+        const uint32_t* row = tiles + (r < R ? r : R - 1) * (uint64_t)(n_tiles + 1) + t;
+        lo[i] = row[0];
+        hi[i] = r < R ? row[1] : lo[i];
     }
+#pragma unroll
+    for (uint32_t i = 0; i < kTotalRows; i++) sum += hi[i] - lo[i];
     if (sum) atomicAdd(&total[t], sum);
 }
 
@@ -267,19 +279,19 @@ __global__ __launch_bounds__(1024) void tile_order_kernel(uint32_t n_tiles, cons
     for (uint32_t g = threadIdx.x; g < n_groups; g += blockDim.x) order[atomicAdd(&s_at[cls(g)], 1u)] = g;
 }
 
-template <int VT>
+template <int VT, int COLS>
 __global__ __launch_bounds__(kPlaceThreads) void place_tile_kernel(
     uint64_t R, uint64_t C, uint32_t n_tiles, const uint32_t* __restrict__ tiles, const uint64_t* __restrict__ rowptr,
     const uint64_t* __restrict__ columns, const float* __restrict__ values, const float* __restrict__ scale,
     const uint64_t* __restrict__ tile_base, const uint32_t* __restrict__ order, uint64_t* __restrict__ colptr,
     uint32_t* __restrict__ crow, void* __restrict__ cval_out) {
     typedef typename StoredValue<VT>::type V;
-    __shared__ uint32_t s_next[kTileCols];     // counts, then where each column's next entry goes
-    __shared__ uint32_t s_mask[2][kTileCols];  // rows of the block that hold the column (low, high half)
+    __shared__ uint32_t s_next[COLS];     // counts, then where each column's next entry goes
+    __shared__ uint32_t s_mask[2][COLS];  // rows of the block that hold the column (low, high half)
     __shared__ uint32_t s_wave[kPlaceThreads / 64 + 1];
     __shared__ uint32_t s_before[kListRows];
     __shared__ uint32_t s_word[kListRows];
-    constexpr int kWaves = kPlaceThreads / 64, kCols = kTileCols / kPlaceThreads;
+    constexpr int kWaves = kPlaceThreads / 64, kCols = COLS / kPlaceThreads;
     constexpr uint32_t kUnits = 64;  // a group's units: eight to a wavefront, all in flight
     static_assert(kUnits >= kTileCols / 64 && kUnits == 8 * kWaves, "any row fits a group");
     const uint32_t turn = blockIdx.x / kXcd;  // workgroup blockIdx.x runs on XCD blockIdx.x % kXcd
@@ -287,12 +299,12 @@ __global__ __launch_bounds__(kPlaceThreads) void place_tile_kernel(
     if (slot >= (n_tiles + kTileGroup - 1) / kTileGroup) return;
     const uint32_t tile = order[slot] * kTileGroup + turn % kTileGroup;
     if (tile >= n_tiles) return;
-    const uint64_t c0 = (uint64_t)tile * kTileCols;
+    const uint64_t c0 = (uint64_t)tile * COLS;
     const uint64_t base = tile_base[tile];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const TileRows T{s_before, s_word, s_wave};
     V* __restrict__ cval = (V*)cval_out;
-    for (int i = tid; i < kTileCols; i += kPlaceThreads) {
+    for (int i = tid; i < COLS; i += kPlaceThreads) {
         s_next[i] = 0u;
         s_mask[0][i] = 0u;
         s_mask[1][i] = 0u;
@@ -703,38 +715,47 @@ hipError_t launch_pack_rows(uint64_t R, const uint64_t* rowptr, const float* val
     return hipGetLastError();
 }
 
-uint64_t csc_tiles(uint64_t C) { return (C + kTileCols - 1) / kTileCols; }
-uint64_t csc_tile_groups(uint64_t C) { return (csc_tiles(C) + kTileGroup - 1) / kTileGroup; }
+uint32_t csc_tile_cols(uint64_t R, uint64_t C, bool narrow) {
+    return narrow && C < kNarrowBelow && C <= kNarrowRow * R ? kNarrowTile : kTileCols;
+}
+uint64_t csc_tiles(uint64_t C, uint32_t tile_cols) { return (C + tile_cols - 1) / tile_cols; }
+uint64_t csc_tile_groups(uint64_t C, uint32_t tile_cols) {
+    return (csc_tiles(C, tile_cols) + kTileGroup - 1) / kTileGroup;
+}
 
 hipError_t launch_row_tiles(uint64_t R, const uint64_t* rowptr, const uint64_t* columns, const float* values,
-                            uint64_t C, uint32_t* tiles, float* scale, uint32_t* unsorted, hipStream_t stream) {
+                            uint64_t C, uint32_t tile_cols, uint32_t* tiles, float* scale, uint32_t* unsorted,
+                            hipStream_t stream) {
     if (R == 0) return hipSuccess;
     hipLaunchKernelGGL(row_tiles_kernel, dim3((unsigned)R), dim3(256), 0, stream, rowptr, columns, values, C,
-                       (uint32_t)csc_tiles(C), tiles, scale, unsorted);
+                       (uint32_t)__builtin_ctz(tile_cols), (uint32_t)csc_tiles(C, tile_cols), tiles, scale, unsorted);
     return hipGetLastError();
 }
 
-hipError_t launch_tile_totals(uint64_t R, uint64_t C, const uint32_t* tiles, uint32_t* total, hipStream_t stream) {
+hipError_t launch_tile_totals(uint64_t R, uint64_t C, uint32_t tile_cols, const uint32_t* tiles, uint32_t* total, hipStream_t stream) {
     if (R == 0 || C == 0) return hipSuccess;
-    const uint32_t n_tiles = (uint32_t)csc_tiles(C);
-    const uint32_t rows_per = 64;
-    hipLaunchKernelGGL(tile_totals_kernel, dim3((n_tiles + 255) / 256, (unsigned)((R + rows_per - 1) / rows_per)),
-                       dim3(256), 0, stream, R, n_tiles, rows_per, tiles, total);
+    const uint32_t n_tiles = (uint32_t)csc_tiles(C, tile_cols);
+    hipLaunchKernelGGL(tile_totals_kernel, dim3((n_tiles + 255) / 256, (unsigned)((R + kTotalRows - 1) / kTotalRows)),
+                       dim3(256), 0, stream, R, n_tiles, tiles, total);
     return hipGetLastError();
 }
 
-hipError_t launch_place_tiles(int vtype, uint64_t R, uint64_t C, const uint32_t* tiles, const uint64_t* rowptr,
+hipError_t launch_place_tiles(int vtype, uint64_t R, uint64_t C, uint32_t tile_cols, const uint32_t* tiles, const uint64_t* rowptr,
                               const uint64_t* columns, const float* values, const float* scale,
                               const uint64_t* tile_base, uint32_t* order, uint64_t* colptr, uint32_t* crow,
                               void* cval, hipStream_t stream) {
     if (C == 0) return hipSuccess;
-    const uint32_t n_tiles = (uint32_t)csc_tiles(C);
-    const uint32_t n_groups = (uint32_t)csc_tile_groups(C);
+    const uint32_t n_tiles = (uint32_t)csc_tiles(C, tile_cols);
+    const uint32_t n_groups = (uint32_t)csc_tile_groups(C, tile_cols);
     hipLaunchKernelGGL(tile_order_kernel, dim3(1), dim3(1024), 0, stream, n_tiles, tile_base, order);
     const dim3 g((n_groups + kXcd - 1) / kXcd * kXcd * kTileGroup), b(kPlaceThreads);
-    const auto kernel = vtype == FD_VAL_F32    ? place_tile_kernel<FD_VAL_F32>
-                        : vtype == FD_VAL_BF16 ? place_tile_kernel<FD_VAL_BF16>
-                                               : place_tile_kernel<FD_VAL_FP16>;
+    const bool narrow = tile_cols == kNarrowTile;
+    const auto kernel =
+        vtype == FD_VAL_F32
+            ? (narrow ? place_tile_kernel<FD_VAL_F32, kNarrowTile> : place_tile_kernel<FD_VAL_F32, kTileCols>)
+        : vtype == FD_VAL_BF16
+            ? (narrow ? place_tile_kernel<FD_VAL_BF16, kNarrowTile> : place_tile_kernel<FD_VAL_BF16, kTileCols>)
+            : (narrow ? place_tile_kernel<FD_VAL_FP16, kNarrowTile> : place_tile_kernel<FD_VAL_FP16, kTileCols>);
     hipLaunchKernelGGL(kernel, g, b, 0, stream, R, C, n_tiles, tiles, rowptr, columns, values, scale, tile_base, order,
                        colptr, crow, cval);
     return hipGetLastError();

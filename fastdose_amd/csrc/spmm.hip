@@ -62,12 +62,13 @@ int hip_result(hipError_t e) {
 // The voxel-major copy tile by tile (launch_place_tiles); *built is false when a row's columns do
 // not ascend or the tile table does not fit in memory (the general path's scratch can be smaller: 4 bytes
 // per column, and 2 per entry of 16-bit values), and nothing of the copy is written then.
-int build_by_tiles(const fd_dosemat* m, fd_spmm& p, const uint64_t* rowptr, hipStream_t s, bool* built) {
-    const uint64_t nt = csc_tiles(p.cols), R = p.rows;
+int build_by_tiles(const fd_dosemat* m, fd_spmm& p, const uint64_t* rowptr, uint32_t tile_cols, hipStream_t s,
+                   bool* built) {
+    const uint64_t nt = csc_tiles(p.cols, tile_cols), R = p.rows;
     DevBuf<uint64_t> base;    // exclusive scan of the tiles' totals (nt + 1), then the scan's scratch
     DevBuf<uint32_t> total;   // entries of each tile (nt), unsorted flag, the tile table, the tiles' order
     if (base.reserve(nt + 1 + scan_scratch_size(nt)) != FD_OK ||
-        total.reserve(nt + 1 + R * (nt + 1) + csc_tile_groups(p.cols)) != FD_OK) {
+        total.reserve(nt + 1 + R * (nt + 1) + csc_tile_groups(p.cols, tile_cols)) != FD_OK) {
         base.release();
         return FD_OK;
     }
@@ -76,16 +77,16 @@ int build_by_tiles(const fd_dosemat* m, fd_spmm& p, const uint64_t* rowptr, hipS
         uint32_t* tiles = total.ptr + nt + 1;
         hipError_t e = launch_fill_u32(total.ptr, nt + 1, 0u, s);
         if (e == hipSuccess)
-            e = launch_row_tiles(R, rowptr, m->columns.ptr, m->values.ptr, p.cols, tiles,
+            e = launch_row_tiles(R, rowptr, m->columns.ptr, m->values.ptr, p.cols, tile_cols, tiles,
                                  p.vtype == FD_VAL_F32 ? nullptr : p.scale.ptr, total.ptr + nt, s);
         if (e == hipSuccess)
             e = hipMemcpyAsync(&unsorted, total.ptr + nt, sizeof(unsorted), hipMemcpyDeviceToHost, s);
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         if (e != hipSuccess || unsorted) return e;
-        e = launch_tile_totals(R, p.cols, tiles, total.ptr, s);
+        e = launch_tile_totals(R, p.cols, tile_cols, tiles, total.ptr, s);
         if (e == hipSuccess) e = launch_scan_u32(total.ptr, nt, base.ptr, base.ptr + nt, base.ptr + nt + 1, s);
         if (e == hipSuccess)
-            e = launch_place_tiles(p.vtype, R, p.cols, tiles, rowptr, m->columns.ptr, m->values.ptr, p.scale.ptr,
+            e = launch_place_tiles(p.vtype, R, p.cols, tile_cols, tiles, rowptr, m->columns.ptr, m->values.ptr, p.scale.ptr,
                                    base.ptr, tiles + R * (nt + 1), p.colptr.ptr, p.crow.ptr, p.cval.ptr, s);
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         *built = e == hipSuccess;
@@ -202,9 +203,13 @@ int fd_spmm_create(const fd_dosemat* m, int value_type, fd_spmm** out, void* str
     bool built = false;
     // The tile table holds a u32 per (row, tile): rows of a few entries in a large volume, whose table
     // would outgrow the entries themselves, take the general path, as do rows with unsorted columns.
-    if (r == FD_OK && p->cols < (1ull << 32) && p->rows <= (1ull << 20) &&
-        p->rows * (csc_tiles(p->cols) + 1) * sizeof(uint32_t) <= 8 * p->nnz + (1ull << 20))
-        r = build_by_tiles(m, *p, rowptr.ptr, s, &built);
+    auto fits = [&](uint32_t tile_cols) {
+        return p->cols < (1ull << 32) && p->rows <= (1ull << 20) &&
+               p->rows * (csc_tiles(p->cols, tile_cols) + 1) * sizeof(uint32_t) <= 8 * p->nnz + (1ull << 20);
+    };
+    uint32_t tile_cols = csc_tile_cols(p->rows, p->cols, true);
+    if (!fits(tile_cols)) tile_cols = csc_tile_cols(p->rows, p->cols, false);
+    if (r == FD_OK && fits(tile_cols)) r = build_by_tiles(m, *p, rowptr.ptr, tile_cols, s, &built);
     if (r == FD_OK && !built) r = build_by_sorting(m, *p, rowptr.ptr, s);
     rowptr.release();
     if (r != FD_OK) {

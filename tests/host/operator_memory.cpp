@@ -70,8 +70,9 @@ hipError_t hipMemcpyAsync(void* to, const void*, size_t n, hipMemcpyKind k, hipS
 namespace fdi {
 void set_error(const std::string& m) { g_message = m; }
 uint64_t scan_scratch_size(uint64_t n) { return n / 4096 + 2; }
-uint64_t csc_tiles(uint64_t C) { return (C + 2047) / 2048; }
-uint64_t csc_tile_groups(uint64_t C) { return (csc_tiles(C) + 15) / 16; }
+uint32_t csc_tile_cols(uint64_t, uint64_t C, bool narrow) { return narrow && C < 400000 ? 512 : 2048; }
+uint64_t csc_tiles(uint64_t C, uint32_t cols) { return (C + cols - 1) / cols; }
+uint64_t csc_tile_groups(uint64_t C, uint32_t cols) { return (csc_tiles(C, cols) + 15) / 16; }
 hipError_t launch_fill_u32(uint32_t*, uint64_t, uint32_t, hipStream_t) { return launched(); }
 hipError_t launch_fill_u64(uint64_t*, uint64_t, uint64_t, hipStream_t) { return launched(); }
 hipError_t launch_scan_u32(const uint32_t*, uint64_t, uint64_t*, uint64_t*, uint64_t*, hipStream_t) {
@@ -84,12 +85,14 @@ hipError_t launch_global_rows(int, const uint64_t*, const uint64_t*, const uint6
 hipError_t launch_pack_rows(uint64_t, const uint64_t*, const float*, int, float*, uint16_t*, hipStream_t) {
     return launched();
 }
-hipError_t launch_row_tiles(uint64_t, const uint64_t*, const uint64_t*, const float*, uint64_t, uint32_t*, float*,
-                            uint32_t*, hipStream_t) {
+hipError_t launch_row_tiles(uint64_t, const uint64_t*, const uint64_t*, const float*, uint64_t, uint32_t, uint32_t*,
+                            float*, uint32_t*, hipStream_t) {
     return launched();
 }
-hipError_t launch_tile_totals(uint64_t, uint64_t, const uint32_t*, uint32_t*, hipStream_t) { return launched(); }
-hipError_t launch_place_tiles(int, uint64_t, uint64_t, const uint32_t*, const uint64_t*, const uint64_t*, const float*,
+hipError_t launch_tile_totals(uint64_t, uint64_t, uint32_t, const uint32_t*, uint32_t*, hipStream_t) {
+    return launched();
+}
+hipError_t launch_place_tiles(int, uint64_t, uint64_t, uint32_t, const uint32_t*, const uint64_t*, const uint64_t*, const float*,
                               const float*, const uint64_t*, uint32_t*, uint64_t*, uint32_t*, void*, hipStream_t) {
     g_tiles++;
     return launched();

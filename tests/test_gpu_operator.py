@@ -259,3 +259,28 @@ def test_one_vector_beyond_the_float_range(torch_cuda, vtype, x1):
         assert np.all(np.abs(one.astype(np.float64) - two) <= 8 * U * np.abs(two))
     else:
         assert np.array_equal(one, two, equal_nan=True)
+
+
+@pytest.mark.parametrize("R,cols", [(47, 192 * 2048 - 1), (48, 192 * 2048 - 1), (48, 192 * 2048), (2, 2 * 8192 + 1),
+                                    (2, 2 * 8192), (1500, 511), (1500, 513), (70, 300 * 2048 + 5)])
+def test_tile_widths(torch_cuda, R, cols):
+    """Tiles of 512 columns below 192 x 2048 columns and with a row for 8192 of them at least, of 2048 otherwise:
+    both sides of the lines, rows with every column of some tiles, against the general path, bit for bit."""
+    torch = torch_cuda
+    rng = np.random.default_rng([R, cols])
+    rows = []
+    for r in range(R):
+        start = int(rng.integers(0, max(1, cols - 3000)))
+        long = np.arange(start, min(cols, start + int(rng.integers(1, 3000)))) if r % 9 == 1 else np.zeros(0, np.int64)
+        rows.append(np.unique(np.concatenate([rng.integers(0, cols, 900), long, [0, cols - 1]])))
+    off = np.concatenate([[0], np.cumsum([len(c) for c in rows])])
+    c = np.concatenate(rows).astype(np.int64)
+    v = rng.uniform(0.01, 1.0, len(c)).astype(np.float32)
+    back = np.concatenate([np.arange(off[r], off[r + 1])[::-1] for r in range(R)])
+    x = torch.rand((R, 3), device="cuda")
+    for vtype in (fd.FD_VAL_F32, fd.FD_VAL_BF16, fd.FD_VAL_FP16):
+        y = []
+        for m in ((off, c, v), (off, c[back], v[back])):
+            with fd.Spmm(dose_mat(torch, cols, [m]), vtype) as op:
+                y.append(op.run(x).cpu().numpy())
+        assert np.array_equal(*y) and (y[0][0] > 0).all() and (y[0][-1] > 0).all()
