@@ -158,6 +158,6 @@ hipError_t launch_col_scatter(uint64_t R, const uint64_t* rowptr, const uint64_t
 hipError_t launch_col_sort(uint64_t C, const uint64_t* colptr, uint32_t* crow, void* cval, int vbytes,
                            hipStream_t stream);
 hipError_t launch_spmm(int vtype, uint64_t C, const uint64_t* colptr, const uint32_t* crow, const void* cval,
-                       const float* scale, const float* X, int k, uint64_t R, float* Y, hipStream_t stream);
+                       const float* scale, const float* X, int k, uint64_t R, uint64_t nnz, float* Y, hipStream_t stream);
 
 }  // namespace fdi

@@ -557,8 +557,8 @@ __global__ __launch_bounds__(256) void spmm_wide_kernel(uint64_t C, const uint64
 // 0.07 ms of it, the rest the gathers of rows, scales and x, whose lines keep the L1 busy.  Limits of E
 // and kSplitEntries: a factor of two either way costs 5-10 %.
 // SCALED (16-bit values, one vector): the workgroup holds scale times x of all rows in LDS, one gather
-// instead of two, and takes kScaledGroups times 256 columns to be worth it: 0.17 -> 0.15 ms (512 columns the
-// same, 2048 0.17).  With FP32 values, which have no scale, x in LDS takes 10 % longer, and with
+// instead of two, and takes kScaledGroups times 256 columns to be worth it (which is not so everywhere,
+// worth_scaling): 0.17 -> 0.15 ms (512 columns the same, 2048 0.17).  With FP32 values, which have no scale, x in LDS takes 10 % longer, and with
 // four vectors the table's size costs what it saves.  Its length: 16 KiB leave eight workgroups to a CU.
 // Where scale times x is not finite (the row's other entries times x may be), the product is taken entry by
 // entry as without the table.
@@ -794,12 +794,22 @@ hipError_t launch_col_sort(uint64_t C, const uint64_t* colptr, uint32_t* crow, v
 
 namespace {
 
+// Whether one vector goes through the table of scales times x: it has to fit, there have to be entries to
+// gather for (three for two columns; without, 256 rows on 128^3 voxels take 19.6 us with it and 18.8 without,
+// 400 rows 26 and 29), and either two workgroups to a CU hide each other's tables or each has many entries
+// for a row of its table (250 000 columns: 400 pencil rows 17 us with it and 19 without, 4000 rows of 300
+// scattered entries 11 and 8).  Below 2^17 columns most CUs would idle: 4096 rows on 24^3 voxels 56 and 20.
+bool worth_scaling(uint64_t C, uint64_t R, uint64_t nnz) {
+    if (R > kScaledRows || nnz < C + C / 2) return false;
+    return C >= (1ull << 19) || (C >= (1ull << 17) && nnz / R >= C / 128);
+}
+
 template <int VT, int V>
 void launch_narrow(int G, const dim3& g, const dim3& b, hipStream_t stream, uint64_t C, const uint64_t* colptr,
                    const uint32_t* crow, const void* cval, const float* scale, const float* X, int k, uint64_t R,
-                   float* Y) {
+                   uint64_t nnz, float* Y) {
     if constexpr (VT != FD_VAL_F32 && V == 1)
-        if (G == 1 && R <= kScaledRows) {
+        if (G == 1 && worth_scaling(C, R, nnz)) {
             const dim3 few(blocks_for((C + kScaledGroups - 1) / kScaledGroups, 65536));
             hipLaunchKernelGGL((spmm_narrow_kernel<VT, 1, 1, true>), few, b, R * sizeof(float), stream, C, colptr, crow,
                                cval, scale, X, k, R, Y);
@@ -832,7 +842,7 @@ void launch_narrow(int G, const dim3& g, const dim3& b, hipStream_t stream, uint
 
 template <int VT>
 hipError_t launch_spmm_typed(uint64_t C, const uint64_t* colptr, const uint32_t* crow, const void* cval,
-                             const float* scale, const float* X, int k, uint64_t R, float* Y, hipStream_t stream) {
+                             const float* scale, const float* X, int k, uint64_t R, uint64_t nnz, float* Y, hipStream_t stream) {
     const dim3 b(256);
     // beyond 128 vectors a column's lanes are all along them and its entries are wave-uniform
     if (k % 4 == 0 && k > 128) {
@@ -845,20 +855,20 @@ hipError_t launch_spmm_typed(uint64_t C, const uint64_t* colptr, const uint32_t*
     int G = 1;
     while (G < 64 && G * V < k) G *= 2;
     if (V == 4)
-        launch_narrow<VT, 4>(G, g, b, stream, C, colptr, crow, cval, scale, X, k, R, Y);
+        launch_narrow<VT, 4>(G, g, b, stream, C, colptr, crow, cval, scale, X, k, R, nnz, Y);
     else
-        launch_narrow<VT, 1>(G, g, b, stream, C, colptr, crow, cval, scale, X, k, R, Y);
+        launch_narrow<VT, 1>(G, g, b, stream, C, colptr, crow, cval, scale, X, k, R, nnz, Y);
     return hipGetLastError();
 }
 
 }  // namespace
 
 hipError_t launch_spmm(int vtype, uint64_t C, const uint64_t* colptr, const uint32_t* crow, const void* cval,
-                       const float* scale, const float* X, int k, uint64_t R, float* Y, hipStream_t stream) {
+                       const float* scale, const float* X, int k, uint64_t R, uint64_t nnz, float* Y, hipStream_t stream) {
     if (C == 0 || k <= 0) return hipSuccess;
-    if (vtype == FD_VAL_F32) return launch_spmm_typed<FD_VAL_F32>(C, colptr, crow, cval, scale, X, k, R, Y, stream);
-    if (vtype == FD_VAL_BF16) return launch_spmm_typed<FD_VAL_BF16>(C, colptr, crow, cval, scale, X, k, R, Y, stream);
-    return launch_spmm_typed<FD_VAL_FP16>(C, colptr, crow, cval, scale, X, k, R, Y, stream);
+    if (vtype == FD_VAL_F32) return launch_spmm_typed<FD_VAL_F32>(C, colptr, crow, cval, scale, X, k, R, nnz, Y, stream);
+    if (vtype == FD_VAL_BF16) return launch_spmm_typed<FD_VAL_BF16>(C, colptr, crow, cval, scale, X, k, R, nnz, Y, stream);
+    return launch_spmm_typed<FD_VAL_FP16>(C, colptr, crow, cval, scale, X, k, R, nnz, Y, stream);
 }
 
 }  // namespace fdi

@@ -243,7 +243,7 @@ int fd_spmm_run(fd_spmm* p, const float* x_dev, int k, float* y_dev, void* strea
     }
     FD_HIP(hipSetDevice(p->device));
     hipError_t e = launch_spmm(p->vtype, p->cols, p->colptr.ptr, p->crow.ptr, p->cval.ptr, p->scale.ptr, x_dev, k,
-                               p->rows, y_dev, (hipStream_t)stream);
+                               p->rows, p->nnz, y_dev, (hipStream_t)stream);
     if (e != hipSuccess) {
         set_error(std::string("spmm: ") + hipGetErrorString(e));
         return FD_ERR_HIP;

@@ -107,7 +107,7 @@ hipError_t launch_col_sort(uint64_t, const uint64_t*, uint32_t*, void*, int, hip
     return launched();
 }
 hipError_t launch_spmm(int, uint64_t, const uint64_t*, const uint32_t*, const void*, const float*, const float*, int,
-                       uint64_t, float*, hipStream_t) {
+                       uint64_t, uint64_t, float*, hipStream_t) {
     return launched();
 }
 }  // namespace fdi

@@ -284,3 +284,48 @@ def test_tile_widths(torch_cuda, R, cols):
             with fd.Spmm(dose_mat(torch, cols, [m]), vtype) as op:
                 y.append(op.run(x).cpu().numpy())
         assert np.array_equal(*y) and (y[0][0] > 0).all() and (y[0][-1] > 0).all()
+
+
+@pytest.mark.parametrize("R,cols,fill", [(2, (1 << 19) - 1, 1.0), (2, 1 << 19, 1.0), (2, 1 << 19, 0.7),
+                                         (255, (1 << 17) + 3, 0.02), (255, (1 << 17) - 3, 0.02),
+                                         (255, (1 << 17) + 3, 0.006), (4096, 1 << 17, 0.009), (4097, 1 << 17, 0.009)])
+def test_one_vector_and_16_bit_values_in_large_volumes(torch_cuda, R, cols, fill):
+    """The products of scales and vector lie in LDS from 2^17 columns on where the columns hold enough entries:
+    both sides of each line."""
+    torch = torch_cuda
+    rng = np.random.default_rng([R, cols, int(1000 * fill)])
+    n = round(fill * cols)
+    c = np.concatenate([np.sort((int(rng.integers(cols)) + np.arange(n)) % cols) for _ in range(R)])
+    v = rng.uniform(0.01, 1.0, R * n).astype(np.float32)
+    x = rng.uniform(-1.0, 1.0, (R, 1)).astype(np.float32)
+    row = np.repeat(np.arange(R), n)
+    dm = dose_mat(torch, cols, [(np.arange(R + 1) * n, c, v)])
+    for vtype in (fd.FD_VAL_BF16, fd.FD_VAL_FP16):
+        stored = rounded(v.reshape(R, n).astype(np.float64), vtype).reshape(-1)
+        with fd.Spmm(dm, vtype) as op:
+            y = op.run(torch.as_tensor(x).cuda()).cpu().numpy()[:, 0]
+        term = stored * x[row, 0].astype(np.float64)
+        want, mag = (np.bincount(c, w, cols) for w in (term, np.abs(term)))
+        assert np.all(np.abs(y - want) <= (np.bincount(c, minlength=cols) + 3) * U * mag), vtype
+
+
+@pytest.mark.parametrize("vtype", [fd.FD_VAL_BF16, fd.FD_VAL_FP16])
+@pytest.mark.parametrize("x1", [1e10, float("inf"), float("nan"), 0.0])
+def test_one_vector_beyond_the_float_range_in_large_volumes(torch_cuda, vtype, x1):
+    """As with few columns, where the products of scales and vector lie in LDS."""
+    torch = torch_cuda
+    cols = (1 << 19) + 5
+    rng = np.random.default_rng(3)
+    v = rng.uniform(1e25, 1e27, (3, cols)).astype(np.float32)
+    v[:, 100] = 1e30
+    c = np.tile(np.arange(cols, dtype=np.int64), 3)
+    with fd.Spmm(dose_mat(torch, cols, [(np.arange(4) * cols, c, v.reshape(-1))]), vtype) as op:
+        x = torch.tensor([[1.0], [x1], [1e-3]], device="cuda")
+        one = op.run(x).cpu().numpy()[:, 0]
+        two = op.run(torch.cat([x, torch.ones_like(x)], 1).contiguous()).cpu().numpy()[:, 0]
+    if x1 == 1e10:
+        assert np.isinf(two[100]) and np.isfinite(np.delete(two, 100)).all()
+    if x1 == 0.0:  # the table's path: q (s x) against (q s) x, three terms of one sign
+        assert np.all(np.abs(one.astype(np.float64) - two) <= 8 * U * np.abs(two))
+    else:
+        assert np.array_equal(one, two, equal_nan=True)
