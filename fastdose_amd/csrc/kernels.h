@@ -102,11 +102,12 @@ hipError_t launch_resample_compact(int n, int Z, const uint64_t* cand_off, const
                                    uint64_t* host_offsets, uint64_t* host_totals, CsrDst dst0, CsrDst dst1,
                                    hipStream_t stream);
 
-// Exclusive scan of count[0..N) (u32) into off[0..N) (u64) plus total[0] = sum.  With scratch
-// (scan_scratch_size(N) u64, nullable) large inputs take a scan by many workgroups.
+// Exclusive scan of count[0..N) (u32) into off[0..N) (u64) plus total[0] = sum; large inputs by many
+// workgroups (scratch: scan_scratch_size(N) u64, a sum per kScanTile counts).
+constexpr uint64_t kScanTile = 4096;
+constexpr uint64_t scan_scratch_size(uint64_t N) { return (N + kScanTile - 1) / kScanTile + 1; }
 hipError_t launch_scan_u32(const uint32_t* count, uint64_t N, uint64_t* off, uint64_t* total, uint64_t* scratch,
                            hipStream_t stream);
-uint64_t scan_scratch_size(uint64_t N);
 
 // Dense (rows x cols, row-major) -> CSR, by segments of rows: nonzero counts per segment, then (after
 // an exclusive scan of them) the fill.

@@ -102,6 +102,7 @@ __global__ __launch_bounds__(kScanThreads) void scan_u32_kernel(const uint32_t* 
 // kernel scans the tile sums in between).
 constexpr int kTileThreads = 256;
 constexpr uint64_t kTile = (uint64_t)kTileThreads * kScanItems;
+static_assert(kTile == kScanTile, "the scratch holds a sum per tile");
 constexpr uint64_t kScanTiles = 4096;
 
 __global__ __launch_bounds__(kTileThreads) void scan_tile_sums_kernel(const uint32_t* __restrict__ count, uint64_t N,
@@ -236,12 +237,10 @@ __global__ void write_offsets_kernel(const uint64_t* __restrict__ seg_off, const
 
 }  // namespace
 
-uint64_t scan_scratch_size(uint64_t N) { return (N + kTile - 1) / kTile + 1; }
-
 hipError_t launch_scan_u32(const uint32_t* count, uint64_t N, uint64_t* off, uint64_t* total, uint64_t* scratch,
                            hipStream_t stream) {
     // one workgroup takes 5 us for up to a pass, and 7 for every further one; two kernels take 9
-    if (!scratch || N <= kScanPass) {
+    if (N <= kScanPass) {
         hipLaunchKernelGGL(scan_u32_kernel, dim3(1), dim3(kScanThreads), 0, stream, count, N, off, total);
         return hipGetLastError();
     }

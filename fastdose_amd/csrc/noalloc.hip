@@ -23,7 +23,7 @@ constexpr uint64_t kNoAllocMaxRows = FD_NOALLOC_MAX_ROWS;
 // segment offsets and their total: u64 [kNoAllocMaxRows + 1], scan scratch: u64 [kScanScratch]; then
 // counts per segment: u32 [kNoAllocMaxRows], 256-aligned.  Rows are cut into fewer segments than
 // fd_dense_to_csr would take when there would be more of them than that.
-constexpr uint64_t kScanScratch = kNoAllocMaxRows / 4096 + 2;
+constexpr uint64_t kScanScratch = scan_scratch_size(kNoAllocMaxRows);
 constexpr size_t kOffBytes = (kNoAllocMaxRows + 1 + kScanScratch) * sizeof(uint64_t);
 constexpr size_t kCntStart = (kOffBytes + 255) / 256 * 256;
 constexpr size_t kScratchBytes = kCntStart + kNoAllocMaxRows * sizeof(uint32_t);
@@ -89,10 +89,6 @@ extern "C" int fd_dense_to_csr_noalloc(const float* dense_dev, uint64_t rows, ui
         FD_HIP(launch_dense_count(dense_dev, rows, cols, split, cnt, s));
     } else if (rows > 0) {
         FD_HIP(launch_fill_u32(cnt, n, 0, s));
-    }
-    if (scan_scratch_size(n) > kScanScratch) {  // the scan's own tile size decides
-        set_error("scan scratch of the allocation-free entry point too small");
-        return FD_ERR_UNSUPPORTED;
     }
     FD_HIP(launch_scan_u32(cnt, n, off, off + n, off + kNoAllocMaxRows + 1, s));
     uint64_t total = 0;

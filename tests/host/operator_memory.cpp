@@ -69,7 +69,6 @@ hipError_t hipMemcpyAsync(void* to, const void*, size_t n, hipMemcpyKind k, hipS
 
 namespace fdi {
 void set_error(const std::string& m) { g_message = m; }
-uint64_t scan_scratch_size(uint64_t n) { return n / 4096 + 2; }
 uint32_t csc_tile_cols(uint64_t, uint64_t C, bool narrow) { return narrow && C < 400000 ? 512 : 2048; }
 uint64_t csc_tiles(uint64_t C, uint32_t cols) { return (C + cols - 1) / cols; }
 uint64_t csc_tile_groups(uint64_t C, uint32_t cols) { return (csc_tiles(C, cols) + 15) / 16; }
