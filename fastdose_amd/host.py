@@ -221,36 +221,35 @@ class Context:
         cap = C.c_uint64()
         call("fd_resample_capacity", self._h, arr, n, C.byref(cap))
 
-        def arrays(room):
-            return (torch.empty(room, dtype=torch.int64, device=dev), torch.empty(room, dtype=torch.float32, device=dev))
-
-        def resample(cols, vals):
-            room = 0 if cols is None else len(cols)
+        def resample(room):
+            """The call with arrays of that room (0: none, which gives the size); (code, entries, arrays)."""
+            cols = torch.empty(room, dtype=torch.int64, device=dev) if room else None
+            vals = torch.empty(room, dtype=torch.float32, device=dev) if room else None
             csr = CSR(0, 0, room, offsets.data_ptr(), cols.data_ptr() if room else None,
                       vals.data_ptr() if room else None)
             rc = load().fd_resample_csr(self._h, arr, n, C.c_void_p(dose_dev.data_ptr()), stride, extent,
                                         C.byref(csr), _stream_arg(stream))
-            return rc, int(csr.nnz)
+            return rc, int(csr.nnz), cols, vals
 
         # room for the estimate, so that one call does; where that room, or the call's scratch beside it, does
         # not fit on the device, a call without room first, and arrays of the exact size after it
+        room = max(cap.value, 1)
         try:
-            cols, vals = arrays(max(cap.value, 1))
+            rc, nnz, cols, vals = resample(room)
+            fits = rc != _lib.FD_ERR_HIP or b"out of memory" not in load().fd_last_error()
         except torch.OutOfMemoryError:
-            cols = vals = None
-        rc, nnz = resample(cols, vals)
-        if rc == _lib.FD_ERR_HIP and cols is not None and b"out of memory" in load().fd_last_error():
+            fits = False
+        if not fits:
             cols = vals = None
             if dev.type == "cuda":
                 torch.cuda.empty_cache()  # the library allocates beside torch
-            rc, nnz = resample(None, None)
+            rc, nnz, cols, vals = resample(0)
         if rc == _lib.FD_ERR_CAPACITY or (rc == _lib.FD_OK and cols is None):
             cols = vals = None
-            cols, vals = arrays(max(nnz, 1))
-            if nnz:
-                rc, nnz = resample(cols, vals)
+            room = max(nnz, 1)
+            rc, nnz, cols, vals = resample(room)
         _lib.check(rc, "fd_resample_csr")
-        if len(cols) > 2 * nnz + 1024:  # the result should not hold on to much more memory than it needs
+        if room > 2 * nnz + 1024:  # the result should not hold on to much more memory than it needs
             try:
                 return offsets, cols[:nnz].clone(), vals[:nnz].clone()
             except torch.OutOfMemoryError:
