@@ -70,7 +70,7 @@ __global__ void global_rows_kernel(int n_mat, const uint64_t* __restrict__ row_f
 // kNarrowTile: in small volumes, where the tiles are fewer than the CUs, and with enough rows for a tile's
 // serial part (the rounds over its rows) to weigh more than a tile table of four times the size: an
 // operator of 60 pencil rows on 61 x 63 x 65 voxels is built in 95 us instead of 111, of 400 rows in 222
-// instead of 267; 7 rows would take 82 instead of 77.  The general path still is up to a tenth faster for
+// instead of 267; 7 rows would take 82 instead of 77.  The general path still is up to 15 % faster for
 // rows of a few entries scattered over a small volume, but its sort of one crowded column can take seconds.
 constexpr int kTileCols = 2048, kNarrowTile = 512;
 constexpr uint64_t kNarrowBelow = 192 * (uint64_t)kTileCols, kNarrowRow = 8192;
@@ -554,7 +554,8 @@ __global__ __launch_bounds__(256) void spmm_wide_kernel(uint64_t C, const uint64
 // entries is split over the four wavefronts (the longest tile would otherwise outlast the rest).
 // One BF16 vector product over 49 M entries (6.4 M voxels, 2 660 rows) takes 0.17 ms where one column
 // per wavefront with lanes along k took 5.4 ms; reading the entries and column pointers (350 MB) is
-// 0.07 ms of it, the rest the gathers of rows, scales and x, whose lines keep the L1 busy.  Limits of E
+// 0.07 ms of it, the rest the data path of vector memory (79 % busy with SCALED, 92 % with FP32 values, 55 and
+// 85 M L1 accesses: short runs of entries, and the gathers of scales and x).  Limits of E
 // and kSplitEntries: a factor of two either way costs 5-10 %.
 // SCALED (16-bit values, one vector): the workgroup holds scale times x of all rows in LDS, one gather
 // instead of two, and takes kScaledGroups times 256 columns to be worth it (which is not so everywhere,

@@ -13,12 +13,13 @@
 // 32-byte read per sample instead of eight gathers, no bounds tests, and rays of any direction
 // share cache lines.
 //
-// It is bound by vector instructions on small batches (1.0 issued per CU and cycle at 256 beamlets of
-// 137 slices) and by the record reads on large ones (the data path of vector memory 99 % busy in a
-// 20-beam plan: a read is issued for nearly every sample, since some lane of the wavefront changes its
-// base voxel).  So a sample has few instructions: base voxel and fraction are one conversion and one
-// v_fract per axis, the record offset is two 24-bit multiply-adds and three bit selects.  45.4 -> 37.2 M
-// wavefront instructions and 80 -> 69 us for 256 beamlets, 2.16 -> 2.05 ms in the plan.
+// It is bound by vector instructions and record reads together on small batches (0.86 instructions issued
+// per CU and cycle and the data path of vector memory 81 % busy at 256 beamlets of 137 slices) and by the
+// reads on large ones (0.69 and 98 % in a 20-beam plan: a read is issued for nearly every sample, since
+// some lane of the wavefront changes its base voxel).  So a sample has few instructions: base voxel and
+// fraction are one conversion and one v_fract per axis, the record offset is two 24-bit multiply-adds and
+// three bit selects.  45.4 -> 37.2 M wavefront instructions and 80 -> 69 us for 256 beamlets, 2.16 -> 2.05 ms
+// in the plan.
 //
 // The radiological path is a prefix sum along each ray, which one lane per ray would walk alone
 // (256 rays per beamlet: one wavefront per SIMD on small batches).  Each ray is cut into 1, 2, 4,
